@@ -139,9 +139,10 @@ int64_t mi_paged_decode_workspace_bytes(int32_t batch, int32_t max_blocks, int32
  *   max_blocks is 0).  The launch's blocks are cut into equal ranges, one per workgroup
  *   (and head group); sequences cut between ranges leave partials that a second, small
  *   launch merges (it also writes the zero rows).  Launches of at most one (sequence, KV
- *   head) per CU with max_blocks <= 512 run a single per-sequence kernel instead, which
- *   leaves the workspace untouched; the environment variable MI_DECODE_PATH=stream or =seq
- *   forces either kernel where both apply.
+ *   head) per CU, or with batch * max_blocks * num_kv_heads <= 98304, with max_blocks <= 512 run
+ *   the per-sequence kernels instead: one launch that leaves the workspace untouched when it
+ *   keeps the sequences whole, else one that cuts them and the merge.  The environment variable
+ *   MI_DECODE_PATH=stream or =seq forces either form where both apply.
  * Specialised for head_dim 128, block_size 16, num_kv_heads in {1, 2, 4, 8} and GQA groups
  * num_heads / num_kv_heads in {1, 2, 4, 5, 8} (query head h reads KV head h / group, as
  * _repeat_key_value does, src/mini_infra/model/qwen3.py:147-156); other shapes return
@@ -159,14 +160,15 @@ int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, const void*
  * mi_paged_decode_attention_fused -- mi_qk_norm_rope's decode form (q/k RMSNorm + RoPE of the new
  * tokens, K/V rows into their slots: qwen3.py:182-217 with _apply_paged_kv_pool's append :282-283)
  * followed by mi_paged_decode_attention (qwen3.py:219-292), with the same results bit for bit.
- * Where the per-sequence kernel serves the launch (batch * num_kv_heads <= CUs, max_blocks <= 512)
- * it is one launch whose workgroups rotate their own q heads and append their own K/V head;
- * otherwise it runs the two entry points, rotating q into q_scratch.
+ * Where the per-sequence kernels serve the launch (see mi_paged_decode_attention; projection rows,
+ * weights and cos / sin 16-byte aligned) their workgroups rotate their own q heads and append their
+ * own K/V head; otherwise it runs the two entry points, rotating q into q_scratch.  Without a
+ * workspace they keep the sequences whole.
  * q: [batch] rows of num_heads * 128 (q_row_stride), k / v: rows of num_kv_heads * 128;
  * cos / sin: [batch, 128]; q_scratch: [batch, num_heads, 128] bf16 (always required).
  * The remaining arguments are those of mi_qk_norm_rope and mi_paged_decode_attention.  Each row's
  * slot must lie in one of its own blocks (decode packing puts it at position context - 1): in the
- * one-launch form only the row's own workgroups are ordered after its append.
+ * per-sequence form only the row's own workgroups are ordered after its append.
  */
 int32_t mi_paged_decode_attention_fused(void* out, int64_t out_row_stride, const void* q, int64_t q_row_stride,
                                         const void* k, int64_t k_row_stride, const void* v, int64_t v_row_stride,

@@ -115,19 +115,10 @@ struct PrefillArgs {
   int64_t row_tokens;
 };
 
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// bf16 rounding of one float as an fp32 value in one instruction: the packed convert with a zero
-// low half leaves bf16(x) in the high half and zeros below, which is exactly bf16(x) as fp32.
-__device__ __forceinline__ float round_bf16_hi(float x) {
-  return __builtin_bit_cast(float, __builtin_convertvector((f32x2){0.0f, x}, bf16x2));
-}
-
 // The reference's scores: bf16(bf16(q . k) * scale) (src/mini_infra/model/qwen3.py:243), in place.
 __device__ __forceinline__ void reference_scores(f32x4& v, float scale) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = round_bf16_hi(round_bf16_hi(v[i]) * scale);
+  for (int i = 0; i < 4; ++i) v[i] = round_bf16(round_bf16(v[i]) * scale);
 }
 
 // One 16-byte-per-lane load straight into LDS: lane i writes bytes [16 i, 16 i + 16) of the

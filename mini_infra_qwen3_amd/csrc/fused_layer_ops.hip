@@ -183,37 +183,7 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_vec_kernel(const QkArgs
   const u32x4 w = *reinterpret_cast<const u32x4*>((is_q ? a.q_weight : a.k_weight) + 8 * j);
   const u32x4 cs = *reinterpret_cast<const u32x4*>(a.cos + t * 128 + 8 * j);
   const u32x4 sn = *reinterpret_cast<const u32x4*>(a.sin + t * 128 + 8 * j);
-  float xf[8];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    xf[2 * e] = bf16_lo(x[e]);
-    xf[2 * e + 1] = bf16_hi(x[e]);
-  }
-  double sq = 0.0;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) sq += static_cast<double>(xf[e]) * xf[e];
-  const float r = rms_inv(dpp_sum16_f64(sq), 128.0, a.eps);
-  float y[8];
-  u32x4 yb;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    y[2 * e] = round_bf16(bf16_lo(w[e]) * round_bf16(xf[2 * e] * r));
-    y[2 * e + 1] = round_bf16(bf16_hi(w[e]) * round_bf16(xf[2 * e + 1] * r));
-    yb[e] = pack_bf16x2(y[2 * e], y[2 * e + 1]);
-  }
-  u32x4 pb;  // the rotate_half partner's normalised values (elements 64 apart): DPP row_ror:8 = lane ^ 8
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    pb[e] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(yb[e]), 0x128, 0xf, 0xf, false));
-  const float sign = j < 8 ? -1.0f : 1.0f;  // element e < 64: y cos - y[e + 64] sin; else y cos + y[e - 64] sin
-  u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float o0 = round_bf16(round_bf16(y[2 * e] * bf16_lo(cs[e])) + round_bf16(sign * bf16_lo(pb[e]) * bf16_lo(sn[e])));
-    const float o1 =
-        round_bf16(round_bf16(y[2 * e + 1] * bf16_hi(cs[e])) + round_bf16(sign * bf16_hi(pb[e]) * bf16_hi(sn[e])));
-    o[e] = pack_bf16x2(o0, o1);
-  }
+  const u32x4 o = norm_rope_piece(x, w, cs, sn, a.eps, j);
   if (!live) return;
   if (is_q) {
     *reinterpret_cast<u32x4*>(a.q_out + (t * a.q_heads + h) * 128 + 8 * j) = o;

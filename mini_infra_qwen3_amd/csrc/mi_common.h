@@ -106,18 +106,17 @@ constexpr int kMaxLayersPerLaunch = 32;
 __device__ __forceinline__ float bf16_lo(uint32_t pair) { return __uint_as_float(pair << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t pair) { return __uint_as_float(pair & 0xffff0000u); }
 
-// fp32 -> bf16 with round-to-nearest-even (NaN kept quiet): add 0x7fff plus the
-// lowest kept bit, then truncate -- the standard bit-level RNE construction.
-__device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return u >> 16;
-}
-__device__ __forceinline__ float round_bf16(float f) { return __uint_as_float(f32_to_bf16_bits(f) << 16); }
+// fp32 -> bf16 with round-to-nearest-even (NaN kept quiet): one packed convert (v_cvt_pk_bf16_f32).
+// Over all 2^32 inputs it gives the bits of the integer construction (add 0x7fff plus the lowest kept
+// bit, truncate; NaN payloads kept with the quiet bit set), which takes 6 instructions and a NaN test.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
 }
+__device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) { return pack_bf16x2(f, 0.0f); }
+// bf16(f) as fp32: converted into the high half with zeros below, which is that value.
+__device__ __forceinline__ float round_bf16(float f) { return __uint_as_float(pack_bf16x2(0.0f, f)); }
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
 
 // Cross-lane steps without LDS permutes: a 16-lane DPP butterfly within each row (xor 1, xor 2,
@@ -172,6 +171,25 @@ __device__ __forceinline__ float xmax32(float x) {
   return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
 }
 
+__device__ __forceinline__ float xsum16_f32(float x) {
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float xsum32_f32(float x) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ int wave_sum_i32(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, false);   // quad_perm [1,0,3,2]
+  x += __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, false);   // quad_perm [2,3,0,1]
+  x += __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, false);  // row_half_mirror
+  x += __builtin_amdgcn_update_dpp(0, x, 0x140, 0xf, 0xf, false);  // row_mirror
+  const auto p = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(x), static_cast<uint32_t>(x), false, false);
+  const uint32_t y = p[0] + p[1];
+  const auto q = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+  return static_cast<int>(q[0] + q[1]);
+}
+
 // ------------------------------------------------------- RMSNorm, exact ---
 // The reference's RMSNorm (src/mini_infra/model/qwen3.py:67-78) is
 //   h = x.float(); y = w * (h * rsqrt(h.pow(2).mean(-1) + eps)).to(bf16)
@@ -208,6 +226,46 @@ __device__ __forceinline__ void norm_rope_head(const uint16_t* src, const uint16
   // element l:      y*cos - y[l+64]*sin ; element l+64: y*cos + y[l]*sin  (rotate_half = cat(-y2, y1))
   o0 = round_bf16(round_bf16(y0 * bf16_bits_to_f32(cos[lane])) + round_bf16(-y1 * bf16_bits_to_f32(sin[lane])));
   o1 = round_bf16(round_bf16(y1 * bf16_bits_to_f32(cos[lane + 64])) + round_bf16(y0 * bf16_bits_to_f32(sin[lane + 64])));
+}
+
+// The same for lane j of 16 (one DPP row) holding elements [8 j, 8 j + 8) of the head, its weights and
+// its cos / sin row as 16-byte pieces: the sum of squares is exact in fp64 in any order, and
+// rotate_half pairs lane j with lane j ^ 8 (DPP row_ror:8), so the piece returned has the bits of
+// norm_rope_head.  Every lane of the wavefront must be active.
+__device__ __forceinline__ u32x4 norm_rope_piece(const u32x4 x, const u32x4 w, const u32x4 cs, const u32x4 sn, float eps,
+                                                 int j) {
+  float xf[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t v = x[e];
+    xf[2 * e] = bf16_lo(v);
+    xf[2 * e + 1] = bf16_hi(v);
+  }
+  double sq = 0.0;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sq += static_cast<double>(xf[e]) * xf[e];
+  const float r = rms_inv(dpp_sum16_f64(sq), 128.0, eps);
+  float y[8];
+  uint32_t yb[4], pb[4];  // the normalised values, and the partner's (elements 64 apart)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    y[2 * e] = round_bf16(bf16_lo(w[e]) * round_bf16(xf[2 * e] * r));
+    y[2 * e + 1] = round_bf16(bf16_hi(w[e]) * round_bf16(xf[2 * e + 1] * r));
+    yb[e] = pack_bf16x2(y[2 * e], y[2 * e + 1]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    pb[e] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(yb[e]), 0x128, 0xf, 0xf, false));
+  const float sign = j < 8 ? -1.0f : 1.0f;  // element e < 64: y cos - y[e + 64] sin; else y cos + y[e - 64] sin
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float o0 = round_bf16(round_bf16(y[2 * e] * bf16_lo(cs[e])) + round_bf16(sign * bf16_lo(pb[e]) * bf16_lo(sn[e])));
+    const float o1 =
+        round_bf16(round_bf16(y[2 * e + 1] * bf16_hi(cs[e])) + round_bf16(sign * bf16_hi(pb[e]) * bf16_hi(sn[e])));
+    o[e] = pack_bf16x2(o0, o1);
+  }
+  return o;
 }
 
 }  // namespace mi

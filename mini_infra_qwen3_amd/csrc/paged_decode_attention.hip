@@ -86,11 +86,10 @@ constexpr float kRescaleSlack = 8.0f;
 
 static_assert(kDepth >= 2 && kDepth - 1 < kWindow, "the ring looks ahead less than one id window");
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 #ifndef MI_DECODE_MFMA_GROUP
@@ -104,16 +103,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // group); matrix-core form 6.75 / 6.71 / 6.56 / 6.51 / 6.35.  At group 2, interleaved in one
 // process (8 x 20 launches each), the matrix-core form took 461.5 µs (median) against 463.3.
 constexpr int kMfmaGroup = MI_DECODE_MFMA_GROUP;
-#ifndef MI_DECODE_SEQ_MFMA_GROUP
-#define MI_DECODE_SEQ_MFMA_GROUP 2
-#endif
-// The per-sequence kernel (small launches: latency-bound) takes the matrix-core form from this
-// group size up.  At group 2 the matrix-core form measured faster (6.4 against 7.8 µs per layer at
-// batch 1, 9.5 against 11.6 at 6, 22.0 against 22.8 at 32; contexts U[32, 1150]); in the
-// bandwidth-kernel e2e runs of config 5 (two repetitions each, one machine) the decode step went
-// from 2.144-2.145 to 2.104-2.121 ms alternating and from 2.127-2.136 to 2.114-2.118 ms mixed.
-constexpr int kSeqMfmaGroup = MI_DECODE_SEQ_MFMA_GROUP;
-
 struct DecodeArgs {
   uint16_t* out;
   int64_t out_row;                 // elements
@@ -129,9 +118,15 @@ struct DecodeArgs {
   int32_t batch;                   // sequences of this launch
   int32_t max_blocks;
   int32_t streams;                 // block ranges; grid = streams x head groups
+  int32_t part_blocks;             // parts kernel: table blocks of a part; 0: the stripe kernel
+  int32_t splits;                  // parts per sequence, ceil(max_blocks / part_blocks); stripe kernel:
+                                   // workgroups per (sequence, KV head) (1: no partials)
   float scale;                     // softmax scale (natural units)
-  float* ws_acc;                   // [streams, 2, heads, 128]: slot 0 = range's first (cut) sequence, 1 = last
-  float* ws_ml;                    // [streams, 2, heads, 2] = (m, l) in log2 units
+  // Partials, [slots, heads, 128] and [slots, heads, 2] = (m, l) in log2 units.  Stream kernel: slots
+  // 2 s and 2 s + 1 are range s's first (cut) and last sequence; parts kernel: b splits + part; stripe
+  // kernel: b kStripes + stripe.
+  float* ws_acc;
+  float* ws_ml;
   // Fused form of the per-sequence kernel: raw q / k / v projection rows of the new tokens, the
   // q/k norm weights, cos / sin rows [batch, 128] and the slots of the new K/V rows.
   const uint16_t* q_raw;
@@ -193,10 +188,22 @@ __device__ __forceinline__ int blocks_of(int64_t n) {
   return n <= 0 ? 0 : static_cast<int>((n + kBlockSize - 1) / kBlockSize);
 }
 
-// Range holding block x of N: the last s with floor(s N / streams) <= x.
-__device__ __forceinline__ int stream_of(int64_t x, int64_t total, int streams) {
-  return static_cast<int>(((x + 1) * streams - 1) / total);
-}
+// The cut of N > 0 blocks into min(streams, N) ranges, none empty: range s starts at block
+// s q + min(s, rem) (the first rem ranges hold q + 1 blocks, the rest q).  32-bit arithmetic: N < 2^31,
+// checked by the entry point.
+struct Ranges {
+  int count, q, rem;
+  __device__ __forceinline__ Ranges(int total, int streams) {
+    count = max(min(streams, total), 1);
+    q = total / count;
+    rem = total - q * count;
+  }
+  __device__ __forceinline__ int begin(int s) const { return s * q + min(s, rem); }
+  __device__ __forceinline__ int of(int x) const {  // the range holding block x
+    const int wide = rem * (q + 1);                 // blocks of the first rem ranges
+    return x < wide ? x / (q + 1) : rem + (x - wide) / q;
+  }
+};
 
 __device__ __forceinline__ void store_bf16x8(uint16_t* dst, const float* o, float inv) {
   uint4 v;
@@ -240,7 +247,7 @@ __device__ int scan_blocks(const DecodeArgs& a, int* s_off, int* s_wave) {
 }
 
 // Sequence of block x (x < total): the last b with s_off[b] <= x (empty sequences are skipped).
-__device__ __forceinline__ int row_of(const int* s_off, int batch, int64_t x) {
+__device__ __forceinline__ int row_of(const int* s_off, int batch, int x) {
   int lo = 0, hi = batch;  // s_off[lo] <= x < s_off[hi]
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
@@ -469,9 +476,9 @@ __global__ __launch_bounds__(64 * kWaves, (kGroupsPerCu * kWaves + 3) / 4) void 
   }
   const int stream = wg / kHeadGroups;
   const int hg = wg - stream * kHeadGroups;
-  const int64_t lo = static_cast<int64_t>(stream) * total / a.streams;
-  const int64_t hi = static_cast<int64_t>(stream + 1) * total / a.streams;
-  if (lo >= hi) return;
+  const Ranges rg(total, a.streams);
+  if (total == 0 || stream >= rg.count) return;
+  const int lo = rg.begin(stream), hi = rg.begin(stream + 1);
 
   const int lane = threadIdx.x & 63;
   const int dl = lane & 15;
@@ -488,22 +495,22 @@ __global__ __launch_bounds__(64 * kWaves, (kGroupsPerCu * kWaves + 3) / 4) void 
 
   // Block ids of window [base, base + 64), one per lane (indices past the range repeat its
   // last block; ids outside the pool read block 0).
-  auto fetch_ids = [&](int64_t base, uint32_t& id_lo, uint32_t& id_hi) {
-    const int64_t x = min(base + lane, hi - 1);
+  auto fetch_ids = [&](int base, uint32_t& id_lo, uint32_t& id_hi) {
+    const int x = min(base + lane, hi - 1);
     const int b = row_of(s_off, a.batch, x);
     int64_t id = a.block_tables[b * a.bt_stride + (x - s_off[b])];
     if (id < 0 || id >= a.num_blocks) id = 0;
     id_lo = static_cast<uint32_t>(id);
     id_hi = static_cast<uint32_t>(static_cast<uint64_t>(id) >> 32);
   };
-  int64_t wbase = lo;
+  int wbase = lo;
   uint32_t cur_lo, cur_hi, nxt_lo, nxt_hi;
   fetch_ids(wbase, cur_lo, cur_hi);
   fetch_ids(wbase + kWindow, nxt_lo, nxt_hi);
 
   u32x4 kbuf[kDepth][4], vbuf[kDepth][4];
   // Loads block y (clamped to the range) into ring slot `slot`; y never passes the next window.
-  auto issue = [&](int slot, int64_t y) {
+  auto issue = [&](int slot, int y) {
     y = min(y, hi - 1);
     if (y >= wbase + kWindow) {  // wave-uniform: slide the window, fetch the one after
       wbase += kWindow;
@@ -511,7 +518,7 @@ __global__ __launch_bounds__(64 * kWaves, (kGroupsPerCu * kWaves + 3) / 4) void 
       cur_hi = nxt_hi;
       fetch_ids(wbase + kWindow, nxt_lo, nxt_hi);
     }
-    const int j = static_cast<int>(y - wbase);
+    const int j = y - wbase;
     const uint32_t blo = __builtin_amdgcn_readlane(cur_lo, j);
     const uint32_t bhi = __builtin_amdgcn_readlane(cur_hi, j);
     const int64_t base = static_cast<int64_t>((static_cast<uint64_t>(bhi) << 32) | blo) * kBlockElems;
@@ -526,10 +533,10 @@ __global__ __launch_bounds__(64 * kWaves, (kGroupsPerCu * kWaves + 3) / 4) void 
   for (int s = 0; s < kDepth - 1; ++s) issue(s, lo + s);  // ring slot of block x: (x - lo) % kDepth
 
   int b = row_of(s_off, a.batch, lo);
-  int64_t x = lo;
+  int x = lo;
   while (x < hi) {
-    const int64_t row_lo = s_off[b], row_hi = s_off[b + 1];
-    const int64_t seg_end = min(hi, row_hi);
+    const int row_lo = s_off[b], row_hi = s_off[b + 1];
+    const int seg_end = min(hi, row_hi);
     const int n32 = static_cast<int>(context_of(a, b));  // contexts are bounded by max_blocks * 16 < 2^31
     const uint16_t* qp = a.query + b * a.q_row + (g * kG) * a.q_head;
     uint4 q[kMfma ? 1 : kG];
@@ -550,14 +557,14 @@ __global__ __launch_bounds__(64 * kWaves, (kGroupsPerCu * kWaves + 3) / 4) void 
       st.init();
     }
 
-    const int64_t seg_begin = x;
-    for (int64_t x0 = x - (x - lo) % kDepth; x0 < seg_end; x0 += kDepth) {
+    const int seg_begin = x;
+    for (int x0 = x - (x - lo) % kDepth; x0 < seg_end; x0 += kDepth) {
 #pragma unroll
       for (int s = 0; s < kDepth; ++s) {
-        const int64_t xb = x0 + s;
+        const int xb = x0 + s;
         if (xb < seg_begin || xb >= seg_end) continue;  // wave-uniform
         issue((s + kDepth - 1) % kDepth, xb + kDepth - 1);
-        const int tok_base = static_cast<int>(xb - row_lo) * kBlockSize;
+        const int tok_base = (xb - row_lo) * kBlockSize;
         if constexpr (kMfma)
           attend_block_mfma(ms, qf, kbuf[s], vbuf[s], s_kst[threadIdx.x >> 6], scale, tok_base, n32, lane);
         else
@@ -626,187 +633,521 @@ __global__ __launch_bounds__(64 * kWaves, (kGroupsPerCu * kWaves + 3) / 4) void 
   }
 }
 
-// ---- Small launches: one workgroup per (sequence, KV head).  Its kSeqWaves wavefronts take
-// blocks w, w + kSeqWaves, ... of the sequence with the stream kernel's per-block arithmetic
-// (same lane layout, rounding points and lazy rescale), merge their four rows, then merge the
-// wavefronts' softmax states through LDS and write the bf16 rows: one launch, nothing in the
-// workspace.  A few sequences then spread over many wavefronts instead of a few block ranges
-// that a second launch has to merge.
-#ifndef MI_DECODE_SEQ_WAVES
-#define MI_DECODE_SEQ_WAVES 8
+// ---- Small launches.  Two forms share the prologue below; both spread long tables over more CUs than
+// they have (sequence, KV head) pairs, because one CU takes in no more than 47-62 bytes/ns of K/V
+// whatever the loads in flight (8192 tokens on one CU per KV head: 87-92 us with rings of 2 to 4, 8 or 16
+// wavefronts), and both are chains of dependent memory round trips of 1.4-2 us each, so everything
+// that depends on nothing (context, block ids, the projection rows and tables of the prologue) is
+// loaded together and no load is issued for a block that is not used.
+//  * stripes, tables of up to kStripeMaxBlocks blocks: a sequence always falls into kStripes stripes,
+//    stripe v being blocks v, v + kStripes, ..., each attended by one wavefront with the stream
+//    kernel's per-block arithmetic and merged in order.  One workgroup holds all stripes (and writes
+//    the rows), or kStripeWaves each hold some and the merge launch joins them: the bits are the same.
+//  * parts, longer tables or more pairs: contiguous ranges of the table, two blocks a step.
+// Measured against the form before (the stripes of a pair always in one workgroup, with a ring that
+// re-read the last block past its end), us per layer with the prologue and the merge, passes in a graph:
+// one sequence of 417 tokens 8.4 -> 6.9 (stripes in one workgroup); 8 of U[32, 1150] 18.4 -> 13.3, 24
+// 21.6 -> 17.7, 12 with 4 heads per KV head 18.0 -> 14.3 (stripes spread one by one; by twos 13.5 / 18.4 /
+// 14.9, by fours 15.0 / 21.2 / 15.0); 3 lognormal to 8192 89 -> 17.7, 21 with 8 heads per KV head 102 ->
+// 54.7 (parts).  Rings of 2 / 3 / 4 blocks: 13.4 / 13.3 / 13.3 at 8 sequences, 14.8 / 14.3 / 15.5 at 12.
+constexpr int kStripes = 8;
+#ifndef MI_DECODE_STRIPE_WAVES
+#define MI_DECODE_STRIPE_WAVES 1
 #endif
-#ifndef MI_DECODE_SEQ_DEPTH
-#define MI_DECODE_SEQ_DEPTH 2
+#ifndef MI_DECODE_STRIPE_DEPTH
+#define MI_DECODE_STRIPE_DEPTH 3
 #endif
-constexpr int kSeqWaves = MI_DECODE_SEQ_WAVES;
-constexpr int kSeqMaxBlocks = 64 * kSeqWaves;  // a lane holds one block id of its wavefront
+constexpr int kStripeWaves = MI_DECODE_STRIPE_WAVES;  // stripes (wavefronts) of a workgroup when they are spread
+constexpr int kStripeDepth = MI_DECODE_STRIPE_DEPTH;  // blocks of a stripe in registers, the current one included
+constexpr int kPartWaves = 4;
+constexpr int kPartMaxBlocks = 64 * kPartWaves;  // a lane holds one block id of its wavefront
+constexpr int kSeqMaxBlocks = 64 * kStripes;
+constexpr int kPairTokens = 2 * kBlockSize;
 
-// kFused: the workgroup first does what mi_qk_norm_rope's decode form does for its heads --
-// wavefronts 0 and 1 normalise and rotate query heads 2 g and 2 g + 1 into LDS, wavefront 2 key
-// head g, which it writes with value head g into the sequence's new slot -- then attends.  The
-// barrier after the pool stores makes them visible to the workgroup's own loads of that block
-// (the slot's lines are not in the CU cache before: no other workgroup reads head g of this
-// sequence, and the cache starts every launch clean).
-template <int kKvHeads, int kG, bool kFused>
-__global__ __launch_bounds__(64 * kSeqWaves) void paged_decode_seq_kernel(const DecodeArgs a) {
-  constexpr int kRowElems = kKvHeads * kHeadDim;
-  constexpr int kBlockElems = kBlockSize * kRowElems;
-  constexpr int kSeqDepth = MI_DECODE_SEQ_DEPTH;  // ring: the next kSeqDepth - 1 blocks of the wavefront in flight
-  __shared__ float s_acc[kSeqWaves][kG][kHeadDim];
-  __shared__ float s_ml[kSeqWaves][kG][2];
-  __shared__ __align__(16) uint16_t s_q[kFused ? kG : 1][kHeadDim];
-  constexpr bool kMfmaForm = kG >= kSeqMfmaGroup;
-  __shared__ __align__(16) uint16_t s_kst[kMfmaForm ? kSeqWaves : 1][kMfmaForm ? kBlockSize * kKStageRow : 8];
-  const int b = blockIdx.x;
-  const int g = blockIdx.y;
-  const int w = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int dl = lane & 15;
-  const int r = lane >> 4;
-  if constexpr (kFused) {
-    // Unit u < kG: query head g kG + u, normalised and rotated into LDS; unit kG: key head g,
-    // written with value head g into the sequence's new slot.  Wavefront w takes units
-    // w, w + kSeqWaves, ...
-    for (int u = w; u <= kG; u += kSeqWaves) {  // wave-uniform
-      const bool is_q = u < kG;
-      const uint16_t* src = is_q ? a.q_raw + b * a.q_raw_row + (g * kG + u) * kHeadDim
-                                 : a.k_raw + b * a.k_raw_row + g * kHeadDim;
-      float o0, o1;
-      norm_rope_head(src, is_q ? a.q_weight : a.k_weight, a.cos + b * kHeadDim, a.sin + b * kHeadDim, a.eps, lane,
-                     o0, o1);
-      if (is_q) {
-        s_q[u][lane] = static_cast<uint16_t>(f32_to_bf16_bits(o0));
-        s_q[u][lane + 64] = static_cast<uint16_t>(f32_to_bf16_bits(o1));
-      } else {
-        const int64_t slot = a.slot_mapping[b * a.slot_stride];
-        if (slot >= 0 && slot < a.num_slots) {
-          uint16_t* kd = const_cast<uint16_t*>(a.key_pool) + (slot * kKvHeads + g) * kHeadDim;
-          uint16_t* vd = const_cast<uint16_t*>(a.value_pool) + (slot * kKvHeads + g) * kHeadDim;
-          const uint16_t* vs = a.v_raw + b * a.v_raw_row + g * kHeadDim;
-          kd[lane] = static_cast<uint16_t>(f32_to_bf16_bits(o0));
-          kd[lane + 64] = static_cast<uint16_t>(f32_to_bf16_bits(o1));
-          vd[lane] = vs[lane];
-          vd[lane + 64] = vs[lane + 64];
-        }
+// The fused form's prologue: what mi_qk_norm_rope's decode form does for KV head g of sequence b.  16
+// lanes per head normalise and rotate the kG query heads and the key head into LDS; the workgroup told
+// to append writes the key head with value head g into the sequence's new slot.  The wavefronts that
+// attend the slot's block do not read that row back: they put the key head and the value row in place
+// of what they loaded, so no load waits for the append, in this workgroup or another.
+template <int kKvHeads, int kG, int kWaves>
+struct Prologue {
+  static constexpr int kUnits = kG + 1;  // query heads, then the new key
+  static constexpr int kPasses = (kUnits + 4 * kWaves - 1) / (4 * kWaves);
+  u32x4 x[kPasses], w[kPasses], c, s, v;
+  int64_t slot;  // the new token's slot; -1: none
+
+  // Unit of 16-lane row r in a pass; past the last one the key head again.
+  static __device__ __forceinline__ int unit(int pass, int wave, int r) {
+    return min(4 * (pass * kWaves + wave) + r, kG);
+  }
+  __device__ __forceinline__ void load(const DecodeArgs& a, int b, int g, int wave, int r, int dl) {
+    slot = a.slot_mapping[b * a.slot_stride];
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      const int u = unit(p, wave, r);
+      x[p] = *reinterpret_cast<const u32x4*>((u < kG ? a.q_raw + b * a.q_raw_row + (g * kG + u) * kHeadDim
+                                                     : a.k_raw + b * a.k_raw_row + g * kHeadDim) + 8 * dl);
+      w[p] = *reinterpret_cast<const u32x4*>((u < kG ? a.q_weight : a.k_weight) + 8 * dl);
+    }
+    c = *reinterpret_cast<const u32x4*>(a.cos + b * kHeadDim + 8 * dl);
+    s = *reinterpret_cast<const u32x4*>(a.sin + b * kHeadDim + 8 * dl);
+    v = *reinterpret_cast<const u32x4*>(a.v_raw + b * a.v_raw_row + g * kHeadDim + 8 * dl);
+  }
+  // heads: [kUnits][128] in LDS, complete after the barrier inside.
+  __device__ __forceinline__ void run(const DecodeArgs& a, int g, int wave, int r, int dl, bool append,
+                                      uint16_t (*heads)[kHeadDim]) {
+    if (slot >= a.num_slots || slot < 0) slot = -1;
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      if (4 * (p * kWaves + wave) >= kUnits) break;  // wave-uniform
+      const int u = unit(p, wave, r);
+      const u32x4 o = norm_rope_piece(x[p], w[p], c, s, a.eps, dl);
+      *reinterpret_cast<u32x4*>(&heads[u][8 * dl]) = o;
+      if (append && u == kG && slot >= 0) {  // the repeated units write the same bytes
+        const int64_t at = (slot * kKvHeads + g) * kHeadDim + 8 * dl;
+        *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(a.key_pool) + at) = o;
+        *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(a.value_pool) + at) = v;
       }
     }
     __syncthreads();
   }
-  const int n = static_cast<int>(context_of(a, b));
+};
+
+// Workgroup -> (KV head, sequence, split): ids go round-robin to the XCDs; the heads of one (sequence,
+// split) are neighbours, and the head an XCD gets rotates from one to the next, so every XCD gets an
+// even share of each sequence and of the heads' columns of the pool rows.
+struct SeqUnit {
+  int g, b, split;
+};
+template <int kKvHeads>
+__device__ __forceinline__ SeqUnit seq_unit(int batch) {
+  const int u = static_cast<int>(blockIdx.x) / kKvHeads;
+  const int split = u / batch;
+  return {(static_cast<int>(blockIdx.x) + u) % kKvHeads, u - split * batch, split};
+}
+
+// Q^T fragments of a wavefront: head dl (zero past the group), dims 32 ks + 8 r .. +8.
+template <int kG, bool kFused>
+__device__ __forceinline__ void query_fragments(const DecodeArgs& a, int b, int g, int r, int dl,
+                                                const uint16_t (*heads)[kHeadDim], bf16x8 (&qf)[4]) {
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    if constexpr (kFused)
+      qf[ks] = dl < kG ? *reinterpret_cast<const bf16x8*>(&heads[dl < kG ? dl : 0][32 * ks + 8 * r]) : bf16x8{};
+    else
+      qf[ks] = dl < kG ? *reinterpret_cast<const bf16x8*>(a.query + b * a.q_row + (g * kG + dl) * a.q_head + 32 * ks + 8 * r)
+                       : bf16x8{};
+  }
+}
+
+// One head's 8 dims of the kStripes stripe states, joined in stripe order (log-sum-exp).
+struct StripeMerge {
+  float m[kStripes], l[kStripes];
+  float4 x[kStripes], y[kStripes];
+  __device__ __forceinline__ void store(uint16_t* dst) const {
+    float M = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < kStripes; ++v) M = fmaxf(M, m[v]);
+    float L = 0.0f, o[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[d] = 0.0f;
+#pragma unroll
+    for (int v = 0; v < kStripes; ++v) {
+      const float e = m[v] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[v] - M);
+      L += e * l[v];
+      o[0] += e * x[v].x; o[1] += e * x[v].y; o[2] += e * x[v].z; o[3] += e * x[v].w;
+      o[4] += e * y[v].x; o[5] += e * y[v].y; o[6] += e * y[v].z; o[7] += e * y[v].w;
+    }
+    store_bf16x8(dst, o, 1.0f / L);
+  }
+};
+
+// kWaves stripes per workgroup: kStripes (rows written here) or kStripeWaves (states to the workspace).
+template <int kKvHeads, int kG, bool kFused, int kWaves>
+__global__ __launch_bounds__(64 * kWaves, 2) void paged_decode_stripe_kernel(const DecodeArgs a) {
+  constexpr int kRowElems = kKvHeads * kHeadDim;
+  constexpr int kBlockElems = kBlockSize * kRowElems;
+  static_assert(kG <= 8, "a stripe's merged rows overlay its K staging");
+  // Each wavefront's K staging; its output rows overlay it after the last block.
+  __shared__ __align__(16) uint16_t s_kst[kWaves][kBlockSize * kKStageRow];
+  __shared__ float s_ml[kWaves][kG][2];
+  __shared__ __align__(16) uint16_t s_q[kFused ? kG + 1 : 1][kHeadDim];
+  const SeqUnit unit = seq_unit<kKvHeads>(a.batch);
+  const int g = unit.g, b = unit.b;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int dl = lane & 15;
+  const int r = lane >> 4;
+  const int stripe = unit.split * kWaves + w;
+
+  // Lane i holds the id of block stripe + kStripes i (ids outside the pool read block 0; entries past
+  // the table repeat its last one and are not used).
+  int64_t id = a.block_tables[b * a.bt_stride + min(stripe + kStripes * lane, a.max_blocks - 1)];
+  const int64_t ctx = a.context_lens[b * a.ctx_stride];
+  Prologue<kKvHeads, kG, kWaves> pro;
+  if constexpr (kFused) pro.load(a, b, g, w, r, dl);
+  const int n = static_cast<int>(min(ctx, static_cast<int64_t>(a.max_blocks) * kBlockSize));
   const int nblk = blocks_of(n);
+  if (id < 0 || id >= a.num_blocks) id = 0;
+  const uint32_t id_lo = static_cast<uint32_t>(id), id_hi = static_cast<uint32_t>(static_cast<uint64_t>(id) >> 32);
+  const int cnt = nblk > stripe ? (nblk - 1 - stripe) / kStripes + 1 : 0;  // blocks stripe + kStripes i, i < cnt <= 64
+
+  // Byte offsets of the lane's first pieces inside a block (the block's base address is uniform).
+  const uint32_t k_off = 2u * (r * kRowElems + g * kHeadDim + 8 * dl);
+  const uint32_t v_off = 2u * (4 * r * kRowElems + g * kHeadDim + 8 * dl);
+  u32x4 kbuf[kStripeDepth][4], vbuf[kStripeDepth][4];
+  auto issue = [&](int ring, int i) {
+    const uint32_t blo = __builtin_amdgcn_readlane(id_lo, i);
+    const uint32_t bhi = __builtin_amdgcn_readlane(id_hi, i);
+    const int64_t base = static_cast<int64_t>((static_cast<uint64_t>(bhi) << 32) | blo) * kBlockElems;
+    const char* kp = reinterpret_cast<const char*>(a.key_pool + base);
+    const char* vp = reinterpret_cast<const char*>(a.value_pool + base);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) kbuf[ring][t] = load_vec<kNtLoads>(reinterpret_cast<const u32x4*>(kp + t * 8 * kRowElems + k_off));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) vbuf[ring][t] = load_vec<kNtLoads>(reinterpret_cast<const u32x4*>(vp + t * 2 * kRowElems + v_off));
+  };
+#pragma unroll
+  for (int s = 0; s < kStripeDepth - 1; ++s)
+    if (s < cnt) issue(s, s);  // wave-uniform; in flight during the prologue
+
+  uint64_t slot_lanes = 0;  // lanes whose block holds the new token's slot
+  if constexpr (kFused) {
+    pro.run(a, g, w, r, dl, unit.split == 0, s_q);
+    if (pro.slot >= 0) slot_lanes = __builtin_amdgcn_ballot_w64(id == (pro.slot >> 4));
+  }
+  uint16_t* out_b = a.out + b * a.out_row + (g * kG) * kHeadDim;  // query heads g kG .. g kG + kG - 1
+  if (nblk == 0) {  // empty context: zero rows (uniform over the workgroup)
+    if (unit.split == 0)
+      for (int i = threadIdx.x; i < kG * 16; i += 64 * kWaves) *reinterpret_cast<uint4*>(out_b + 8 * i) = uint4{0, 0, 0, 0};
+    return;
+  }
+  bf16x8 qf[4];
+  query_fragments<kG, kFused>(a, b, g, r, dl, s_q, qf);
+  MfmaState ms;
+  ms.m = -INFINITY;
+  ms.l = 0.0f;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) ms.o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int i0 = 0; i0 < cnt; i0 += kStripeDepth) {
+#pragma unroll
+    for (int s = 0; s < kStripeDepth; ++s) {
+      const int i = i0 + s;
+      if (i >= cnt) break;  // wave-uniform
+      if (i + kStripeDepth - 1 < cnt) issue((s + kStripeDepth - 1) % kStripeDepth, i + kStripeDepth - 1);
+      if constexpr (kFused) {
+        if ((slot_lanes >> i) & 1) {  // the new token's rows in place of what was loaded
+          const int t = static_cast<int>(pro.slot & 15);
+          const u32x4 kn = *reinterpret_cast<const u32x4*>(&s_q[kFused ? kG : 0][8 * dl]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            kbuf[s][e] = 4 * e + r == t ? kn : kbuf[s][e];
+            vbuf[s][e] = 4 * r + e == t ? pro.v : vbuf[s][e];
+          }
+        }
+      }
+      attend_block_mfma(ms, qf, kbuf[s], vbuf[s], s_kst[w], a.scale, (stripe + kStripes * i) * kBlockSize, n, lane);
+    }
+  }
+
+  // Lane: heads 4 r + i, dims 8 dl .. +8; head j's max and sum live in lane j.
+  const float lsum = xsum32_f32(xsum16_f32(ms.l));
+  float* s_acc = reinterpret_cast<float*>(s_kst[w]);  // [kG][128]
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int j = 4 * r + i;
+    const float Lj = __shfl(lsum, j);
+    const float Mj = __shfl(ms.m, j);
+    if (j >= kG) continue;
+    float4 lo4 = make_float4(ms.o[0][i], ms.o[1][i], ms.o[2][i], ms.o[3][i]);
+    float4 hi4 = make_float4(ms.o[4][i], ms.o[5][i], ms.o[6][i], ms.o[7][i]);
+    float4* dst;
+    float* ml;
+    if constexpr (kWaves == kStripes) {
+      dst = reinterpret_cast<float4*>(s_acc + j * kHeadDim + 8 * dl);
+      ml = s_ml[w][j];
+    } else {
+      const int64_t at = (static_cast<int64_t>(b) * kStripes + stripe) * (kKvHeads * kG) + g * kG + j;
+      dst = reinterpret_cast<float4*>(a.ws_acc + at * kHeadDim + 8 * dl);
+      ml = a.ws_ml + at * 2;
+    }
+    dst[0] = lo4;
+    dst[1] = hi4;
+    if (dl == 0) {
+      ml[0] = Mj;
+      ml[1] = Lj;
+    }
+  }
+  if constexpr (kWaves == kStripes) {
+    __syncthreads();
+    if (threadIdx.x < kG * 16) {
+      const int h = threadIdx.x >> 4, dm = threadIdx.x & 15;
+      StripeMerge sm;
+#pragma unroll
+      for (int v = 0; v < kStripes; ++v) {
+        const float4* src = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(s_kst[v]) + h * kHeadDim + 8 * dm);
+        sm.m[v] = s_ml[v][h][0];
+        sm.l[v] = s_ml[v][h][1];
+        sm.x[v] = src[0];
+        sm.y[v] = src[1];
+      }
+      sm.store(out_b + h * kHeadDim + 8 * dm);
+    }
+  }
+}
+
+// The merge launch of spread stripes: one thread per (query head of the KV head, 8 dims), every load
+// issued at once; empty contexts have been written.
+template <int kKvHeads, int kG>
+__global__ __launch_bounds__(kG * 16 < 64 ? 64 : kG * 16) void paged_decode_stripe_merge_kernel(const DecodeArgs a) {
+  const int b = blockIdx.x, g = blockIdx.y;
+  const int h = min(static_cast<int>(threadIdx.x) >> 4, kG - 1), dm = threadIdx.x & 15;
+  StripeMerge sm;
+  const int64_t n = context_of(a, b);
+#pragma unroll
+  for (int v = 0; v < kStripes; ++v) {
+    const int64_t at = (static_cast<int64_t>(b) * kStripes + v) * (kKvHeads * kG) + g * kG + h;
+    const float2 ml = *reinterpret_cast<const float2*>(a.ws_ml + at * 2);
+    const float4* src = reinterpret_cast<const float4*>(a.ws_acc + at * kHeadDim + 8 * dm);
+    sm.m[v] = ml.x;
+    sm.l[v] = ml.y;
+    sm.x[v] = src[0];
+    sm.y[v] = src[1];
+  }
+  if (n <= 0 || threadIdx.x >= kG * 16) return;
+  sm.store(a.out + b * a.out_row + (g * kG + h) * kHeadDim + 8 * dm);
+}
+
+// ---- Parts.  Part p is the a.part_blocks table blocks from p part_blocks on (those inside the context),
+// so that its block ids do not wait for the context length.  Its kPartWaves wavefronts take pairs of
+// blocks w, w + kPartWaves, ... (32 tokens a step), each pair's K registers loaded again as soon as they
+// are in LDS and its V registers as soon as they are multiplied, then merge their states through LDS.
+// kb / vb: the lane's K pieces (token 4 i + r of each block, dims 8 dl .. +8: whole 256-byte rows per
+// instruction) and V pieces (token 4 r + i).  kst: the wavefront's 32-row K staging in LDS, through
+// which K reaches the MFMA A layout.
+//  * S^T = K Q^T per block as in attend_block_mfma; lane: head dl, tokens 4 r + i of both blocks.
+//  * O += P V in one v_mfma_f32_16x16x32_bf16 per output tile: k index 8 r + e is token 4 r + e of the
+//    first block for e < 4, token 4 r + e - 4 of the second for the rest, so P and V both stay in the
+//    lanes that hold them.
+__device__ __forceinline__ void stage_pair(const u32x4 (&kb)[2][4], uint16_t* kst, int lane) {
+  const int dl = lane & 15, r = lane >> 4;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x4*>(kst + (kBlockSize * h + 4 * i + r) * kKStageRow + 8 * dl) = kb[h][i];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Probabilities of the staged pair (first token tok_base, tokens from n on masked) as the A operand.
+__device__ __forceinline__ bf16x8 pair_probs(MfmaState& st, const bf16x8 (&qf)[4], const uint16_t* kst, float scale,
+                                             int tok_base, int n, int lane) {
+  const int dl = lane & 15, r = lane >> 4;
+  f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          *reinterpret_cast<const bf16x8*>(kst + (kBlockSize * h + dl) * kKStageRow + 32 * ks + 8 * r), qf[ks], acc[h],
+          0, 0, 0);
+  // The next pair's staging stores follow these reads in the wavefront's LDS order.
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  float sc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sc[e] = score_log2(acc[e >> 2][e & 3], scale);
+  if (tok_base + kPairTokens > n) {  // uniform
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sc[e] = tok_base + kBlockSize * (e >> 2) + 4 * r + (e & 3) < n ? sc[e] : -INFINITY;
+  }
+  float mb = sc[0];
+#pragma unroll
+  for (int e = 1; e < 8; ++e) mb = fmaxf(mb, sc[e]);
+  if (__builtin_amdgcn_ballot_w64(mb > st.m + kRescaleSlack) != 0) {  // lazy rescale (wave-uniform)
+    const float nm = fmaxf(st.m, xmax32(xmax16(mb)));
+    const float al = (nm == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(st.m - nm);
+    st.m = nm;
+    st.l *= al;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // O rows are heads 4 r + i: lane h holds head h's factor
+      const float ai = __shfl(al, 4 * r + i);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) st.o[t][i] *= ai;
+    }
+  }
+  const float ref = st.m == -INFINITY ? 0.0f : st.m;
+  f32x8 p;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) p[e] = __builtin_amdgcn_exp2f(sc[e] - ref);
+  st.l += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+  return __builtin_convertvector(p, bf16x8);
+}
+
+__device__ __forceinline__ void pair_values(MfmaState& st, const bf16x8 pa, const u32x4 (&vb)[2][4]) {
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
+    u32x4 v;  // tokens 0, 1 | 2, 3 of the first block, then of the second, at dim t
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      v[2 * h] = __builtin_amdgcn_perm(vb[h][1][t >> 1], vb[h][0][t >> 1], sel);
+      v[2 * h + 1] = __builtin_amdgcn_perm(vb[h][3][t >> 1], vb[h][2][t >> 1], sel);
+    }
+    st.o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, __builtin_bit_cast(bf16x8, v), st.o[t], 0, 0, 0);
+  }
+}
+
+// Three wavefronts per SIMD (a budget of 128 registers would spill: 2-3 times slower).
+template <int kKvHeads, int kG, bool kFused>
+__global__ __launch_bounds__(64 * kPartWaves, 3) void paged_decode_parts_kernel(const DecodeArgs a) {
+  constexpr int kRowElems = kKvHeads * kHeadDim;
+  constexpr int kBlockElems = kBlockSize * kRowElems;
+  static_assert(kG <= 16, "at most 16 query heads per KV head");
+  // Each wavefront's K staging; its merged output rows overlay it after the last pair.
+  constexpr int kStageElems = kPairTokens * kKStageRow;
+  static_assert(kStageElems * sizeof(uint16_t) >= kG * kHeadDim * sizeof(float), "the output rows fit the staging");
+  __shared__ __align__(16) uint16_t s_kst[kPartWaves][kStageElems];
+  __shared__ float s_ml[kPartWaves][kG][2];
+  __shared__ __align__(16) uint16_t s_q[kFused ? kG + 1 : 1][kHeadDim];
+  const SeqUnit unit = seq_unit<kKvHeads>(a.batch);
+  const int g = unit.g, b = unit.b, part = unit.split;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int dl = lane & 15;
+  const int r = lane >> 4;
+  const int lo = part * a.part_blocks;
+
+  // Lane 2 j + h holds the id of block h of the wavefront's pair j (ids outside the pool read block 0).
+  // Entries past the table repeat its last one (not used).
+  const int my_blk = lo + 2 * (w + kPartWaves * (lane >> 1)) + (lane & 1);
+  int64_t id = a.block_tables[b * a.bt_stride + min(my_blk, a.max_blocks - 1)];
+  const int64_t ctx = a.context_lens[b * a.ctx_stride];
+  Prologue<kKvHeads, kG, kPartWaves> pro;
+  if constexpr (kFused) pro.load(a, b, g, w, r, dl);
+  const int n = static_cast<int>(min(ctx, static_cast<int64_t>(a.max_blocks) * kBlockSize));
+  const int nblk = blocks_of(n);
+  if (part > 0 && lo >= nblk) return;  // uniform
+  if (id < 0 || id >= a.num_blocks) id = 0;
+  const uint32_t id_lo = static_cast<uint32_t>(id), id_hi = static_cast<uint32_t>(static_cast<uint64_t>(id) >> 32);
+  const int hi = min(lo + a.part_blocks, nblk);
+  const int tok_end = min(n, hi * kBlockSize);
+  const int pairs = (hi - lo + 1) / 2;
+  const int cnt = pairs > w ? (pairs - 1 - w) / kPartWaves + 1 : 0;  // pairs w + kPartWaves j, j < cnt <= 32
+
+  // Byte offsets of the lane's first pieces inside a block (the block's base address is uniform).
+  const uint32_t k_off = 2u * (r * kRowElems + g * kHeadDim + 8 * dl);
+  const uint32_t v_off = 2u * (4 * r * kRowElems + g * kHeadDim + 8 * dl);
+  u32x4 kb[2][4], vb[2][4];
+  // The lane that holds block h of pair j; past the part's end that of the block before (masked).
+  auto id_lane = [&](int j, int h) { return 2 * j + ((lo + 2 * (w + kPartWaves * j) + h < hi) ? h : 0); };
+  auto block_id = [&](int j, int h) {
+    const int i = id_lane(j, h);
+    const uint32_t blo = __builtin_amdgcn_readlane(id_lo, i);
+    const uint32_t bhi = __builtin_amdgcn_readlane(id_hi, i);
+    return static_cast<int64_t>((static_cast<uint64_t>(bhi) << 32) | blo);
+  };
+  auto load_keys = [&](int j) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const char* kp = reinterpret_cast<const char*>(a.key_pool + block_id(j, h) * kBlockElems);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) kb[h][t] = load_vec<kNtLoads>(reinterpret_cast<const u32x4*>(kp + t * 8 * kRowElems + k_off));
+    }
+  };
+  auto load_values = [&](int j) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const char* vp = reinterpret_cast<const char*>(a.value_pool + block_id(j, h) * kBlockElems);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) vb[h][t] = load_vec<kNtLoads>(reinterpret_cast<const u32x4*>(vp + t * 2 * kRowElems + v_off));
+    }
+  };
+  if (cnt > 0) {  // wave-uniform
+    load_keys(0);
+    load_values(0);
+  }
+
+  uint64_t slot_lanes = 0;  // lanes whose block holds the new token's slot
+  if constexpr (kFused) {
+    pro.run(a, g, w, r, dl, part == 0, s_q);
+    if (pro.slot >= 0) slot_lanes = __builtin_amdgcn_ballot_w64(id == (pro.slot >> 4));
+  }
   uint16_t* out_b = a.out + b * a.out_row + (g * kG) * kHeadDim;  // query heads g kG .. g kG + kG - 1
   if (nblk == 0) {  // empty context: zero rows (uniform over the workgroup)
     if (threadIdx.x < kG * 16) *reinterpret_cast<uint4*>(out_b + 8 * threadIdx.x) = uint4{0, 0, 0, 0};
     return;
   }
-  const float scale = a.scale;
-  constexpr bool kMfma = kMfmaForm;  // lane layout and per-block arithmetic as in the stream kernel
-  static_assert(kG <= 16, "at most 16 query heads per KV head");
-  const int k_off = r * kRowElems + g * kHeadDim + 8 * dl;
-  const int v_off = kMfma ? 4 * r * kRowElems + g * kHeadDim + 8 * dl : k_off;
-  constexpr int kKStep = 4 * kRowElems;
-  constexpr int kVStep = kMfma ? kRowElems : 4 * kRowElems;
-  const int cnt = nblk > w ? (nblk - 1 - w) / kSeqWaves + 1 : 0;  // blocks w + kSeqWaves i, i < cnt <= 64
-
-  // Lane i holds the id of block w + kSeqWaves i (ids outside the pool read block 0).
-  uint32_t id_lo = 0, id_hi = 0;
-  if (lane < cnt) {
-    int64_t id = a.block_tables[b * a.bt_stride + w + kSeqWaves * lane];
-    if (id < 0 || id >= a.num_blocks) id = 0;
-    id_lo = static_cast<uint32_t>(id);
-    id_hi = static_cast<uint32_t>(static_cast<uint64_t>(id) >> 32);
-  }
-  uint4 q[kMfma ? 1 : kG];
   bf16x8 qf[4];
-  RowState<kMfma ? 1 : kG> st;
+  query_fragments<kG, kFused>(a, b, g, r, dl, s_q, qf);
   MfmaState ms;
-  if constexpr (kMfma) {  // Q^T fragments: head dl (zero past the group), dims 32 ks + 8 r .. +8
+  ms.m = -INFINITY;
+  ms.l = 0.0f;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if constexpr (kFused)
-        qf[ks] = dl < kG ? *reinterpret_cast<const bf16x8*>(&s_q[dl < kG ? dl : 0][32 * ks + 8 * r]) : bf16x8{};
-      else
-        qf[ks] = dl < kG ? *reinterpret_cast<const bf16x8*>(a.query + b * a.q_row + (g * kG + dl) * a.q_head +
-                                                            32 * ks + 8 * r)
-                         : bf16x8{};
-    }
-    ms.m = -INFINITY;
-    ms.l = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) ms.o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  } else {
-#pragma unroll
-    for (int j = 0; j < kG; ++j) {
-      if constexpr (kFused)
-        q[j] = *reinterpret_cast<const uint4*>(&s_q[j][8 * dl]);
-      else
-        q[j] = *reinterpret_cast<const uint4*>(a.query + b * a.q_row + (g * kG + j) * a.q_head + 8 * dl);
-    }
-    st.init();
-  }
+  for (int t = 0; t < 8; ++t) ms.o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  u32x4 kbuf[kSeqDepth][4], vbuf[kSeqDepth][4];
-  auto issue = [&](int slot, int i) {  // block w + kSeqWaves i, clamped to the wavefront's last
-    i = min(i, cnt - 1);
-    const uint32_t blo = __builtin_amdgcn_readlane(id_lo, i);
-    const uint32_t bhi = __builtin_amdgcn_readlane(id_hi, i);
-    const int64_t base = static_cast<int64_t>((static_cast<uint64_t>(bhi) << 32) | blo) * kBlockElems;
-    const uint16_t* kp = a.key_pool + base + k_off;
-    const uint16_t* vp = a.value_pool + base + v_off;
+  uint16_t* kst = s_kst[w];
+  const float scale = a.scale;
+  // The new token's rows in place of what was loaded from its slot (wave-uniform branch).
+  auto in_slot_block = [&](int j, int h) { return (slot_lanes >> id_lane(j, h)) & 1; };
+  auto patch_keys = [&](int j) {
+    if constexpr (kFused) {
+      const int t = static_cast<int>(pro.slot & 15);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) kbuf[slot][t] = load_vec<kNtLoads>(reinterpret_cast<const u32x4*>(kp + t * kKStep));
+      for (int h = 0; h < 2; ++h) {
+        if (!in_slot_block(j, h)) continue;
+        const u32x4 kn = *reinterpret_cast<const u32x4*>(&s_q[kFused ? kG : 0][8 * dl]);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) vbuf[slot][t] = load_vec<kNtLoads>(reinterpret_cast<const u32x4*>(vp + t * kVStep));
+        for (int i = 0; i < 4; ++i) kb[h][i] = 4 * i + r == t ? kn : kb[h][i];
+      }
+    }
   };
-  if (cnt > 0) {  // wave-uniform
+  auto patch_values = [&](int j) {
+    if constexpr (kFused) {
+      const int t = static_cast<int>(pro.slot & 15);
 #pragma unroll
-    for (int s = 0; s < kSeqDepth - 1; ++s) issue(s, s);  // ring slot of block i: i % kSeqDepth
-    if (kSeqDepth == 1) issue(0, 0);
-    // Whole rounds of kSeqDepth blocks, so that the loads stay in straight-line code the compiler
-    // can count: indices past cnt re-read the last block and mask all its tokens (block
-    // w + kSeqWaves i >= nblk starts at or past the context end).
-    for (int i0 = 0; i0 < cnt; i0 += kSeqDepth) {
+      for (int h = 0; h < 2; ++h) {
+        if (!in_slot_block(j, h)) continue;
 #pragma unroll
-      for (int s = 0; s < kSeqDepth; ++s) {
-        const int i = i0 + s;
-        if (kSeqDepth > 1) issue((s + kSeqDepth - 1) % kSeqDepth, i + kSeqDepth - 1);
-        else if (i > 0) issue(0, i);
-        if constexpr (kMfma)
-          attend_block_mfma(ms, qf, kbuf[s], vbuf[s], s_kst[w], scale, (w + kSeqWaves * i) * kBlockSize, n, lane);
-        else
-          attend_block<kG>(st, q, kbuf[s], vbuf[s], scale, (w + kSeqWaves * i) * kBlockSize, n, r);
+        for (int i = 0; i < 4; ++i) vb[h][i] = 4 * r + i == t ? pro.v : vb[h][i];
       }
     }
+  };
+  auto tok_base = [&](int j) { return (lo + 2 * (w + kPartWaves * j)) * kBlockSize; };
+  for (int j = 0; j + 1 < cnt; ++j) {
+    patch_keys(j);
+    stage_pair(kb, kst, lane);
+    load_keys(j + 1);
+    const bf16x8 pa = pair_probs(ms, qf, kst, scale, tok_base(j), tok_end, lane);
+    patch_values(j);
+    pair_values(ms, pa, vb);
+    load_values(j + 1);
+  }
+  if (cnt > 0) {
+    patch_keys(cnt - 1);
+    stage_pair(kb, kst, lane);
+    const bf16x8 pa = pair_probs(ms, qf, kst, scale, tok_base(cnt - 1), tok_end, lane);
+    patch_values(cnt - 1);
+    pair_values(ms, pa, vb);
   }
 
-  // ---- merge the four rows of the wavefront (log-sum-exp), then the wavefronts through LDS
-  if constexpr (kMfma) {  // lane: heads 4 r + i, dims 8 dl .. +8; head j's max and sum live in lane j
-    float lsum = ms.l + __shfl_xor(ms.l, 16);
-    lsum += __shfl_xor(lsum, 32);
+  // ---- merge the wavefronts through LDS (log-sum-exp).  Lane: heads 4 r + i, dims 8 dl .. +8; head
+  // j's max and sum live in lane j.
+  float* s_acc = reinterpret_cast<float*>(kst);  // [kG][128]
+  const float lsum = xsum32_f32(xsum16_f32(ms.l));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int j = 4 * r + i;
-      const float Lj = __shfl(lsum, j);
-      const float Mj = __shfl(ms.m, j);
-      if (j >= kG) continue;
+  for (int i = 0; i < 4; ++i) {
+    const int j = 4 * r + i;
+    const float Lj = __shfl(lsum, j);
+    const float Mj = __shfl(ms.m, j);
+    if (j >= kG) continue;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) s_acc[w][j][8 * dl + t] = ms.o[t][i];
-      if (dl == 0) {
-        s_ml[w][j][0] = Mj;
-        s_ml[w][j][1] = Lj;
-      }
-    }
-  }
-  float M[kMfma ? 1 : kG];
-  if constexpr (!kMfma) merge_rows<kG>(st, M);
-#pragma unroll
-  for (int j = 0; j < (kMfma ? 0 : kG); ++j) {  // row r holds heads j = r, r + 4, ... (every row has all after the merge)
-    if ((j & 3) != r) continue;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) s_acc[w][j][8 * dl + d] = st.acc[j][d];
+    for (int t = 0; t < 8; ++t) s_acc[j * kHeadDim + 8 * dl + t] = ms.o[t][i];
     if (dl == 0) {
-      s_ml[w][j][0] = M[j];
-      s_ml[w][j][1] = st.l[j];
+      s_ml[w][j][0] = Mj;
+      s_ml[w][j][1] = Lj;
     }
   }
   __syncthreads();
@@ -814,11 +1155,161 @@ __global__ __launch_bounds__(64 * kSeqWaves) void paged_decode_seq_kernel(const 
     const int h = threadIdx.x >> 4;
     const int dm = threadIdx.x & 15;
     float Mx = -INFINITY;
-    for (int v = 0; v < kSeqWaves; ++v) Mx = fmaxf(Mx, s_ml[v][h][0]);
+#pragma unroll
+    for (int v = 0; v < kPartWaves; ++v) Mx = fmaxf(Mx, s_ml[v][h][0]);
     float L = 0.0f, o[8];
 #pragma unroll
     for (int d = 0; d < 8; ++d) o[d] = 0.0f;
-    for (int v = 0; v < kSeqWaves; ++v) {
+#pragma unroll
+    for (int v = 0; v < kPartWaves; ++v) {
+      const float mv = s_ml[v][h][0];
+      const float e = mv == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mv - Mx);
+      L += e * s_ml[v][h][1];
+      const float4* src = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(s_kst[v]) + h * kHeadDim + 8 * dm);
+      const float4 x = src[0], y = src[1];
+      o[0] += e * x.x; o[1] += e * x.y; o[2] += e * x.z; o[3] += e * x.w;
+      o[4] += e * y.x; o[5] += e * y.y; o[6] += e * y.z; o[7] += e * y.w;
+    }
+    if (nblk <= a.part_blocks) {  // in one part
+      store_bf16x8(out_b + h * kHeadDim + 8 * dm, o, 1.0f / L);
+    } else {
+      const int64_t at = (static_cast<int64_t>(b) * a.splits + part) * (kKvHeads * kG) + g * kG + h;
+      float4* dst = reinterpret_cast<float4*>(a.ws_acc + at * kHeadDim + 8 * dm);
+      dst[0] = make_float4(o[0], o[1], o[2], o[3]);
+      dst[1] = make_float4(o[4], o[5], o[6], o[7]);
+      if (dm == 0) *reinterpret_cast<float2*>(a.ws_ml + at * 2) = make_float2(Mx, L);
+    }
+  }
+}
+
+// ---- The merge launch: one workgroup per (sequence, KV head) joins the partials its sequence left
+// (log-sum-exp) and writes the bf16 rows; a sequence in one piece has been written already.
+//  * stream kernel (kParts false): a sequence cut by range boundaries left the first range's
+//    last-sequence slot, then the first-sequence slot of every later range up to the one holding its
+//    last block; empty contexts get their zero rows here.
+//  * parts kernel (kParts true): slot b splits + part for each part (that kernel writes the zero rows
+//    itself).
+// A launch of a few microseconds is a chain of latencies, so it is kept short: 16 lanes cover the
+// 128 dims and 16 partials are read side by side, every head's loads before any is used, with
+// one reduction over the contexts (stream form) and 32-bit range arithmetic.
+constexpr int kMergeThreads = 256;
+constexpr int kMergeRows = kMergeThreads / 16;  // partials read side by side
+
+template <int kKvHeads, int kG, bool kParts>
+__global__ __launch_bounds__(kMergeThreads) void paged_decode_merge_kernel(const DecodeArgs a) {
+  constexpr int kHeads = kKvHeads * kG;
+  constexpr int kWaves = kMergeThreads / 64;
+  __shared__ float s_acc[kWaves][kG][kHeadDim];
+  __shared__ float s_ml[kWaves][kG][2];
+  const int b = blockIdx.x, g = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int dm = tid & 15, row = tid >> 4;
+  uint16_t* out_b = a.out + b * a.out_row + g * kG * kHeadDim;
+  // Partial p of the sequence, this lane's 8 dims of every head.
+  float2 ml[kG];
+  float4 x[kG], y[kG];
+  auto load_partial = [&](int64_t slot) {
+    const int64_t unit = slot * kHeads + g * kG;
+#pragma unroll
+    for (int j = 0; j < kG; ++j) {
+      ml[j] = *reinterpret_cast<const float2*>(a.ws_ml + (unit + j) * 2);
+      const float4* src = reinterpret_cast<const float4*>(a.ws_acc + (unit + j) * kHeadDim + 8 * dm);
+      x[j] = src[0];
+      y[j] = src[1];
+    }
+  };
+  const int64_t ctx = context_of(a, b);
+  int first = 0, count;  // partials [first, first + count)
+  if constexpr (kParts) {
+    // The first round goes out beside the context (slots no part wrote are read and not used).
+    load_partial(static_cast<int64_t>(b) * a.splits + min(row, a.splits - 1));
+    count = (blocks_of(ctx) + a.part_blocks - 1) / a.part_blocks;
+  } else {
+    __shared__ int s_sum[kWaves][2];
+    const int nblk = blocks_of(ctx);
+    int before = 0, total = 0;  // blocks of the sequences before b, and of all
+    for (int i = tid; i < a.batch; i += kMergeThreads) {
+      const int v = blocks_of(context_of(a, i));
+      total += v;
+      before += i < b ? v : 0;
+    }
+    before = wave_sum_i32(before);
+    total = wave_sum_i32(total);
+    if (lane == 0) {
+      s_sum[w][0] = before;
+      s_sum[w][1] = total;
+    }
+    __syncthreads();
+    before = total = 0;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) {
+      before += s_sum[v][0];
+      total += s_sum[v][1];
+    }
+    if (nblk == 0) {  // uniform
+      if (tid < kG * 16) *reinterpret_cast<uint4*>(out_b + 8 * tid) = uint4{0, 0, 0, 0};
+      return;
+    }
+    const Ranges rg(total, a.streams);
+    first = rg.of(before);
+    count = rg.of(before + nblk - 1) - first + 1;
+  }
+  if (count <= 1) return;  // uniform: written by the attention kernel
+
+  float m[kG], l[kG], acc[kG][8];
+#pragma unroll
+  for (int j = 0; j < kG; ++j) {
+    m[j] = -INFINITY;
+    l[j] = 0.0f;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[j][d] = 0.0f;
+  }
+  for (int p = row; p < count; p += kMergeRows) {
+    if (!kParts)
+      load_partial(static_cast<int64_t>(first + p) * 2 + (p == 0 ? 1 : 0));
+    else if (p >= kMergeRows)
+      load_partial(static_cast<int64_t>(b) * a.splits + p);
+#pragma unroll
+    for (int j = 0; j < kG; ++j) {
+      const float nm = fmaxf(m[j], ml[j].x);
+      const float e0 = m[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j] - nm);
+      const float e1 = ml[j].x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml[j].x - nm);
+      m[j] = nm;
+      l[j] = e0 * l[j] + e1 * ml[j].y;
+      const float v[8] = {x[j].x, x[j].y, x[j].z, x[j].w, y[j].x, y[j].y, y[j].z, y[j].w};
+#pragma unroll
+      for (int d = 0; d < 8; ++d) acc[j][d] = e0 * acc[j][d] + e1 * v[d];
+    }
+  }
+  // The wavefront's four rows, then the wavefronts through LDS.
+#pragma unroll
+  for (int j = 0; j < kG; ++j) {
+    const float mx = xmax32(xmax16(m[j]));
+    const float e = m[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j] - mx);
+    const float ls = xsum32_f32(xsum16_f32(l[j] * e));
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[j][d] = xsum32_f32(xsum16_f32(acc[j][d] * e));
+    if (lane < 16) {
+#pragma unroll
+      for (int d = 0; d < 8; ++d) s_acc[w][j][8 * dm + d] = acc[j][d];
+      if (dm == 0) {
+        s_ml[w][j][0] = mx;
+        s_ml[w][j][1] = ls;
+      }
+    }
+  }
+  __syncthreads();
+  if (tid < kG * 16) {
+    const int h = row;
+    float Mx = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) Mx = fmaxf(Mx, s_ml[v][h][0]);
+    float L = 0.0f, o[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[d] = 0.0f;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) {
       const float mv = s_ml[v][h][0];
       const float e = mv == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mv - Mx);
       L += e * s_ml[v][h][1];
@@ -827,86 +1318,6 @@ __global__ __launch_bounds__(64 * kSeqWaves) void paged_decode_seq_kernel(const 
     }
     store_bf16x8(out_b + h * kHeadDim + 8 * dm, o, 1.0f / L);
   }
-}
-
-// Finishes what the stream kernel left: sequences cut by a range boundary (merge of their
-// partials: the cut range's last-sequence slot, then the first-sequence slot of every later
-// range up to the one holding the sequence's last block) and empty contexts (zero rows).
-// grid: batch; block: heads * 16 lanes rounded up to whole wavefronts, lane (h, dm) < heads * 16
-// owns dims [8 dm, 8 dm + 8) of head h.
-template <int kHeads>
-constexpr int merge_threads() { return (kHeads * 16 + 63) / 64 * 64; }
-
-template <int kHeads>
-__global__ __launch_bounds__(merge_threads<kHeads>()) void paged_decode_merge_kernel(const DecodeArgs a) {
-  constexpr int kThreads = merge_threads<kHeads>();
-  extern __shared__ int s_off[];
-  __shared__ int s_wave[kThreads / 64];
-  const int total = scan_blocks<kThreads>(a, s_off, s_wave);
-  const int b = blockIdx.x;
-  if (threadIdx.x >= kHeads * 16) return;
-  const int h = threadIdx.x >> 4;
-  const int dm = threadIdx.x & 15;
-  uint16_t* dst = a.out + b * a.out_row + h * kHeadDim + 8 * dm;
-  const int nblk = s_off[b + 1] - s_off[b];
-  if (nblk == 0) {
-    *reinterpret_cast<uint4*>(dst) = uint4{0, 0, 0, 0};
-    return;
-  }
-  const int first = stream_of(s_off[b], total, a.streams);
-  const int last = stream_of(s_off[b + 1] - 1, total, a.streams);
-  if (first == last) return;  // written by the stream kernel
-  // Partials: the first range's last-sequence slot (1), then the first-sequence slot (0) of each
-  // later non-empty range up to `last` (empty ranges -- fewer blocks than ranges -- wrote nothing).
-  auto slot_of = [&](int k) -> int64_t { return (static_cast<int64_t>(k) * 2 + (k == first ? 1 : 0)) * kHeads + h; };
-  auto empty = [&](int k) {
-    return static_cast<int64_t>(k) * total / a.streams >= static_cast<int64_t>(k + 1) * total / a.streams;
-  };
-  // kMergeUnroll partials per step with independent loads (a serial chain of dependent loads
-  // would make a launch of many cut sequences latency-bound).
-  constexpr int kMergeUnroll = 4;
-  float M = -INFINITY;
-  for (int k0 = first; k0 <= last; k0 += kMergeUnroll) {
-    float m[kMergeUnroll];
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) {
-      const int k = k0 + u;
-      m[u] = (k <= last && !empty(k)) ? a.ws_ml[slot_of(k) * 2] : -INFINITY;
-    }
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) M = fmaxf(M, m[u]);
-  }
-  float L = 0.0f, acc[8];
-#pragma unroll
-  for (int d = 0; d < 8; ++d) acc[d] = 0.0f;
-  for (int k0 = first; k0 <= last; k0 += kMergeUnroll) {
-    float m[kMergeUnroll], l[kMergeUnroll];
-    float4 xv[kMergeUnroll], yv[kMergeUnroll];
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) {
-      const int k = k0 + u;
-      if (k <= last && !empty(k)) {
-        const int64_t slot = slot_of(k);
-        m[u] = a.ws_ml[slot * 2];
-        l[u] = a.ws_ml[slot * 2 + 1];
-        const float4* src = reinterpret_cast<const float4*>(a.ws_acc + slot * kHeadDim + 8 * dm);
-        xv[u] = src[0];
-        yv[u] = src[1];
-      } else {
-        m[u] = -INFINITY;
-        l[u] = 0.0f;
-        xv[u] = yv[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) {
-      const float w = m[u] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[u] - M);
-      L += w * l[u];
-      acc[0] += w * xv[u].x; acc[1] += w * xv[u].y; acc[2] += w * xv[u].z; acc[3] += w * xv[u].w;
-      acc[4] += w * yv[u].x; acc[5] += w * yv[u].y; acc[6] += w * yv[u].z; acc[7] += w * yv[u].w;
-    }
-  }
-  store_bf16x8(dst, acc, 1.0f / L);
 }
 
 int head_groups_for(int32_t num_kv_heads) {
@@ -925,27 +1336,88 @@ int streams_for(int32_t batch, int32_t max_blocks, int32_t num_kv_heads) {
   return static_cast<int>(s < 1 ? 1 : s);
 }
 
-// The per-sequence kernel serves launches of at most one workgroup per CU with tables it can
-// hold; MI_DECODE_PATH=stream or =seq (environment) forces one kernel where both apply.
+#ifndef MI_DECODE_PART_GROUPS
+#define MI_DECODE_PART_GROUPS 6
+#endif
+#ifndef MI_DECODE_STRIPE_BLOCKS
+#define MI_DECODE_STRIPE_BLOCKS 128
+#endif
+#ifndef MI_DECODE_STRIPE_PAIRS
+#define MI_DECODE_STRIPE_PAIRS 256
+#endif
+// Workgroups per CU that the parts of a launch aim at, by the table's length (contexts fill part of it):
+// 21 sequences lognormal to 8192 took 65 / 62 / 56 / 56 us with 2 / 3 / 6 / 10.
+constexpr int kPartGroupsPerCu = MI_DECODE_PART_GROUPS;
+// Stripes up to this table length and number of (sequence, KV head) pairs: beyond 128 blocks a stripe
+// is a serial chain of more than 16 of them; beyond 256 pairs, parts won (64 sequences of U[32, 1150]
+// 39.5 against 41.7 us, 40 of them 26.0 against 27.1).
+constexpr int kStripeMaxBlocks = MI_DECODE_STRIPE_BLOCKS;
+constexpr int kStripeMaxPairs = MI_DECODE_STRIPE_PAIRS;
+
+// Which small-launch form takes a launch, from its table length and the partials the workspace (sized by
+// streams_for, two slots per range; has_workspace false: none) holds.
+void cut_sequences(DecodeArgs& a, int32_t num_kv_heads, bool has_workspace) {
+  const int64_t pairs = static_cast<int64_t>(a.batch) * num_kv_heads;
+  const int64_t slots = has_workspace ? 2ll * streams_for(a.batch, a.max_blocks, num_kv_heads) / a.batch : 0;
+  a.part_blocks = 0;
+  a.splits = 1;
+  if (a.max_blocks <= kStripeMaxBlocks && pairs <= kStripeMaxPairs) {
+    // Spread where the workspace holds a partial per stripe (tables from 64 blocks on).
+    if (slots >= kStripes) a.splits = kStripes / kStripeWaves;
+    return;
+  }
+  int64_t parts = (static_cast<int64_t>(device_cus()) * kPartGroupsPerCu + pairs - 1) / pairs;
+  parts = parts < slots ? parts : slots;
+  if (parts < 2) return;
+  const int64_t step = 2 * kPartWaves;
+  int64_t blocks = ((a.max_blocks + parts - 1) / parts + step - 1) / step * step;
+  blocks = blocks < kPartMaxBlocks ? blocks : kPartMaxBlocks;
+  a.part_blocks = static_cast<int32_t>(blocks < a.max_blocks ? blocks : a.max_blocks);
+  a.splits = (a.max_blocks + a.part_blocks - 1) / a.part_blocks;
+}
+
+// The per-sequence kernel serves launches of at most one (sequence, KV head) pair per CU, and larger
+// ones while their tables hold no more than kSeqWork (block, KV head) pairs; beyond that the stream
+// kernel's equal ranges win.  Measured, us per layer with the prologue, per-sequence / stream: 40 and 64
+// sequences U[32, 1150] 25.4 / 29.9 and 39.2 / 43.6, 128 of U[32, 400] 28.1 / 35.5, 128 of U[32, 1150]
+// (73,728 pairs) 56-58 / 62; 40 lognormal to 8192 with 5 heads per KV head (163,840 pairs) 112 / 94, 100
+// of them with 2 264 / 216.  MI_DECODE_PATH=stream or =seq (environment) forces one kernel where both
+// apply.
+constexpr int64_t kSeqWork = 98304;
 bool use_seq_path(int32_t batch, int32_t max_blocks, int32_t num_kv_heads) {
   if (max_blocks <= 0 || max_blocks > kSeqMaxBlocks) return false;
   const char* forced = getenv("MI_DECODE_PATH");
   if (forced && strcmp(forced, "stream") == 0) return false;
   if (forced && strcmp(forced, "seq") == 0) return true;
-  return static_cast<int64_t>(batch) * num_kv_heads <= device_cus();
+  const int64_t pairs = static_cast<int64_t>(batch) * num_kv_heads;
+  return pairs <= device_cus() || pairs * max_blocks <= kSeqWork;
 }
 
 template <int kKvHeads, int kG, bool kFused>
 int32_t launch_decode(const DecodeArgs& a, bool seq_path, hipStream_t s) {
   constexpr int kWaves = kKvHeads < kMaxWaves ? kKvHeads : kMaxWaves;
   constexpr int kHeadGroups = kKvHeads / kWaves;
-  constexpr int kHeads = kKvHeads * kG;
-  constexpr int kMergeThreads = merge_threads<kHeads>();
   const size_t lds = sizeof(int) * (static_cast<size_t>(a.batch) + 1);
+  const dim3 pairs(a.batch, kKvHeads);
   if (seq_path) {
     if (a.max_blocks > kSeqMaxBlocks) return fail(MI_ERR_UNSUPPORTED, "mi_paged_decode_attention: table too long");
-    paged_decode_seq_kernel<kKvHeads, kG, kFused><<<dim3(a.batch, kKvHeads), 64 * kSeqWaves, 0, s>>>(a);
-    return check_launch("mi_paged_decode_attention(seq)");
+    const uint32_t groups = static_cast<uint32_t>(a.batch) * a.splits * kKvHeads;
+    if (a.part_blocks > 0) {
+      paged_decode_parts_kernel<kKvHeads, kG, kFused><<<groups, 64 * kPartWaves, 0, s>>>(a);
+      const int32_t rc = check_launch("mi_paged_decode_attention(parts)");
+      if (rc != MI_OK || a.splits == 1) return rc;
+      paged_decode_merge_kernel<kKvHeads, kG, true><<<pairs, kMergeThreads, 0, s>>>(a);
+      return check_launch("mi_paged_decode_attention(merge)");
+    }
+    if (a.splits == 1) {
+      paged_decode_stripe_kernel<kKvHeads, kG, kFused, kStripes><<<groups, 64 * kStripes, 0, s>>>(a);
+      return check_launch("mi_paged_decode_attention(stripes)");
+    }
+    paged_decode_stripe_kernel<kKvHeads, kG, kFused, kStripeWaves><<<groups, 64 * kStripeWaves, 0, s>>>(a);
+    const int32_t rc = check_launch("mi_paged_decode_attention(stripes)");
+    if (rc != MI_OK) return rc;
+    paged_decode_stripe_merge_kernel<kKvHeads, kG><<<pairs, kG * 16 < 64 ? 64 : kG * 16, 0, s>>>(a);
+    return check_launch("mi_paged_decode_attention(merge)");
   }
   if constexpr (kFused) return fail(MI_ERR_UNSUPPORTED, "mi_paged_decode_attention: fused form needs the per-sequence kernel");
   if (a.max_blocks > 0) {
@@ -953,7 +1425,7 @@ int32_t launch_decode(const DecodeArgs& a, bool seq_path, hipStream_t s) {
     int32_t rc = check_launch("mi_paged_decode_attention");
     if (rc != MI_OK) return rc;
   }
-  paged_decode_merge_kernel<kHeads><<<a.batch, kMergeThreads, lds, s>>>(a);
+  paged_decode_merge_kernel<kKvHeads, kG, false><<<pairs, kMergeThreads, 0, s>>>(a);
   return check_launch("mi_paged_decode_attention(merge)");
 }
 
@@ -1070,6 +1542,7 @@ extern "C" int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, 
     a.batch = nb;
     a.max_blocks = max_blocks;
     a.streams = streams;
+    if (seq_path) cut_sequences(a, num_kv_heads, true);
     a.scale = scale;
     a.ws_acc = ws_acc;
     a.ws_ml = ws_ml;
@@ -1097,8 +1570,12 @@ extern "C" int32_t mi_paged_decode_attention_fused(
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention_fused: pool too large");
   if (const int32_t rc = check_heads("mi_paged_decode_attention_fused", num_heads, num_kv_heads, head_dim, block_size))
     return rc;
-  if (!use_seq_path(batch, max_blocks, num_kv_heads) || max_blocks == 0) {
-    // Large launches: the two-launch form (the append and q rotation, then the stream kernel).
+  // The prologue of the per-sequence kernel moves 16-byte pieces of the projection rows and tables.
+  const bool pieces = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(q_weight) && aligned16(k_weight) &&
+                      aligned16(cos) && aligned16(sin) && q_row_stride % 8 == 0 && k_row_stride % 8 == 0 &&
+                      v_row_stride % 8 == 0;
+  if (!use_seq_path(batch, max_blocks, num_kv_heads) || max_blocks == 0 || !pieces) {
+    // The append and q rotation in a launch of their own (large launches; rows of other alignments).
     int32_t rc = mi_qk_norm_rope(q_scratch, nullptr, nullptr, q, q_row_stride, k, k_row_stride, v, v_row_stride,
                                  q_weight, k_weight, cos, sin, batch, num_heads, num_kv_heads, head_dim, eps,
                                  slot_mapping, slot_stride, key_pool, value_pool, num_blocks * block_size, stream);
@@ -1108,7 +1585,7 @@ extern "C" int32_t mi_paged_decode_attention_fused(
                                      max_blocks, context_lens, context_lens_stride, batch, num_heads, num_kv_heads,
                                      head_dim, block_size, scale, workspace, workspace_bytes, stream);
   }
-  // One launch: the per-sequence kernel with the prologue.  Shape checks as in the two entry points.
+  // The per-sequence kernel with the prologue.  Shape checks as in the two entry points.
   if (!out || !key_pool || !value_pool || !context_lens || !block_tables)
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention_fused: null pointer argument");
   if (!aligned16(out) || !aligned16(key_pool) || !aligned16(value_pool) || out_row_stride % 8 != 0)
@@ -1129,6 +1606,13 @@ extern "C" int32_t mi_paged_decode_attention_fused(
   a.batch = batch;
   a.max_blocks = max_blocks;
   a.streams = 1;
+  const int64_t need = mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size);
+  const bool room = workspace && workspace_bytes >= need && aligned16(workspace);
+  cut_sequences(a, num_kv_heads, room);
+  if (room) {
+    a.ws_acc = static_cast<float*>(workspace);
+    a.ws_ml = a.ws_acc + static_cast<int64_t>(streams_for(batch, max_blocks, num_kv_heads)) * 2 * num_heads * kHeadDim;
+  }
   a.scale = scale;
   a.q_raw = static_cast<const uint16_t*>(q);
   a.k_raw = static_cast<const uint16_t*>(k);

@@ -1,0 +1,98 @@
+"""The per-sequence decode kernels (stripes, spread stripes, parts): tables at the length where sequences start to be cut, contexts
+that end inside, at and past part boundaries, and the fused prologue with the new token's slot in the
+first, a middle and the last part.  Fused against the two entry points it stands for, bit for bit (the
+new rows are put in place in registers, not read back from the pool), and against the oracle with the
+tolerance of the decode tests (2e-2 max-abs on bf16 outputs)."""
+
+import pytest
+import torch
+
+from mini_infra_qwen3_amd import data_plane
+from oracle import torch_ref
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-2
+SCALE = 128 ** -0.5
+
+
+def _case(seed, ctx, width, group, kv_heads=8):
+    gen = torch.Generator().manual_seed(seed)
+    num_blocks = 1 + sum(-(-max(n, 1) // 16) for n in ctx) + 4
+    tables = torch.zeros(len(ctx), width, dtype=torch.long)
+    perm = torch.randperm(num_blocks - 1, generator=gen) + 1
+    at = 0
+    for b, n in enumerate(ctx):
+        need = -(-max(n, 1) // 16)
+        tables[b, :need] = perm[at:at + need]
+        at += need
+    kp = torch.randn(num_blocks, 16, kv_heads, 128, generator=gen).to(torch.bfloat16)
+    vp = torch.randn(num_blocks, 16, kv_heads, 128, generator=gen).to(torch.bfloat16)
+    heads = group * kv_heads
+    qkv = torch.randn(len(ctx), (heads + 2 * kv_heads) * 128, generator=gen).to(torch.bfloat16)
+    w = [(1 + 0.1 * torch.randn(128, generator=gen)).to(torch.bfloat16) for _ in range(2)]
+    angle = torch.randn(len(ctx), 128, generator=gen)
+    return kp, vp, tables, qkv, w, angle.cos().to(torch.bfloat16), angle.sin().to(torch.bfloat16)
+
+
+# Widths 32 and 63: stripes in one workgroup, 64 to 128 spread, 129 on parts (72 with 64 rows too); 520 is past the
+# per-sequence kernel.  Contexts: empty, one token, the edges of a 16-token block and of 8-block parts.
+@pytest.mark.parametrize("width,ctx", [
+    (32, [512, 511, 1, 0, 497]),
+    (63, [1000, 3, 0]),
+    (64, [1024, 1009, 0, 15]),
+    (128, [2048, 1]),
+    (129, [2064, 129, 128, 127, 0]),
+    (33, [528, 513, 512, 129, 128, 127, 1, 0]),
+    (72, [1150, 1025, 1024, 255, 256, 257, 17, 16, 15]),
+    (72, [1 + 29 * i % 1150 for i in range(64)]),
+    (512, [8192, 4097, 300]),
+    (520, [8300, 40]),
+])
+@pytest.mark.parametrize("group", [1, 2, 8])
+def test_fused_equals_the_two_entry_points(native_lib, device, width, ctx, group):
+    kp, vp, tables, qkv, (qw, kw), cos, sin = _case(width + group, ctx, width, group)
+    heads, kv = group * 8, 8
+    slots = torch.tensor([int(tables[b, (n - 1) // 16]) * 16 + (n - 1) % 16 if n else -1 for b, n in enumerate(ctx)])
+    # Three rows put their token elsewhere in their own blocks: the first part, and a middle block.
+    slots[0] = int(tables[0, 0]) * 16 + 3
+    if len(ctx) > 2 and ctx[2] > 40:
+        slots[2] = int(tables[2, (ctx[2] - 1) // 32]) * 16 + 15
+    dev = [t.to(device) for t in (kp, vp, tables, qkv, qw, kw, cos, sin, slots)]
+    kp_d, vp_d, tables_d, qkv_d, qw_d, kw_d, cos_d, sin_d, slots_d = dev
+    ctx_d = torch.tensor(ctx).to(device)
+    q, k, v = qkv_d.split((heads * 128, kv * 128, kv * 128), dim=1)
+    kp2, vp2 = kp_d.clone(), vp_d.clone()
+    out = data_plane.paged_decode_attention_fused(q, k, v, qw_d, kw_d, cos_d, sin_d, 1e-6, slots_d, kp_d, vp_d, tables_d,
+                                                  ctx_d, SCALE)
+    q_rot, _, _ = data_plane.qk_norm_rope(q, k, v, qw_d, kw_d, cos_d, sin_d, 1e-6, slot_mapping=slots_d, key_pool=kp2,
+                                          value_pool=vp2)
+    want = data_plane.paged_decode_attention(q_rot.view(len(ctx), heads, 128), kp2, vp2, tables_d, ctx_d, SCALE)
+    assert torch.equal(kp_d.view(torch.int16), kp2.view(torch.int16))
+    assert torch.equal(vp_d.view(torch.int16), vp2.view(torch.int16))
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    ref = torch_ref.paged_decode_attention(q_rot.view(len(ctx), heads, 128).cpu(), kp2.cpu(), vp2.cpu(), tables,
+                                           torch.tensor(ctx), SCALE)
+    live = torch.tensor(ctx) > 0
+    assert (out.float().cpu()[live] - ref.float().view(len(ctx), -1)[live]).abs().max().item() <= TOL
+    assert not out.cpu()[~live].any()
+
+
+def test_fused_takes_rows_of_any_alignment(native_lib, device):
+    """Projection rows that start on a 2-byte boundary: the append and rotation run on their own."""
+    ctx = [300, 17]
+    kp, vp, tables, qkv, (qw, kw), cos, sin = _case(3, ctx, 72, 2)
+    slots = torch.tensor([int(tables[b, (n - 1) // 16]) * 16 + (n - 1) % 16 for b, n in enumerate(ctx)]).to(device)
+    kp, vp, tables, qkv, qw, kw, cos, sin = [t.to(device) for t in (kp, vp, tables, qkv, qw, kw, cos, sin)]
+    odd = torch.zeros(2, qkv.shape[1] + 1, dtype=torch.bfloat16, device=device)
+    odd[:, 1:] = qkv
+    outs = []
+    for rows in (qkv, odd[:, 1:]):
+        q, k, v = rows.split((2048, 1024, 1024), dim=1)
+        pools = kp.clone(), vp.clone()
+        outs.append((data_plane.paged_decode_attention_fused(q, k, v, qw, kw, cos, sin, 1e-6, slots, *pools, tables,
+                                                             torch.tensor(ctx).to(device), SCALE), *pools))
+    for a, b in zip(*outs):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
