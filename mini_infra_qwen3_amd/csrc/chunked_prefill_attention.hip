@@ -38,41 +38,46 @@
 //    move logits by ~1e-2, so dropping them would leave the 2e-2 parity band.
 //  * The two waves of a SIMD run in step (one workgroup barrier per tile), so per tile the
 //    matrix work, the score roundings, exponentials and converts, and the LDS operand latency
-//    largely add up.
+//    largely add up: of 655 us at 4 x 2048 queries behind 10240 tokens, a timing copy without the softmax
+//    took 299, one without the products 385, one with neither (the loads alone) 216.  Orders in which one
+//    wave of a SIMD multiplies while the other does its softmax were no gain (779 us with one barrier per
+//    tile, 806 with one per phase): a wave alone issues a VALU instruction in about 5 cycles, two
+//    together in 3.
 #include <algorithm>
 #include <initializer_list>
+#include <mutex>
 
-#include "mi_common.h"
+#include "decode_block.h"
 
 namespace mi {
 namespace {
 
-constexpr int kHeadDim = 128;
-constexpr int kBlockSize = 16;
 constexpr int kGroup = 2;  // query heads per workgroup (a pair of one GQA group)
-#ifndef MI_PREFILL_WAVES_PER_HEAD
-#define MI_PREFILL_WAVES_PER_HEAD 4
-#endif
-constexpr int kWavesPerHead = MI_PREFILL_WAVES_PER_HEAD;
-#ifndef MI_PREFILL_NT
-#define MI_PREFILL_NT 2
-#endif
-constexpr int kNt = MI_PREFILL_NT;                        // 16-query MFMA column tiles per wave
-constexpr int kQPerWave = 16 * kNt;
-constexpr int kQTile = kQPerWave * kWavesPerHead;         // queries per head per workgroup
-constexpr int kWavesPerSimd = kNt == 1 ? 4 : 2;           // occupancy the register budget is set for
 constexpr int kKTile = 64;                 // keys per KV tile
-constexpr int kThreads = 64 * kGroup * kWavesPerHead;    // one workgroup per CU at 4 waves per head
-constexpr int kSpans = kKTile / 4;                       // 1 KiB LDS spans (4 rows of 256 B) per K or V tile
-static_assert(kSpans % (kThreads / 64) == 0, "every wave moves the same number of spans");
-constexpr int kMaxHistoryBlocks = 16384;   // history table staged in LDS: 64 KiB at most (256k tokens)
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kRescaleSlack = 8.0f;
+constexpr int kSpans = kKTile / 4;         // 1 KiB LDS spans (4 rows of 256 B) per K or V tile
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
+// Shape of a workgroup.  kNt: 16-query MFMA column tiles per wave; kWavesPerHead: waves side by side on
+// the queries of a head; kKeySplit: wave groups that take every kKeySplit-th KV tile of the same queries
+// and merge their states at the end.
+template <int kNtV, int kWavesPerHeadV, int kKeySplitV>
+struct Shape {
+  static constexpr int kNt = kNtV, kWavesPerHead = kWavesPerHeadV, kKeySplit = kKeySplitV;
+  static constexpr int kQPerWave = 16 * kNt;
+  static constexpr int kQTile = kQPerWave * kWavesPerHead;       // queries per head per workgroup
+  static constexpr int kGroupWaves = kGroup * kWavesPerHead;     // waves that share a KV tile
+  static constexpr int kThreads = 64 * kGroupWaves * kKeySplit;
+  static constexpr int kTileBytes = kKTile * 256;                // one K or V tile
+  static constexpr int kLdsBytes = 4 * kTileBytes * kKeySplit;   // K and V, double-buffered, per wave group
+  static constexpr int kSpansPerWave = kSpans / kGroupWaves;
+  static_assert(kSpans % kGroupWaves == 0, "every wave moves the same number of spans");
+  static_assert(kBlockSize % (4 * kSpansPerWave) == 0, "a wave's spans of a tile must lie in one pool block");
+};
+using Wide = Shape<2, 4, 1>;       // 128 queries, 8 waves
+using Half = Shape<2, 2, 1>;       // 64 queries, 4 waves: two workgroups a CU, not in step
+using HalfSplit = Shape<2, 2, 2>;  // 64 queries, 8 waves, the keys in two halves
+using Narrow = Shape<1, 2, 2>;     // 32 queries, 8 waves, the keys in two halves
+constexpr int kLdsPerGroup = 160 * 1024;
+constexpr int kMaxHistoryBlocks = 16384;   // history table staged in LDS: 64 KiB at most (256k tokens)
 
 struct PrefillArgs {
   uint16_t* out;
@@ -107,6 +112,9 @@ struct PrefillArgs {
   int32_t decode_rows;
   const int64_t* slot_mapping;
   int64_t slot_stride;
+  // Decode rows only: one workgroup per (row, KV head) attends them block by block (decode_row) instead
+  // of as one-query tiles.
+  int32_t stripes;
   // Ragged chunk rows (a mixed step's chunks packed back to back): when set, the len_b real tokens
   // of row b are flat tokens row_first[b] .. row_first[b] + len_b - 1 of query / key / value / out
   // (the token strides apply, the row strides are unused; row_first[b] is clamped to
@@ -121,28 +129,158 @@ __device__ __forceinline__ void reference_scores(f32x4& v, float scale) {
   for (int i = 0; i < 4; ++i) v[i] = round_bf16(round_bf16(v[i]) * scale);
 }
 
-// One 16-byte-per-lane load straight into LDS: lane i writes bytes [16 i, 16 i + 16) of the
-// 1 KiB span at LDS address lds (wave-uniform, passed in M0; one wait state between the M0 write
+// One 16-byte-per-lane load straight into LDS, from a uniform base and a byte offset per lane: lane i
+// writes bytes [16 i, 16 i + 16) of the 1 KiB span at LDS address lds (wave-uniform, passed in M0; one wait state between the M0 write
 // and the load).  Issued by inline assembly: the compiler's own form ties every later LDS read to
 // the completion of all such loads (it cannot tell the two tile buffers apart), which would wait
 // for tile t + 1 before reading tile t.  The compiler does not see these loads, so the kernel waits
 // for them itself (vmcnt(0) before each tile barrier).  The LDS address goes in through an M0
 // operand constraint, so the compiler writes M0 itself and knows its value across the asm.
-__device__ __forceinline__ void dma16(const void* gptr, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "{m0}"(lds) : "memory");
+__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
+}
+
+// A decode row of a mixed step (its single new token) by one workgroup of kStripes wavefronts per KV head,
+// with the arithmetic of the decode kernels: stripe v attends blocks v, v + kStripes, ... of the history
+// and the token, whose K and V rows (not yet in the pool, and appended here) are put in place of what its
+// position's slot held.  As a one-query tile a row took 2 us per 64 keys, and the longest decode context
+// was the longest chain of the launch.
+constexpr int kRowDepth = 3;                             // blocks of a stripe in registers
+constexpr int kRowStageElems = kBlockSize * kKStageRow;  // a wavefront's K staging; its output rows overlay it
+constexpr int kRowMaxBlocks = 64 * kStripes - 1;         // a lane holds one block id; one more for the token
+constexpr int kRowMaxGroup = 8;
+template <int kKvHeads>
+__device__ __forceinline__ void decode_row(const PrefillArgs& a, const int unit, unsigned char* smem) {
+  constexpr int kRowElems = kKvHeads * kHeadDim;
+  constexpr int kBlockElems = kBlockSize * kRowElems;
+  static_assert(kRowMaxGroup * kHeadDim * sizeof(float) <= kRowStageElems * sizeof(uint16_t), "rows fit the staging");
+  uint16_t* s_kst = reinterpret_cast<uint16_t*>(smem);                                                  // [kStripes]
+  float* s_ml = reinterpret_cast<float*>(smem + kStripes * kRowStageElems * sizeof(uint16_t));          // [kStripes][8][2]
+  const int b = unit / kKvHeads;
+  const int g = (unit + b) % kKvHeads;  // every XCD gets every head in turn
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int dl = lane & 15, r = lane >> 4;
+  int64_t id = a.history_blocks[b * a.history_stride + min(w + kStripes * lane, a.max_history_blocks - 1)];
+  const int64_t ctx = a.start_lens[b * a.lens_stride];
+  const u32x4 k_new = *reinterpret_cast<const u32x4*>(a.key + b * a.k_row + g * a.k_head + 8 * dl);
+  const u32x4 v_new = *reinterpret_cast<const u32x4*>(a.value + b * a.v_row + g * a.v_head + 8 * dl);
+  bf16x8 qf[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+    qf[ks] = dl < a.group ? *reinterpret_cast<const bf16x8*>(a.query + b * a.q_row + (g * a.group + dl) * a.q_head +
+                                                             32 * ks + 8 * r)
+                          : bf16x8{};
+  uint16_t* out_b = a.out + b * a.out_row + g * a.group * kHeadDim;
+  if (ctx <= 0) {  // a padding row (uniform)
+    if (threadIdx.x < a.group * 16) *reinterpret_cast<uint4*>(out_b + 8 * threadIdx.x) = uint4{0, 0, 0, 0};
+    return;
+  }
+  const int nh = static_cast<int>(min(ctx - 1, static_cast<int64_t>(a.max_history_blocks) * kBlockSize));
+  const int nblk = nh / kBlockSize + 1;  // the last one holds the token, at position nh
+  const int cnt = nblk > w ? (nblk - 1 - w) / kStripes + 1 : 0;
+  if (id < 0 || id >= a.num_blocks) id = 0;
+  const uint32_t id_lo = static_cast<uint32_t>(id);  // the pool has fewer than 2^31 blocks
+  if (threadIdx.x < 32) {  // append the token's K and V rows of KV head g
+    const int64_t slot = a.slot_mapping[b * a.slot_stride];
+    if (slot >= 0 && slot < a.num_blocks * kBlockSize) {
+      uint16_t* pool = threadIdx.x < 16 ? a.key_pool : a.value_pool;
+      *reinterpret_cast<u32x4*>(pool + (slot * kKvHeads + g) * kHeadDim + 8 * dl) = threadIdx.x < 16 ? k_new : v_new;
+    }
+  }
+  const uint32_t k_off = 2u * (r * kRowElems + g * kHeadDim + 8 * dl);
+  const uint32_t v_off = 2u * (4 * r * kRowElems + g * kHeadDim + 8 * dl);
+  u32x4 kbuf[kRowDepth][4], vbuf[kRowDepth][4];
+  auto issue = [&](int ring, int i) {
+    const int64_t base = static_cast<int64_t>(__builtin_amdgcn_readlane(id_lo, i)) * kBlockElems;
+    const char* kp = reinterpret_cast<const char*>(a.key_pool + base);
+    const char* vp = reinterpret_cast<const char*>(a.value_pool + base);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) kbuf[ring][t] = load_vec<true>(reinterpret_cast<const u32x4*>(kp + t * 8 * kRowElems + k_off));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) vbuf[ring][t] = load_vec<true>(reinterpret_cast<const u32x4*>(vp + t * 2 * kRowElems + v_off));
+  };
+#pragma unroll
+  for (int s = 0; s < kRowDepth - 1; ++s)
+    if (s < cnt) issue(s, s);  // wave-uniform
+  MfmaState ms;
+  ms.m = -INFINITY;
+  ms.l = 0.0f;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) ms.o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int i0 = 0; i0 < cnt; i0 += kRowDepth) {
+#pragma unroll
+    for (int s = 0; s < kRowDepth; ++s) {
+      const int i = i0 + s;
+      if (i >= cnt) break;  // wave-uniform
+      if (i + kRowDepth - 1 < cnt) issue((s + kRowDepth - 1) % kRowDepth, i + kRowDepth - 1);
+      if (w + kStripes * i == nblk - 1) {
+        const int t = nh % kBlockSize;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          kbuf[s][e] = 4 * e + r == t ? k_new : kbuf[s][e];
+          vbuf[s][e] = 4 * r + e == t ? v_new : vbuf[s][e];
+        }
+      }
+      attend_block_mfma(ms, qf, kbuf[s], vbuf[s], s_kst + w * kRowStageElems, a.scale, (w + kStripes * i) * kBlockSize,
+                        nh + 1, lane);
+    }
+  }
+  // Lane: heads 4 r + i, dims 8 dl .. +8; head j's max and sum live in lane j.
+  const float lsum = xsum32_f32(xsum16_f32(ms.l));
+  float* rows = reinterpret_cast<float*>(s_kst + w * kRowStageElems);  // [group][128]
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int j = 4 * r + i;
+    const float Lj = __shfl(lsum, j);
+    const float Mj = __shfl(ms.m, j);
+    if (j >= a.group) continue;
+    float4* dst = reinterpret_cast<float4*>(rows + j * kHeadDim + 8 * dl);
+    dst[0] = make_float4(ms.o[0][i], ms.o[1][i], ms.o[2][i], ms.o[3][i]);
+    dst[1] = make_float4(ms.o[4][i], ms.o[5][i], ms.o[6][i], ms.o[7][i]);
+    if (dl == 0) *reinterpret_cast<float2*>(s_ml + (w * kRowMaxGroup + j) * 2) = make_float2(Mj, Lj);
+  }
+  __syncthreads();
+  if (threadIdx.x < a.group * 16) {
+    const int h = threadIdx.x >> 4, dm = threadIdx.x & 15;
+    StripeMerge sm;
+#pragma unroll
+    for (int v = 0; v < kStripes; ++v) {
+      const float4* src = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(s_kst + v * kRowStageElems) +
+                                                          h * kHeadDim + 8 * dm);
+      sm.m[v] = s_ml[(v * kRowMaxGroup + h) * 2];
+      sm.l[v] = s_ml[(v * kRowMaxGroup + h) * 2 + 1];
+      sm.x[v] = src[0];
+      sm.y[v] = src[1];
+    }
+    sm.store(out_b + h * kHeadDim + 8 * dm);
+  }
 }
 
 // One launch serves up to two sets of rows (a mixed step's chunk rows and its decode rows): the
-// first a0.groups workgroups take a0, the rest a1.
-template <int kKvHeads>
-__global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kernel(const PrefillArgs a0,
-                                                                                   const PrefillArgs a1) {
-  // K and V tiles row-major, 256-byte rows, 16-byte chunk c of row r stored at chunk c ^ (r % 16).
-  __shared__ __align__(1024) uint16_t sK[2][kKTile * kHeadDim];
-  __shared__ __align__(1024) uint16_t sV[2][kKTile * kHeadDim];
-  extern __shared__ int s_hblk[];  // [ceil(nh / 16)] history block ids of this row (dynamic LDS)
+// first a0.groups workgroups take a0, the next a1.groups a1; the last z.groups write zero rows.
+template <int kKvHeads, typename S>
+__global__ __launch_bounds__(S::kThreads, 2) void chunked_prefill_kernel(const PrefillArgs a0, const PrefillArgs a1,
+                                                                   const ZeroRows z) {
+  constexpr int kNt = S::kNt, kQPerWave = S::kQPerWave, kQTile = S::kQTile, kThreads = S::kThreads;
+  constexpr int kKeySplit = S::kKeySplit, kSpansPerWave = S::kSpansPerWave;
+  constexpr uint32_t kTileBytes = S::kTileBytes;
+  // Dynamic LDS.  Per wave group two K tiles, then two V tiles: row-major, 256-byte rows, 16-byte chunk
+  // c of row r stored at chunk c ^ (r % 16).  Then the history block ids of this row, [ceil(nh / 16)].
+  extern __shared__ __align__(1024) unsigned char s_raw[];
+  int* s_hblk = reinterpret_cast<int*>(s_raw + S::kLdsBytes);
 
+  if (static_cast<int>(blockIdx.x) >= a0.groups + a1.groups) {  // uniform
+    zero_uncovered_rows(z, static_cast<int>(blockIdx.x) - a0.groups - a1.groups, kThreads);
+    return;
+  }
   const bool second = static_cast<int>(blockIdx.x) >= a0.groups;  // uniform
+  if constexpr (kThreads == 64 * kStripes) {
+    if (second && a1.stripes) {  // uniform
+      decode_row<kKvHeads>(a1, static_cast<int>(blockIdx.x) - a0.groups, s_raw);
+      return;
+    }
+  }
   const PrefillArgs a = second ? a1 : a0;
 
   // Workgroup -> (row b, head pair hp, query tile qt).  Consecutive workgroup ids go round-robin to
@@ -207,8 +345,10 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform: keeps edge-tile branches real
-  const int hh = w / kWavesPerHead;
-  const int qs = w % kWavesPerHead;
+  const int wk = w / S::kGroupWaves;      // wave group (key split)
+  const int wt = w % S::kGroupWaves;      // wave of the group
+  const int hh = wt / S::kWavesPerHead;
+  const int qs = wt % S::kWavesPerHead;
   const int g = hp / a.pairs;                    // KV head
   const int j0 = (hp - g * a.pairs) * kGroup;    // first head of the pair within the group
   const bool head_live = j0 + hh < a.group;      // wave-uniform: false for the spare half of an odd group
@@ -264,7 +404,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
 
   // ---- tile loads straight into LDS (global_load_lds_dwordx4: lane i of an instruction writes
   // bytes [16 i, 16 i + 16) of a 1 KiB LDS span).  A tile is kSpans such spans of 4 rows for K and
-  // as many for V; wave w moves spans [kSpansPerWave w, kSpansPerWave (w + 1)) of each.  Lane i of
+  // as many for V; wave wt of a group moves spans [kSpansPerWave wt, kSpansPerWave (wt + 1)) of each.  Lane i of
   // span m fetches row 4 m + i / 16, global chunk (i % 16) ^ (row % 16), so that the chunk lands at
   // its swizzled place: the 16 lanes of an MFMA operand read (16 rows, one logical chunk) then hit
   // 16 different chunk positions, i.e. all banks.  In a history tile a wave's spans lie in one pool
@@ -277,7 +417,6 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
     s_hblk[i] = (x < 0 || x >= a.num_blocks) ? 0 : static_cast<int>(x);
   }
   constexpr int64_t kBlkElems = static_cast<int64_t>(kBlockSize) * kKvHeads * kHeadDim;
-  constexpr int kSpansPerWave = kSpans / (kThreads / 64);
   const int drow = lane >> 4;
   const int dchunk = lane & 15;
   const uint16_t* k_rows = a.key + k_base + g * a.k_head;  // padded position rpad
@@ -285,37 +424,60 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
   const uint32_t k_tok = static_cast<uint32_t>(a.k_tok);  // < 2^24, checked by the entry point
   const uint32_t v_tok = static_cast<uint32_t>(a.v_tok);
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
-  static_assert(kBlockSize % (4 * kSpansPerWave) == 0, "a wave's spans of a tile must lie in one pool block");
-  const int wave_blk = 4 * kSpansPerWave * w / kBlockSize;  // pool block of this wave's rows within a tile
+  const int wave_blk = 4 * kSpansPerWave * wt / kBlockSize;  // pool block of this wave's rows within a tile
   const auto hist_slot = [&](const int t) { return min(t * (kKTile / kBlockSize) + wave_blk, max(nhb - 1, 0)); };
   // LDS byte addresses of this wave's first K and V span in buffer 0 (buffer 1 follows at + kTileBytes).
-  constexpr uint32_t kTileBytes = kKTile * kHeadDim * sizeof(uint16_t);
-  const uint32_t k_lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)(&sK[0][kSpansPerWave * w * 512])));
-  const uint32_t v_lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)(&sV[0][kSpansPerWave * w * 512])));
+  unsigned char* tiles = s_raw + wk * 4 * kTileBytes;  // this wave group's
+  const uint32_t k_lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)(tiles + kSpansPerWave * wt * 1024)));
+  const uint32_t v_lds0 = k_lds0 + 2 * kTileBytes;
 
+  // Byte offsets of the lane's pieces: from the pool block in a history tile, from the tile's first row in
+  // a chunk tile that lies inside the row (63 rows at most: below 2^31, token strides being below 2^24).
+  uint32_t hist_off[kSpansPerWave], k_off_in[kSpansPerWave], v_off_in[kSpansPerWave];
+#pragma unroll
+  for (int i = 0; i < kSpansPerWave; ++i) {
+    const int r = 4 * (kSpansPerWave * wt + i) + drow;
+    const uint32_t c16 = static_cast<uint32_t>((dchunk ^ (r & 15)) * 16);
+    hist_off[i] = static_cast<uint32_t>(((r & 15) * kKvHeads + g) * kHeadDim) * 2 + c16;
+    k_off_in[i] = 2 * r * k_tok + c16;
+    v_off_in[i] = 2 * r * v_tok + c16;
+  }
   // hblk: this wave's history block id for tile t (unused for chunk tiles).
   auto dma_tile = [&](const int t, const int buf, const int hblk) {
-    const bool hist = t < n_hist_tiles;
-    const int key0 = (c_lo + t - n_hist_tiles) * kKTile;
+    const char *kbase, *vbase;
+    uint32_t ko[kSpansPerWave], vo[kSpansPerWave];
+    if (t < n_hist_tiles) {
+      const int64_t at = __builtin_amdgcn_readfirstlane(hblk) * kBlkElems;
+      kbase = reinterpret_cast<const char*>(a.key_pool + at);
+      vbase = reinterpret_cast<const char*>(a.value_pool + at);
+#pragma unroll
+      for (int i = 0; i < kSpansPerWave; ++i) ko[i] = vo[i] = hist_off[i];
+    } else {
+      const int key0 = (c_lo + t - n_hist_tiles) * kKTile;
+      const int row0 = min(max(key0, rpad), L - 1);  // the clamp of the tile's first row: below every row's
+      kbase = reinterpret_cast<const char*>(k_rows + static_cast<int64_t>(row0 - rpad) * k_tok);
+      vbase = reinterpret_cast<const char*>(v_rows + static_cast<int64_t>(row0 - rpad) * v_tok);
+      if (key0 >= rpad && key0 + kKTile <= L) {
+#pragma unroll
+        for (int i = 0; i < kSpansPerWave; ++i) {
+          ko[i] = k_off_in[i];
+          vo[i] = v_off_in[i];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < kSpansPerWave; ++i) {
+          const int r = 4 * (kSpansPerWave * wt + i) + drow;
+          const uint32_t c16 = static_cast<uint32_t>((dchunk ^ (r & 15)) * 16);
+          const uint32_t kc = static_cast<uint32_t>(min(max(key0 + r, rpad), L - 1) - row0);
+          ko[i] = 2 * kc * k_tok + c16;
+          vo[i] = 2 * kc * v_tok + c16;
+        }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < kSpansPerWave; ++i) {
-      const int m = kSpansPerWave * w + i;
-      const int r = 4 * m + drow;
-      const uint32_t c8 = static_cast<uint32_t>((dchunk ^ (r & 15)) * 8);
-      const uint16_t* ksrc;
-      const uint16_t* vsrc;
-      if (hist) {
-        const int64_t blk = __builtin_amdgcn_readfirstlane(hblk);
-        const uint32_t off = static_cast<uint32_t>(((r & 15) * kKvHeads + g) * kHeadDim) + c8;
-        ksrc = a.key_pool + blk * kBlkElems + off;
-        vsrc = a.value_pool + blk * kBlkElems + off;
-      } else {
-        const uint32_t kc = static_cast<uint32_t>(min(max(key0 + r, rpad), L - 1) - rpad);
-        ksrc = k_rows + (__umul24(kc, k_tok) + c8);
-        vsrc = v_rows + (__umul24(kc, v_tok) + c8);
-      }
-      dma16(ksrc, __builtin_amdgcn_readfirstlane(k_lds0 + buf * kTileBytes + i * 1024));
-      dma16(vsrc, __builtin_amdgcn_readfirstlane(v_lds0 + buf * kTileBytes + i * 1024));
+      dma16(kbase, ko[i], __builtin_amdgcn_readfirstlane(k_lds0 + buf * kTileBytes + i * 1024));
+      dma16(vbase, vo[i], __builtin_amdgcn_readfirstlane(v_lds0 + buf * kTileBytes + i * 1024));
     }
   };
   // Per-lane LDS byte offsets of the MFMA operands.  K (A of S^T = K Q^T): row 16 mt + ql, global
@@ -347,24 +509,12 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
   for (int nt = 0; nt < kNt; ++nt) m_run[nt] = -INFINITY;
   const float scale = a.scale;
 
-  // Tile t + 1 moves into the other buffer while tile t is computed; each wave waits for its own
-  // loads before the tile barrier, after which every wave's part is in place.
-  __syncthreads();  // s_hblk ready
-  dma_tile(0, 0, s_hblk[hist_slot(0)]);
-  int hblk_next = s_hblk[hist_slot(1)];
-  // s_waitcnt vmcnt(0) (expcnt and lgkmcnt unconstrained) as a real instruction, so that the
-  // compiler also counts the Q fragment loads as complete and waits for nothing inside the loop.
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  __syncthreads();
-
-  auto tile_step = [&](const int t, const int buf) {
-    if (t + 1 < n_tiles) dma_tile(t + 1, buf ^ 1, hblk_next);
-    hblk_next = s_hblk[hist_slot(t + 2)];
-    const char* sKb = reinterpret_cast<const char*>(sK[buf]);
-    const char* sVb = reinterpret_cast<const char*>(sV[buf]);
-
+  // The three parts of a tile's work.  sacc: scores of 64 keys x kQPerWave queries; pf: [nt][ks2]
+  // probabilities as B operands.
+  f32x4 sacc[4][kNt];
+  bf16x8 pf[kNt][2];
+  auto tile_scores = [&](const char* sKb) {
     // ---- S^T = K Q^T for 64 keys x 32 queries
-    f32x4 sacc[4][kNt];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -379,7 +529,8 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
           sacc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[nt][ks], sacc[mt][nt], 0, 0, 0);
       }
     }
-
+  };
+  auto tile_softmax = [&](const int t) {
     // ---- scores, masks (uniform branch: only edge tiles need them)
     const bool is_hist = t < n_hist_tiles;
     const int key0 = is_hist ? t * kKTile : (c_lo + t - n_hist_tiles) * kKTile;
@@ -443,7 +594,6 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
         for (int dt = 0; dt < 9; ++dt) oacc[dt][nt] *= alpha;
       }
     }
-    bf16x8 pf[kNt][2];  // [nt][ks2]
 #pragma unroll
     for (int nt = 0; nt < kNt; ++nt) {
       const float ref = m_run[nt] == -INFINITY ? 0.0f : m_run[nt];
@@ -459,7 +609,8 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
         pf[nt][ks2] = __builtin_convertvector(pv, bf16x8);
       }
     }
-
+  };
+  auto tile_values = [&](const char* sVb) {
     // ---- O^T += V^T P^T
 #pragma unroll
     for (int ks2 = 0; ks2 < 2; ++ks2) {
@@ -478,13 +629,73 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void chunked_prefill_kerne
       for (int nt = 0; nt < kNt; ++nt)
         oacc[8][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_frag, pf[nt][ks2], oacc[8][nt], 0, 0, 0);
     }
+  };
+  const char* k_tiles = reinterpret_cast<const char*>(tiles);
+  const char* v_tiles = k_tiles + 2 * kTileBytes;
 
+  __syncthreads();  // s_hblk ready
+  // Tile t + 1 moves into the other buffer while tile t is computed; each wave waits for its own
+  // loads before the tile barrier, after which every wave's part is in place.
+  if (wk < n_tiles) dma_tile(wk, 0, s_hblk[hist_slot(wk)]);  // wave group wk takes tiles wk, wk + kKeySplit, ...
+  int hblk_next = s_hblk[hist_slot(wk + kKeySplit)];
+  // s_waitcnt vmcnt(0) (expcnt and lgkmcnt unconstrained) as a real instruction, so that the
+  // compiler also counts the Q fragment loads as complete and waits for nothing inside the loop.
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __syncthreads();
+  auto tile_step = [&](const int t, const int buf) {
+    if (t + kKeySplit < n_tiles) dma_tile(t + kKeySplit, buf ^ 1, hblk_next);
+    hblk_next = s_hblk[hist_slot(t + 2 * kKeySplit)];
+    tile_scores(k_tiles + buf * kTileBytes);
+    tile_softmax(t);
+    tile_values(v_tiles + buf * kTileBytes);
+  };
+  // Every wave of the workgroup passes every barrier: the rounds are uniform, and a wave group without
+  // a tile in the last round only waits.
+  auto round_end = [&] {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   };
-  for (int t = 0; t < n_tiles; t += 2) {
-    tile_step(t, 0);
-    if (t + 1 < n_tiles) tile_step(t + 1, 1);
+  for (int t0 = 0; t0 < n_tiles; t0 += 2 * kKeySplit) {
+    if (kKeySplit == 1 || t0 + wk < n_tiles) tile_step(t0 + wk, 0);
+    round_end();
+    if (t0 + kKeySplit < n_tiles) {
+      if (kKeySplit == 1 || t0 + kKeySplit + wk < n_tiles) tile_step(t0 + kKeySplit + wk, 1);
+      round_end();
+    }
+  }
+  if constexpr (kKeySplit > 1) {
+    // Join the wave groups' states: group 0's waves fold in the others' (log-sum-exp), which they leave
+    // in LDS over the tiles (no longer read: the last round's barrier is behind every wave).
+    constexpr int kStateFloats = 33 * kNt * 64;  // per wave: 8 x 4 accumulators and the row sum per column tile
+    static_assert((kKeySplit - 1) * S::kGroupWaves * (kStateFloats + 64 * kNt) * 4 <= S::kLdsBytes, "the states fit the tiles");
+    float* st = reinterpret_cast<float*>(s_raw) + ((wk > 0 ? wk - 1 : 0) * S::kGroupWaves + wt) * (kStateFloats + 64 * kNt) + lane;
+    if (wk > 0) {
+#pragma unroll
+      for (int nt = 0; nt < kNt; ++nt) {
+#pragma unroll
+        for (int e = 0; e < 32; ++e) st[(33 * nt + e) * 64] = oacc[e >> 2][nt][e & 3];
+        st[(33 * nt + 32) * 64] = oacc[8][nt][0];
+        st[(33 * kNt + nt) * 64] = m_run[nt];
+      }
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int k = 1; k < kKeySplit; ++k) {
+      const float* other = st + (k - 1) * S::kGroupWaves * (kStateFloats + 64 * kNt);
+#pragma unroll
+      for (int nt = 0; nt < kNt; ++nt) {
+        const float mo = other[(33 * kNt + nt) * 64];
+        const float mn = fmaxf(m_run[nt], mo);
+        const float e0 = m_run[nt] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run[nt] - mn);
+        const float e1 = mo == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mo - mn);
+        m_run[nt] = mn;
+#pragma unroll
+        for (int e = 0; e < 32; ++e)
+          oacc[e >> 2][nt][e & 3] = e0 * oacc[e >> 2][nt][e & 3] + e1 * other[(33 * nt + e) * 64];
+        oacc[8][nt][0] = e0 * oacc[8][nt][0] + e1 * other[(33 * nt + 32) * 64];
+      }
+    }
   }
 
   // ---- normalise and write: lane holds query qw0 + 16 nt + ql, dims 16 dt + 4 gq + i
@@ -531,14 +742,15 @@ int32_t check_common(const char* name, int32_t num_heads, int32_t num_kv_heads, 
 }
 
 // Fills the row-independent fields; the caller sets the pointers and strides of its rows.
-PrefillArgs rows_args(int32_t batch, int32_t padded_len, int32_t num_heads, int32_t num_kv_heads, float scale) {
+PrefillArgs rows_args(int32_t batch, int32_t padded_len, int32_t num_heads, int32_t num_kv_heads, float scale,
+                      int q_tile) {
   PrefillArgs a{};
   a.batch = batch;
   a.padded_len = padded_len;
   a.group = num_heads / num_kv_heads;
   a.pairs = (a.group + kGroup - 1) / kGroup;
   a.scale = scale;
-  a.tiles = (padded_len + kQTile - 1) / kQTile;
+  a.tiles = (padded_len + q_tile - 1) / q_tile;
   const int64_t pairs = static_cast<int64_t>(num_kv_heads) * a.pairs * batch;
   const int64_t groups = a.tiles * pairs;
   a.groups = groups > 0x3fffffff ? -1 : static_cast<int32_t>(groups);
@@ -552,63 +764,89 @@ PrefillArgs rows_args(int32_t batch, int32_t padded_len, int32_t num_heads, int3
   return a;
 }
 
-int32_t launch_rows(const char* name, const PrefillArgs& a0, const PrefillArgs& a1, int32_t num_kv_heads,
-                    int32_t max_history_blocks, void* stream) {
-  if (a0.groups < 0 || a1.groups < 0 || static_cast<int64_t>(a0.groups) + a1.groups > 0x3fffffff)
-    return fail(MI_ERR_UNSUPPORTED, "%s: too many workgroups", name);
-  if (max_history_blocks > kMaxHistoryBlocks)
-    return fail(MI_ERR_UNSUPPORTED, "%s: history of %d blocks exceeds %d", name, max_history_blocks, kMaxHistoryBlocks);
-  const int groups = a0.groups + a1.groups;
-  if (groups == 0) return ok();
-  const size_t lds = sizeof(int) * static_cast<size_t>(max_history_blocks > 0 ? max_history_blocks : 1);
-  hipStream_t s = as_stream(stream);
-  switch (num_kv_heads) {
-    case 1: chunked_prefill_kernel<1><<<groups, kThreads, lds, s>>>(a0, a1); break;
-    case 2: chunked_prefill_kernel<2><<<groups, kThreads, lds, s>>>(a0, a1); break;
-    case 4: chunked_prefill_kernel<4><<<groups, kThreads, lds, s>>>(a0, a1); break;
-    default: chunked_prefill_kernel<8><<<groups, kThreads, lds, s>>>(a0, a1); break;
-  }
+enum class Form { kWide, kHalf, kHalfSplit, kNarrow };
+
+#ifndef MI_PREFILL_FORM
+#define MI_PREFILL_FORM -1
+#endif
+#ifndef MI_PREFILL_T1
+#define MI_PREFILL_T1 128
+#define MI_PREFILL_T2 248
+#define MI_PREFILL_T3 512
+#endif
+// Which workgroup shape takes a launch of `batch` chunk rows: by the workgroups it would have in the wide
+// one (80 of them occupied 80 CUs for 11 serial key tiles of 2 us).  Measured, us, wide / half / half split /
+// narrow (16 query, 8 KV heads):
+//   1 x 60 behind 4000 tokens           8 workgroups   143 / 111 /  90 /  65
+//   1 x 1000                           64               44 /  35 /  29 /  22
+//   2 x 250-700                        80               27 /  23 /  21 /  16
+//   1 x 2048 behind 2000              128              114 /  86 /  72 /  82
+//   2 x 700-1400                      160               59 /  46 /  37 /  40
+//   3 x 1200                          240               51 /  50 /  48 /  53
+//   2 x 2048 behind 3000              256              144 / 154 / 153 / 214
+//   3 x 1024-2048, none / 5000        360          72 / 327 | 63 / 282 | 72 / 290 | 82 / 346
+//   4 x 2048 behind 10240             512              658 / 679 / 762 / 1135
+Form form_for(int32_t batch, int32_t padded_len, int32_t num_heads, int32_t num_kv_heads, int32_t max_history_blocks) {
+  if (MI_PREFILL_FORM >= 0) return static_cast<Form>(MI_PREFILL_FORM);
+  const int64_t pairs = static_cast<int64_t>(num_kv_heads) * ((num_heads / num_kv_heads + kGroup - 1) / kGroup) * batch;
+  const int64_t wide = pairs * ((padded_len + Wide::kQTile - 1) / Wide::kQTile);
+  if (wide >= MI_PREFILL_T3 || (wide >= MI_PREFILL_T2 && wide <= 256)) return Form::kWide;
+  static_assert(Narrow::kLdsBytes == HalfSplit::kLdsBytes, "one limit");
+  const bool split_fits = Narrow::kLdsBytes + sizeof(int) * static_cast<size_t>(max_history_blocks) <= kLdsPerGroup;
+  if (wide >= MI_PREFILL_T2 || !split_fits) return Form::kHalf;
+  return wide >= MI_PREFILL_T1 ? Form::kHalfSplit : Form::kNarrow;
+}
+
+int q_tile_of(Form f) {
+  return f == Form::kWide ? Wide::kQTile : f == Form::kNarrow ? Narrow::kQTile : Half::kQTile;
+}
+
+template <int kKvHeads, typename S>
+int32_t launch_shape(const char* name, const PrefillArgs& a0, const PrefillArgs& a1, const ZeroRows& z, int groups,
+                     int32_t max_history_blocks, hipStream_t s) {
+  // Dynamic LDS above 64 KiB must be allowed per kernel (gfx950 has 160 KiB per workgroup).
+  static std::once_flag once;
+  static hipError_t err = hipSuccess;
+  std::call_once(once, [] {
+    err = hipFuncSetAttribute(reinterpret_cast<const void*>(chunked_prefill_kernel<kKvHeads, S>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerGroup);
+  });
+  if (err != hipSuccess) return fail(MI_ERR_DEVICE, "%s: hipFuncSetAttribute: %s", name, hipGetErrorString(err));
+  const size_t lds = S::kLdsBytes + sizeof(int) * static_cast<size_t>(max_history_blocks > 0 ? max_history_blocks : 1);
+  chunked_prefill_kernel<kKvHeads, S><<<groups, S::kThreads, lds, s>>>(a0, a1, z);
   return check_launch(name);
 }
 
-// One workgroup per token t of [0, row_tokens): every thread checks its share of the rows, and the
-// workgroup writes a zero row unless one of them covers t.
-constexpr int kZeroThreads = 256;
-__global__ __launch_bounds__(kZeroThreads) void zero_uncovered_kernel(uint16_t* out, int64_t out_tok, int32_t row_elems,
-                                                                       const int64_t* first, const int64_t* lens,
-                                                                       int64_t lens_stride, int32_t rows, int32_t width,
-                                                                       int64_t row_tokens, int32_t vec) {
-  const int64_t t = blockIdx.x;
-  int covered = 0;
-  for (int b = threadIdx.x; b < rows; b += kZeroThreads) {
-    int64_t len = lens[b * lens_stride];
-    len = len < 0 ? 0 : (len > width ? width : len);
-    int64_t f = first[b];
-    f = f < 0 ? 0 : (f > row_tokens - len ? row_tokens - len : f);
-    covered |= t >= f && t < f + len;
+template <typename S>
+int32_t launch_rows(const char* name, const PrefillArgs& a0, const PrefillArgs& a1, ZeroRows z, int32_t num_kv_heads,
+                    int32_t max_history_blocks, void* stream) {
+  z.groups = static_cast<int32_t>((z.tokens + S::kThreads - 1) / S::kThreads);
+  if (a0.groups < 0 || a1.groups < 0 || static_cast<int64_t>(a0.groups) + a1.groups + z.groups > 0x3fffffff)
+    return fail(MI_ERR_UNSUPPORTED, "%s: too many workgroups", name);
+  if (max_history_blocks > kMaxHistoryBlocks)
+    return fail(MI_ERR_UNSUPPORTED, "%s: history of %d blocks exceeds %d", name, max_history_blocks, kMaxHistoryBlocks);
+  const int groups = a0.groups + a1.groups + z.groups;
+  if (groups == 0) return ok();
+  hipStream_t s = as_stream(stream);
+  switch (num_kv_heads) {
+    case 1: return launch_shape<1, S>(name, a0, a1, z, groups, max_history_blocks, s);
+    case 2: return launch_shape<2, S>(name, a0, a1, z, groups, max_history_blocks, s);
+    case 4: return launch_shape<4, S>(name, a0, a1, z, groups, max_history_blocks, s);
+    default: return launch_shape<8, S>(name, a0, a1, z, groups, max_history_blocks, s);
   }
-  if (__syncthreads_or(covered)) return;
-  uint16_t* row = out + t * out_tok;
-  if (vec) {
-    for (int i = threadIdx.x; i < row_elems / 8; i += kZeroThreads) reinterpret_cast<uint4*>(row)[i] = uint4{0, 0, 0, 0};
-  } else {
-    for (int i = threadIdx.x; i < row_elems; i += kZeroThreads) row[i] = 0;
+}
+
+int32_t launch_form(Form form, const char* name, const PrefillArgs& a0, const PrefillArgs& a1, const ZeroRows& z,
+                    int32_t num_kv_heads, int32_t max_history_blocks, void* stream) {
+  switch (form) {
+    case Form::kWide: return launch_rows<Wide>(name, a0, a1, z, num_kv_heads, max_history_blocks, stream);
+    case Form::kHalf: return launch_rows<Half>(name, a0, a1, z, num_kv_heads, max_history_blocks, stream);
+    case Form::kHalfSplit: return launch_rows<HalfSplit>(name, a0, a1, z, num_kv_heads, max_history_blocks, stream);
+    default: return launch_rows<Narrow>(name, a0, a1, z, num_kv_heads, max_history_blocks, stream);
   }
 }
 
 }  // namespace
-
-int32_t zero_uncovered_tokens(const char* what, void* out, int64_t out_tok_stride, int32_t row_elems,
-                              const int64_t* first, const int64_t* lens, int64_t lens_stride, int32_t rows,
-                              int32_t width, int64_t row_tokens, void* stream) {
-  if (row_tokens <= 0) return MI_OK;
-  if (row_tokens > 0x7fffffff) return fail(MI_ERR_UNSUPPORTED, "%s: more than 2^31 - 1 chunk tokens", what);
-  const int32_t vec = aligned16(out) && out_tok_stride % 8 == 0 && row_elems % 8 == 0;
-  zero_uncovered_kernel<<<static_cast<unsigned>(row_tokens), kZeroThreads, 0, as_stream(stream)>>>(
-      static_cast<uint16_t*>(out), out_tok_stride, row_elems, first, lens, lens_stride, rows, width, row_tokens, vec);
-  return check_launch(what);
-}
-
 }  // namespace mi
 
 extern "C" int32_t mi_chunked_prefill_attention(
@@ -642,7 +880,8 @@ extern "C" int32_t mi_chunked_prefill_attention(
     return fail(MI_ERR_UNSUPPORTED, "%s: key/value token strides must be in [0, 2^24)", name);
   if (batch > 65535) return fail(MI_ERR_UNSUPPORTED, "%s: batch > 65535", name);
 
-  PrefillArgs a = rows_args(batch, padded_len, num_heads, num_kv_heads, scale);
+  const Form form = form_for(batch, padded_len, num_heads, num_kv_heads, max_history_blocks);
+  PrefillArgs a = rows_args(batch, padded_len, num_heads, num_kv_heads, scale, q_tile_of(form));
   a.out = static_cast<uint16_t*>(out);
   a.out_row = out_row_stride;
   a.out_tok = out_tok_stride;
@@ -667,7 +906,7 @@ extern "C" int32_t mi_chunked_prefill_attention(
   a.start_lens = start_lens;
   a.chunk_lens = chunk_lens;
   a.lens_stride = lens_stride;
-  return launch_rows(name, a, PrefillArgs{}, num_kv_heads, max_history_blocks, stream);
+  return launch_form(form, name, a, PrefillArgs{}, ZeroRows{}, num_kv_heads, max_history_blocks, stream);
 }
 
 extern "C" int32_t mi_mixed_paged_attention(
@@ -736,8 +975,13 @@ extern "C" int32_t mi_mixed_paged_attention(
     a.num_blocks = num_blocks;
   };
   PrefillArgs a0{}, a1{};
+  const int32_t hist = std::max(chunks ? max_history_blocks : 0, decode_rows > 0 ? max_blocks : 0);
+  // Decode rows alone: the shape whose LDS lets two workgroups share a CU.
+  Form form = !chunks ? Form::kWide : form_for(chunks ? prefill_rows : 0, prefill_width, num_heads, num_kv_heads, hist);
+  if (form == Form::kHalf && decode_rows > 0) form = Form::kWide;  // decode rows take eight wavefronts
+  const int q_tile = q_tile_of(form);
   if (chunks) {
-    a0 = rows_args(prefill_rows, prefill_width, num_heads, num_kv_heads, scale);
+    a0 = rows_args(prefill_rows, prefill_width, num_heads, num_kv_heads, scale, q_tile);
     fill(a0, 0, prefill_width);
     a0.history_blocks = history_blocks;
     a0.history_stride = history_stride;
@@ -749,7 +993,7 @@ extern "C" int32_t mi_mixed_paged_attention(
     a0.row_tokens = chunk_tokens;
   }
   if (decode_rows > 0) {
-    a1 = rows_args(decode_rows, 1, num_heads, num_kv_heads, scale);
+    a1 = rows_args(decode_rows, 1, num_heads, num_kv_heads, scale, q_tile);
     fill(a1, n, 1);
     a1.history_blocks = block_tables;
     a1.history_stride = block_table_stride;
@@ -760,12 +1004,16 @@ extern "C" int32_t mi_mixed_paged_attention(
     a1.decode_rows = 1;
     a1.slot_mapping = slot_mapping;
     a1.slot_stride = slot_stride;
+    // Block by block where the workgroup has kStripes wavefronts, the table has blocks and their ids fit its
+    // lanes; otherwise one-query tiles.
+    a1.stripes = form != Form::kHalf && max_blocks >= 1 && max_blocks <= kRowMaxBlocks && a1.group <= kRowMaxGroup;
+    if (a1.stripes) a1.groups = decode_rows * num_kv_heads;
   }
+  ZeroRows z{};
   if (ragged) {
-    rc = zero_uncovered_tokens(name, out, out_tok_stride, num_heads * head_dim, chunk_first, chunk_lens, lens_stride,
-                               chunks ? prefill_rows : 0, prefill_width, chunk_tokens, stream);
+    rc = zero_rows(z, name, out, out_tok_stride, num_heads * head_dim, chunk_first, chunk_lens, lens_stride,
+                   chunks ? prefill_rows : 0, prefill_width, chunk_tokens, Wide::kThreads);
     if (rc != MI_OK) return rc;
   }
-  return launch_rows(name, a0, a1, num_kv_heads,
-                     std::max(chunks ? max_history_blocks : 0, decode_rows > 0 ? max_blocks : 0), stream);
+  return launch_form(form, name, a0, a1, z, num_kv_heads, hist, stream);
 }

@@ -861,11 +861,17 @@ __device__ __forceinline__ double bf16_at(const u32x4 v, int e) {
 // one-token chunks (history: the context but the token; each as heavy as the chunk's heaviest
 // query tiles, so dispatched first), the rest the chunk rows of a0 -- the sums are exact, so the
 // decode rows get the bits of the exact decode body.
+// The last z.groups workgroups write zero rows.
 template <int kG, bool kCached>
-__global__ __launch_bounds__(kPfThreads) void exact_prefill_kernel(const ExactPrefillArgs a0, const ExactPrefillArgs a1) {
+__global__ __launch_bounds__(kPfThreads) void exact_prefill_kernel(const ExactPrefillArgs a0, const ExactPrefillArgs a1,
+                                                                   const ZeroRows z) {
   constexpr int kQP = kPfCols / kG;  // query positions of a workgroup
   constexpr int kCols = kQP * kG;    // columns in use (15 for G = 5)
   extern __shared__ __align__(16) unsigned char s_raw[];
+  if (static_cast<int>(blockIdx.x) >= a0.groups + a1.groups) {  // uniform
+    zero_uncovered_rows(z, static_cast<int>(blockIdx.x) - a0.groups - a1.groups, kPfThreads);
+    return;
+  }
   const bool decode = static_cast<int>(blockIdx.x) < a1.groups;  // uniform
   const ExactPrefillArgs a = decode ? a1 : a0;
   float* sM = reinterpret_cast<float*>(s_raw);                                    // [waves][16]
@@ -1202,34 +1208,36 @@ int32_t dispatch_exact_decode(const ExactDecodeArgs& a, int32_t batch, int group
 }
 
 template <int kG, bool kCached>
-int32_t launch_exact_prefill(const ExactPrefillArgs& a0, const ExactPrefillArgs& a1, const char* what, hipStream_t s) {
+int32_t launch_exact_prefill(const ExactPrefillArgs& a0, const ExactPrefillArgs& a1, const ZeroRows& z, const char* what,
+                             hipStream_t s) {
   static std::once_flag once;
   static int32_t attr_rc = MI_OK;
   std::call_once(once, [] { attr_rc = allow_lds(exact_prefill_kernel<kG, kCached>, kPfLdsBytes, "exact_prefill_kernel"); });
   if (attr_rc != MI_OK) return attr_rc;
-  if (a0.groups < 0 || a1.groups < 0 || static_cast<int64_t>(a0.groups) + a1.groups > 0x3fffffff)
+  if (a0.groups < 0 || a1.groups < 0 || static_cast<int64_t>(a0.groups) + a1.groups + z.groups > 0x3fffffff)
     return fail(MI_ERR_UNSUPPORTED, "%s: too many workgroups", what);
-  const int groups = a0.groups + a1.groups;
+  const int groups = a0.groups + a1.groups + z.groups;
   if (groups == 0) return ok();
   const size_t lds = static_cast<size_t>(kPfRedBytes) +
                      std::max(static_cast<size_t>(kPfMergeBytes),
                               kCached ? static_cast<size_t>(a0.cache_tiles) * kPfWaves * kPfCacheTileBytes : size_t{0});
-  exact_prefill_kernel<kG, kCached><<<groups, kPfThreads, lds, s>>>(a0, a1);
+  exact_prefill_kernel<kG, kCached><<<groups, kPfThreads, lds, s>>>(a0, a1, z);
   return check_launch(what);
 }
 
 // Both row sets share one score-cache size (the larger of the two; the recomputing form when
 // either set's rows are too long for the cache).
-int32_t dispatch_exact_prefill(ExactPrefillArgs a0, ExactPrefillArgs a1, int group, const char* what, hipStream_t s) {
+int32_t dispatch_exact_prefill(ExactPrefillArgs a0, ExactPrefillArgs a1, const ZeroRows& z, int group, const char* what,
+                               hipStream_t s) {
   const bool cached = (a0.groups == 0 || a0.cache_tiles > 0) && (a1.groups == 0 || a1.cache_tiles > 0);
   const int32_t tiles = cached ? std::max(a0.groups > 0 ? a0.cache_tiles : 0, a1.groups > 0 ? a1.cache_tiles : 0) : 0;
   a0.cache_tiles = a1.cache_tiles = tiles;
   switch (group) {
-    case 1: return cached ? launch_exact_prefill<1, true>(a0, a1, what, s) : launch_exact_prefill<1, false>(a0, a1, what, s);
-    case 2: return cached ? launch_exact_prefill<2, true>(a0, a1, what, s) : launch_exact_prefill<2, false>(a0, a1, what, s);
-    case 4: return cached ? launch_exact_prefill<4, true>(a0, a1, what, s) : launch_exact_prefill<4, false>(a0, a1, what, s);
-    case 5: return cached ? launch_exact_prefill<5, true>(a0, a1, what, s) : launch_exact_prefill<5, false>(a0, a1, what, s);
-    default: return cached ? launch_exact_prefill<8, true>(a0, a1, what, s) : launch_exact_prefill<8, false>(a0, a1, what, s);
+    case 1: return cached ? launch_exact_prefill<1, true>(a0, a1, z, what, s) : launch_exact_prefill<1, false>(a0, a1, z, what, s);
+    case 2: return cached ? launch_exact_prefill<2, true>(a0, a1, z, what, s) : launch_exact_prefill<2, false>(a0, a1, z, what, s);
+    case 4: return cached ? launch_exact_prefill<4, true>(a0, a1, z, what, s) : launch_exact_prefill<4, false>(a0, a1, z, what, s);
+    case 5: return cached ? launch_exact_prefill<5, true>(a0, a1, z, what, s) : launch_exact_prefill<5, false>(a0, a1, z, what, s);
+    default: return cached ? launch_exact_prefill<8, true>(a0, a1, z, what, s) : launch_exact_prefill<8, false>(a0, a1, z, what, s);
   }
 }
 
@@ -1430,7 +1438,7 @@ extern "C" int32_t mi_chunked_prefill_attention_exact(
   // Keys a row can see: its history (at most the table's) plus the chunk up to it.
   exact_rows(a, batch, padded_len, num_heads, num_kv_heads,
              static_cast<int64_t>(max_history_blocks) * kBlockSize + padded_len, scale);
-  const int32_t rc = dispatch_exact_prefill(a, ExactPrefillArgs{}, group, what, as_stream(stream));
+  const int32_t rc = dispatch_exact_prefill(a, ExactPrefillArgs{}, ZeroRows{}, group, what, as_stream(stream));
   return rc == MI_OK ? ok() : rc;
 }
 
@@ -1532,12 +1540,12 @@ extern "C" int32_t mi_mixed_paged_attention_exact(
     a1.slot_stride = slot_stride;
     exact_rows(a1, decode_rows, 1, num_heads, num_kv_heads, static_cast<int64_t>(max_blocks) * kBlockSize + 1, scale);
   }
+  ZeroRows z{};
   if (ragged) {
-    if (const int32_t rc = zero_uncovered_tokens(what, out, out_tok_stride, num_heads * head_dim, chunk_first, chunk_lens,
-                                                 lens_stride, chunks ? prefill_rows : 0, prefill_width, chunk_tokens,
-                                                 stream))
+    if (const int32_t rc = zero_rows(z, what, out, out_tok_stride, num_heads * head_dim, chunk_first, chunk_lens, lens_stride,
+                                     chunks ? prefill_rows : 0, prefill_width, chunk_tokens, kPfThreads))
       return rc;
   }
-  const int32_t rc = dispatch_exact_prefill(a0, a1, group, what, as_stream(stream));
+  const int32_t rc = dispatch_exact_prefill(a0, a1, z, group, what, as_stream(stream));
   return rc == MI_OK ? ok() : rc;
 }

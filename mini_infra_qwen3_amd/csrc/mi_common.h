@@ -17,14 +17,6 @@ int32_t ok();
 // Checks hipGetLastError() after a launch; MI_ERR_DEVICE with the HIP message.
 int32_t check_launch(const char* what);
 
-// Zeroes the out rows of the tokens of [0, row_tokens) that no ragged chunk row of a mixed step
-// covers (row b covers tokens first[b] .. first[b] + len_b - 1, with len_b = lens[b lens_stride]
-// clamped to [0, width] and first[b] to [0, row_tokens - len_b], as the attention kernels clamp
-// them); row_elems bf16 values per token, token stride out_tok_stride.  One launch on `stream`.
-int32_t zero_uncovered_tokens(const char* what, void* out, int64_t out_tok_stride, int32_t row_elems,
-                              const int64_t* first, const int64_t* lens, int64_t lens_stride, int32_t rows,
-                              int32_t width, int64_t row_tokens, void* stream);
-
 // 16-byte vector used by the streaming copies (a native vector type, so the
 // non-temporal builtins accept it).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -112,6 +104,9 @@ __device__ __forceinline__ float bf16_hi(uint32_t pair) { return __uint_as_float
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
+  // Contraction off: with it a compiler may fold a double -> float -> bf16 chain into one rounding, while
+  // the definitions here round twice.
+#pragma clang fp contract(off)
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
 }
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) { return pack_bf16x2(f, 0.0f); }
@@ -188,6 +183,57 @@ __device__ __forceinline__ int wave_sum_i32(int x) {
   const uint32_t y = p[0] + p[1];
   const auto q = __builtin_amdgcn_permlane32_swap(y, y, false, false);
   return static_cast<int>(q[0] + q[1]);
+}
+
+// ------------------------------------------- tokens no ragged row covers ---
+// A mixed step's out rows of the tokens of [0, tokens) that no ragged chunk row covers are zeros (row b
+// covers tokens first[b] .. first[b] + len_b - 1, with len_b = lens[b lens_stride] clamped to [0, width] and
+// first[b] to [0, tokens - len_b], as the attention kernels clamp them).  The mixed kernels give this to
+// `groups` workgroups at the end of their grid; as a launch of its own it took 2.4 us beside them.
+struct ZeroRows {
+  uint16_t* out;       // rows of row_elems values, 16-byte aligned, row_elems and out_tok multiples of 8
+  int64_t out_tok;     // elements
+  const int64_t* first;
+  const int64_t* lens;
+  int64_t lens_stride;
+  int64_t tokens;
+  int32_t rows, width, row_elems;
+  int32_t groups;      // workgroups: ceil(tokens / threads)
+};
+// Workgroup `group` of them: one token per thread, the chunk rows read 64 at a time by each wavefront.
+__device__ __forceinline__ void zero_uncovered_rows(const ZeroRows& z, int group, int threads) {
+  const int lane = threadIdx.x & 63;
+  const int64_t t = static_cast<int64_t>(group) * threads + threadIdx.x;
+  bool live = t < z.tokens;
+  for (int b0 = 0; b0 < z.rows; b0 += 64) {
+    const int b = min(b0 + lane, z.rows - 1);
+    int64_t len = z.lens[b * z.lens_stride];
+    len = len < 0 ? 0 : (len > z.width ? z.width : len);
+    int64_t f = z.first[b];
+    f = f < 0 ? 0 : (f > z.tokens - len ? z.tokens - len : f);
+    const int n = min(z.rows - b0, 64);
+    for (int k = 0; k < n; ++k) {
+      // first + length fit 32 bits: the entry points take fewer than 2^31 chunk tokens
+      const int fk = __builtin_amdgcn_readlane(static_cast<int>(f), k);
+      const int lk = __builtin_amdgcn_readlane(static_cast<int>(len), k);
+      live = live && !(t >= fk && t < static_cast<int64_t>(fk) + lk);
+    }
+  }
+  for (uint64_t todo = __builtin_amdgcn_ballot_w64(live); todo != 0; todo &= todo - 1) {  // wave-uniform
+    const int64_t row = t - lane + __builtin_ctzll(todo);
+    uint16_t* out = z.out + row * z.out_tok;
+    for (int i = lane; i < z.row_elems / 8; i += 64) *reinterpret_cast<u32x4*>(out + 8 * i) = u32x4{0u, 0u, 0u, 0u};
+  }
+}
+// Fills z for a launch of `threads` per workgroup; groups 0 when there is nothing to cover.
+inline int32_t zero_rows(ZeroRows& z, const char* what, void* out, int64_t out_tok_stride, int32_t row_elems,
+                         const int64_t* first, const int64_t* lens, int64_t lens_stride, int32_t rows, int32_t width,
+                         int64_t tokens, int threads) {
+  if (tokens <= 0) return MI_OK;
+  if (tokens > 0x7fffffff) return fail(MI_ERR_UNSUPPORTED, "%s: more than 2^31 - 1 chunk tokens", what);
+  z = ZeroRows{static_cast<uint16_t*>(out), out_tok_stride, first, lens, lens_stride, tokens, rows, width, row_elems,
+               static_cast<int32_t>((tokens + threads - 1) / threads)};
+  return MI_OK;
 }
 
 // ------------------------------------------------------- RMSNorm, exact ---

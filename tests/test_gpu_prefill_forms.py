@@ -1,0 +1,122 @@
+"""The workgroup shapes of chunked prefill (chosen by the launch's size), each at its query and key tile
+edges, and a mixed step's decode rows at the limits of their block-by-block form.  Against the oracle with
+the tolerance of the prefill tests (2e-2 max-abs on bf16 outputs)."""
+
+import pytest
+import torch
+
+from mini_infra_qwen3_amd import data_plane, workloads
+from oracle import torch_ref
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-2
+SCALE = 128 ** -0.5
+
+
+def _chunk_case(seed, starts, lens, kv_heads, group):
+    gen = torch.Generator().manual_seed(seed)
+    width, rows = max(lens), len(lens)
+    totals = [s + n for s, n in zip(starts, lens)]
+    num_blocks = 1 + sum(-(-t // 16) for t in totals)
+    tables = workloads.permuted_tables(totals, num_blocks, gen)
+    kp, vp = (torch.randn(num_blocks, 16, kv_heads, 128, generator=gen).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(rows, group * kv_heads, width, 128, generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn(rows, kv_heads, width, 128, generator=gen).to(torch.bfloat16) for _ in range(2))
+    hist = torch.zeros((rows, max(-(-s // 16) for s in starts)), dtype=torch.long)
+    for b, s in enumerate(starts):
+        hist[b, :-(-s // 16)] = torch.tensor(tables[b][:-(-s // 16)], dtype=torch.long)
+    return q, k, v, kp, vp, hist
+
+
+# Wide-shape workgroups (rows x head pairs x 128-query tiles) decide: below 128 the 32-query split shape,
+# to 247 the 64-query split shape, 248 to 256 and from 512 the wide one, between them the 64-query one.
+@pytest.mark.parametrize("starts,lens,kv_heads,group", [
+    ([0], [1], 8, 2),                              # 8: one query, one key, the second key half idle
+    ([64, 0], [33, 32], 8, 2),                     # 16: one past a 32-query tile
+    ([129, 63, 1], [65, 64, 31], 8, 5),            # 72: odd group, an odd number of key tiles
+    ([0] * 15, [130 - i for i in range(15)], 4, 2),          # 120: the last below 128
+    ([0, 70] * 8, [129 + i for i in range(16)], 4, 2),       # 128: 64-query tiles with split keys
+    ([17] * 31, [97 + i for i in range(31)], 8, 2),          # 248: wide
+    ([0] * 11, [257 + i for i in range(11)], 8, 2),          # 264: 64-query tiles
+    ([0] * 64, [1 + i for i in range(64)], 8, 2),            # 512: wide
+])
+def test_shapes_match_oracle(native_lib, device, starts, lens, kv_heads, group):
+    q, k, v, kp, vp, hist = _chunk_case(len(lens) + sum(lens), starts, lens, kv_heads, group)
+    got = data_plane.chunked_prefill_attention(
+        *(t.to(device) for t in (q, k, v, kp, vp, hist)), torch.tensor(starts, device=device),
+        torch.tensor(lens, device=device), SCALE).float().cpu()
+    ref = torch_ref.chunked_prefill_attention(q, k, v, (kp, vp), hist, starts, lens, SCALE).float()
+    width = q.shape[2]
+    for b, n in enumerate(lens):
+        assert (got[b, width - n:] - ref[b, width - n:]).abs().max().item() <= TOL, f"row {b}"
+        assert not got[b, :width - n].any(), f"row {b}: padding rows must be zero"
+
+
+def _decode_rows(seed, contexts, max_blocks, group, kv_heads):
+    gen = torch.Generator().manual_seed(seed)
+    rows = len(contexts)
+    num_blocks = 1 + rows * max(max_blocks, 1)
+    kp, vp = (torch.randn(num_blocks, 16, kv_heads, 128, generator=gen).to(torch.bfloat16) for _ in range(2))
+    table = (torch.randperm(num_blocks - 1, generator=gen) + 1)[:rows * max_blocks].view(rows, max_blocks)
+    q = torch.randn(rows, group * kv_heads, 128, generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn(rows, kv_heads, 128, generator=gen).to(torch.bfloat16) for _ in range(2))
+    return q, k, v, kp, vp, table
+
+
+# Tables of 511 blocks are the last attended block by block; contexts that end on a block, one past it, and
+# past the table (the history is what the table holds, the token comes after it); no table at all.
+@pytest.mark.parametrize("contexts,max_blocks", [
+    ([1, 2, 16, 17, 128, 129, 0], 9),
+    ([160, 161, 500], 10),
+    ([8176, 8177, 9000, 8000], 511),
+    ([8192, 8193, 100], 512),
+    ([1, 0, 40], 0),
+])
+@pytest.mark.parametrize("group,kv_heads", [(2, 8), (8, 4), (1, 2), (16, 1)])
+def test_decode_rows_of_a_mixed_step(native_lib, device, contexts, max_blocks, group, kv_heads):
+    q, k, v, kp, vp, table = _decode_rows(len(contexts) + max_blocks, contexts, max_blocks, group, kv_heads)
+    rows = len(contexts)
+    none = torch.zeros(0, dtype=torch.long, device=device)
+    pools = kp.to(device), vp.to(device)
+    out = data_plane.mixed_paged_attention(
+        q.to(device), k.to(device), v.to(device), *pools, 0, 0, torch.zeros((0, 0), dtype=torch.long, device=device), none,
+        none, table.to(device), torch.tensor(contexts).to(device), torch.full((rows,), -1).to(device), SCALE).float().cpu()
+    assert torch.equal(pools[0].cpu(), kp) and torch.equal(pools[1].cpu(), vp)
+    for b, n in enumerate(contexts):
+        if n == 0:
+            assert not out[b].any()
+            continue
+        nh = min(n - 1, 16 * max_blocks)
+        keys = torch.cat((kp[table[b]].view(-1, kv_heads, 128)[:nh], k[b:b + 1]))
+        values = torch.cat((vp[table[b]].view(-1, kv_heads, 128)[:nh], v[b:b + 1]))
+        s = torch.einsum("hd,thd->ht", q[b].float(), keys.float().repeat_interleave(group, 1)).to(torch.bfloat16)
+        p = (s * SCALE).to(torch.bfloat16).float().softmax(-1).to(torch.bfloat16)
+        ref = torch.einsum("ht,thd->hd", p.float(), values.float().repeat_interleave(group, 1)).reshape(-1)
+        assert (out[b] - ref).abs().max().item() <= TOL, f"row {b}"
+
+
+def test_uncovered_tokens_of_many_rows(native_lib, device):
+    """130 ragged rows (three reads of 64 by the zeroing workgroups) with a gap before each: zero rows there."""
+    rows, kv_heads, heads = 130, 2, 4
+    gen = torch.Generator().manual_seed(5)
+    lens = torch.randint(0, 6, (rows,), generator=gen)
+    gaps = torch.randint(0, 3, (rows,), generator=gen)
+    first = torch.cumsum(lens + gaps, 0) - lens
+    tokens = int(first[-1] + lens[-1]) + 3
+    q = torch.randn(tokens, heads, 128, generator=gen).to(torch.bfloat16).to(device)
+    k, v = (torch.randn(tokens, kv_heads, 128, generator=gen).to(torch.bfloat16).to(device) for _ in range(2))
+    pool = torch.zeros(2, 16, kv_heads, 128, dtype=torch.bfloat16, device=device)
+    none = torch.zeros(0, dtype=torch.long, device=device)
+    covered = torch.zeros(tokens, dtype=torch.bool)
+    for f, n in zip(first.tolist(), lens.tolist()):
+        covered[f:f + n] = True
+    for exact in (False, True):
+        torch.full((tokens, heads * 128), float("nan"), dtype=torch.bfloat16, device=device)  # likely the next buffer
+        out = data_plane.mixed_paged_attention(
+            q, k, v, pool.clone(), pool.clone(), rows, 6, torch.zeros((rows, 0), dtype=torch.long, device=device),
+            torch.zeros(rows, dtype=torch.long, device=device), lens.to(device),
+            torch.zeros((0, 1), dtype=torch.long, device=device), none, none, SCALE, exact=exact,
+            chunk_first=first.to(device), chunk_tokens=tokens).cpu()
+        assert not out[~covered].any()
+        assert (out[covered].float().abs().sum(1) > 0).all() and torch.isfinite(out[covered].float()).all()
