@@ -161,8 +161,11 @@ struct DecodeLds {
 
 // Exact decode attention of sequence b, KV head g, by the workgroup's kWaves wavefronts.  kPrologue:
 // q / k RMSNorm + RoPE from the raw projection rows and the K/V append.  Plain form: rotated
-// queries; with a.slot_mapping set the rows a.k_new / a.v_new (already rotated) are appended first.
-template <int kG, bool kPrologue, int kWaves>
+// queries.  kToken (plain form, a mixed step's decode rows): the context's last token is not in the pool
+// but in the rows a.k_new / a.v_new (already rotated); they are appended to the row's slot, and attended
+// in place of what the position after the history (the context but the token, as far as the table holds
+// it) has.
+template <int kG, bool kPrologue, bool kToken, int kWaves>
 __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const int g, unsigned char* smem) {
   constexpr int kDecWaves = kWaves;
   constexpr int kDecThreads = 64 * kWaves;
@@ -211,7 +214,7 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
       const int j = i / kHeadDim, d = i - j * kHeadDim;
       s_q[j][d] = bf16_bits_to_f32(a.q[b * a.q_row + (g * kG + j) * a.q_head + d]);
     }
-    if (a.slot_mapping && threadIdx.x < 32) {  // append the token's rotated K and V rows of KV head g
+    if (kToken && threadIdx.x < 32) {  // append the token's rotated K and V rows of KV head g
       const int64_t slot = a.slot_mapping[b * a.slot_stride];
       const int64_t ctx = a.context_lens[b * a.ctx_stride];
       if (ctx > 0 && slot >= 0 && slot < a.num_slots) {
@@ -227,7 +230,10 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
   __syncthreads();
 
   int64_t n64 = a.context_lens[b * a.ctx_stride];
-  n64 = min(n64, static_cast<int64_t>(a.max_blocks) * kBlockSize);
+  if (kToken)
+    n64 = n64 > 0 ? min(n64 - 1, static_cast<int64_t>(a.max_blocks) * kBlockSize) + 1 : 0;
+  else
+    n64 = min(n64, static_cast<int64_t>(a.max_blocks) * kBlockSize);
   const int n = n64 > 0 ? static_cast<int>(n64) : 0;
   const int nblk = (n + kBlockSize - 1) / kBlockSize;
   uint16_t* out_b = a.out + b * a.out_row + (g * kG) * kHeadDim;
@@ -246,8 +252,10 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
   // kGrp at a time, all loads of a group issued before any is used, so a pass costs about one
   // memory round trip per group instead of two per block.
   int64_t lane_id = 0;
+  // With kToken the last block may be one past the table: it repeats the table's last one.
+  const int last_entry = max(a.max_blocks - 1, 0);
   if (lane < cnt) {
-    lane_id = a.block_tables[b * a.bt_stride + w + kDecWaves * lane];
+    lane_id = a.block_tables[b * a.bt_stride + min(w + kDecWaves * lane, last_entry)];
     if (lane_id < 0 || lane_id >= a.num_blocks) lane_id = 0;
   }
   auto block_id = [&](int i) -> int64_t {  // i is wave-uniform
@@ -256,7 +264,7 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
       const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(static_cast<uint64_t>(lane_id) >> 32), i);
       return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
     }
-    const int64_t id = a.block_tables[b * a.bt_stride + w + kDecWaves * i];
+    const int64_t id = a.block_tables[b * a.bt_stride + min(w + kDecWaves * i, last_entry)];
     return id < 0 || id >= a.num_blocks ? 0 : id;
   };
   // Blocks i0 .. i0 + kGrp - 1 of the wavefront (indices past its last block reload the last
@@ -267,6 +275,20 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
       const uint16_t* p = pool + block_id(min(i0 + q, cnt - 1)) * kBlockSize * row_elems + lane_off;
 #pragma unroll
       for (int t = 0; t < 4; ++t) buf[q][t] = *reinterpret_cast<const u32x4*>(p + 4 * t * row_elems);
+    }
+  };
+  // The token's row (its 8 dims of this lane) in place of its position in the last block.
+  u32x4 k_tok{}, v_tok{};
+  if constexpr (kToken) {
+    k_tok = *reinterpret_cast<const u32x4*>(a.k_new + b * a.k_row + g * a.k_head + 8 * dl);
+    v_tok = *reinterpret_cast<const u32x4*>(a.v_new + b * a.v_row + g * a.v_head + 8 * dl);
+  }
+  auto put_token = [&](int i, u32x4 (&buf)[4], const u32x4 row) {  // block i of the wavefront
+    if constexpr (kToken) {
+      if (w + kDecWaves * i != nblk - 1) return;  // wave-uniform
+      const int at = (n - 1) % kBlockSize;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) buf[t] = 4 * t + r == at ? row : buf[t];
     }
   };
   // Scores of the lane row's 4 tokens of block i against the kG queries (equal in the 16 lanes of
@@ -304,6 +326,7 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
     for (int q = 0; q < kGrp; ++q) {
       if (i0 + q >= cnt) break;
       float s[4][kG];
+      put_token(i0 + q, kb[q], k_tok);
       block_scores(kb[q], s);
       const int tok0 = (w + kDecWaves * (i0 + q)) * kBlockSize + r;
 #pragma unroll
@@ -354,6 +377,7 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
       for (int q = 0; q < kGrp; ++q) {
         if (i0 + q >= cnt) break;
         float s[4][kG];
+        put_token(i0 + q, kb[q], k_tok);
         block_scores(kb[q], s);
         const int tok0 = (w + kDecWaves * (i0 + q)) * kBlockSize + r;
 #pragma unroll
@@ -412,6 +436,7 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
     for (int q = 0; q < kGrp; ++q) {
       if (i0 + q >= cnt) break;
       float p[4][kG];
+      put_token(i0 + q, vb[q], v_tok);
       const int tok0 = (w + kDecWaves * (i0 + q)) * kBlockSize + r;
       if (cached) {
 #pragma unroll
@@ -422,6 +447,7 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
         }
       } else {
         float s[4][kG];
+        put_token(i0 + q, kb[q], k_tok);
         block_scores(kb[q], s);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -470,10 +496,10 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
   }
 }
 
-template <int kG, bool kPrologue>
+template <int kG, bool kPrologue, bool kToken>
 __global__ __launch_bounds__(kDecThreads) void exact_decode_kernel(const ExactDecodeArgs a) {
   extern __shared__ __align__(16) unsigned char s_dec[];
-  exact_decode_body<kG, kPrologue, kDecWaves>(a, blockIdx.x, blockIdx.y, s_dec);
+  exact_decode_body<kG, kPrologue, kToken, kDecWaves>(a, blockIdx.x, blockIdx.y, s_dec);
 }
 
 // ------------------------------------------------------------------ split decode ---
@@ -857,13 +883,13 @@ __device__ __forceinline__ double bf16_at(const u32x4 v, int e) {
   return (e & 1) ? bf16_hi(x) : bf16_lo(x);
 }
 
-// One launch serves a mixed step: the first a1.groups workgroups take the decode rows of a1 as
-// one-token chunks (history: the context but the token; each as heavy as the chunk's heaviest
-// query tiles, so dispatched first), the rest the chunk rows of a0 -- the sums are exact, so the
-// decode rows get the bits of the exact decode body.
-// The last z.groups workgroups write zero rows.
+// One launch serves the chunk rows of a0 after, in the first a1.groups workgroups, a mixed step's decode
+// rows where they have no table (as one-token chunks; with a table the decode body takes them in a launch of
+// its own).  The sums are exact, so both give the same bits.
+// The last z.groups workgroups write zero rows.  Three wavefronts per SIMD: two rows of 500-1024 tokens took
+// 87.2 us, 92.4 with the registers of four (8 bytes of them spilled).
 template <int kG, bool kCached>
-__global__ __launch_bounds__(kPfThreads) void exact_prefill_kernel(const ExactPrefillArgs a0, const ExactPrefillArgs a1,
+__global__ __launch_bounds__(kPfThreads, 3) void exact_prefill_kernel(const ExactPrefillArgs a0, const ExactPrefillArgs a1,
                                                                    const ZeroRows z) {
   constexpr int kQP = kPfCols / kG;  // query positions of a workgroup
   constexpr int kCols = kQP * kG;    // columns in use (15 for G = 5)
@@ -1125,18 +1151,18 @@ int32_t allow_lds(Kernel kernel, int bytes, const char* what) {
   return MI_OK;
 }
 
-template <int kG, bool kPrologue>
-int32_t launch_exact_decode(const ExactDecodeArgs& a, int32_t batch, hipStream_t s) {
+template <int kG, bool kPrologue, bool kToken>
+int32_t launch_exact_decode(const ExactDecodeArgs& a, int32_t batch, const char* what, hipStream_t s) {
   static std::once_flag once;
   static int32_t attr_rc = MI_OK;
   using Lds = DecodeLds<kG, kDecWaves>;
   std::call_once(once, [] {
-    attr_rc = allow_lds(exact_decode_kernel<kG, kPrologue>, Lds::kFixed + kDecCacheBytes, "mi_paged_decode_attention_exact");
+    attr_rc = allow_lds(exact_decode_kernel<kG, kPrologue, kToken>, Lds::kFixed + kDecCacheBytes, "exact_decode_kernel");
   });
   if (attr_rc != MI_OK) return attr_rc;
   const size_t lds = Lds::kFixed + static_cast<size_t>(a.cache_tokens) * kG * sizeof(uint16_t);
-  exact_decode_kernel<kG, kPrologue><<<dim3(batch, a.kv_heads), kDecThreads, lds, s>>>(a);
-  return check_launch("mi_paged_decode_attention_exact");
+  exact_decode_kernel<kG, kPrologue, kToken><<<dim3(batch, a.kv_heads), kDecThreads, lds, s>>>(a);
+  return check_launch(what);
 }
 
 template <int kG, bool kPrologue>
@@ -1196,14 +1222,14 @@ ExactSplitLayout exact_split_layout(int32_t batch, int32_t max_blocks, int32_t n
   return l;
 }
 
-template <bool kPrologue>
-int32_t dispatch_exact_decode(const ExactDecodeArgs& a, int32_t batch, int group, hipStream_t s) {
+template <bool kPrologue, bool kToken>
+int32_t dispatch_exact_decode(const ExactDecodeArgs& a, int32_t batch, int group, const char* what, hipStream_t s) {
   switch (group) {
-    case 1: return launch_exact_decode<1, kPrologue>(a, batch, s);
-    case 2: return launch_exact_decode<2, kPrologue>(a, batch, s);
-    case 4: return launch_exact_decode<4, kPrologue>(a, batch, s);
-    case 5: return launch_exact_decode<5, kPrologue>(a, batch, s);
-    default: return launch_exact_decode<8, kPrologue>(a, batch, s);
+    case 1: return launch_exact_decode<1, kPrologue, kToken>(a, batch, what, s);
+    case 2: return launch_exact_decode<2, kPrologue, kToken>(a, batch, what, s);
+    case 4: return launch_exact_decode<4, kPrologue, kToken>(a, batch, what, s);
+    case 5: return launch_exact_decode<5, kPrologue, kToken>(a, batch, what, s);
+    default: return launch_exact_decode<8, kPrologue, kToken>(a, batch, what, s);
   }
 }
 
@@ -1371,7 +1397,8 @@ extern "C" int32_t mi_paged_decode_attention_exact(
       c.sin = a.sin + b0 * static_cast<int64_t>(head_dim);
       c.slot_mapping = slot_mapping + b0 * slot_stride;
     }
-    const int32_t rc = prologue ? dispatch_exact_decode<true>(c, nb, group, s) : dispatch_exact_decode<false>(c, nb, group, s);
+    const int32_t rc = prologue ? dispatch_exact_decode<true, false>(c, nb, group, what, s)
+                                : dispatch_exact_decode<false, false>(c, nb, group, what, s);
     if (rc != MI_OK) return rc;
   }
   return ok();
@@ -1539,6 +1566,41 @@ extern "C" int32_t mi_mixed_paged_attention_exact(
     a1.slot_mapping = slot_mapping;
     a1.slot_stride = slot_stride;
     exact_rows(a1, decode_rows, 1, num_heads, num_kv_heads, static_cast<int64_t>(max_blocks) * kBlockSize + 1, scale);
+    if (max_blocks > 0) {
+      // Tables with blocks: the decode body, in a launch of its own.  As one-token chunks beside the chunk
+      // rows a decode row was the launch's longest chain (four wavefronts, 2 of 16 matrix columns in use):
+      // one chunk of 400-650 tokens with 7 decode rows 110 -> 76 us, one of 60-120 with 16 103 -> 39.  Inside
+      // the chunk kernel the decode body's registers (224) would halve the chunk rows' wavefronts.
+      ExactDecodeArgs d{};
+      d.out = a1.out;
+      d.out_row = a1.out_row;
+      d.q = a1.q;
+      d.q_row = a1.q_row;
+      d.q_head = a1.q_head;
+      d.k_new = a1.k;
+      d.v_new = a1.v;
+      d.k_row = a1.k_row;
+      d.v_row = a1.v_row;
+      d.k_head = a1.k_head;
+      d.v_head = a1.v_head;
+      d.slot_mapping = slot_mapping;
+      d.slot_stride = slot_stride;
+      d.num_slots = num_blocks * kBlockSize;
+      d.key_pool = a1.key_pool;
+      d.value_pool = a1.value_pool;
+      d.num_blocks = num_blocks;
+      d.kv_heads = num_kv_heads;
+      d.block_tables = block_tables;
+      d.bt_stride = block_table_stride;
+      d.max_blocks = max_blocks;
+      d.context_lens = context_lens;
+      d.ctx_stride = context_lens_stride;
+      d.scale = scale;
+      const int64_t tokens = static_cast<int64_t>(max_blocks) * kBlockSize + 1;
+      d.cache_tokens = tokens * group * 2 <= kDecCacheBytes ? static_cast<int32_t>(tokens) : 0;
+      if (const int32_t rc = dispatch_exact_decode<false, true>(d, decode_rows, group, what, as_stream(stream))) return rc;
+      a1.groups = 0;
+    }
   }
   ZeroRows z{};
   if (ragged) {

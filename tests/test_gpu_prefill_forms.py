@@ -73,15 +73,17 @@ def _decode_rows(seed, contexts, max_blocks, group, kv_heads):
     ([8192, 8193, 100], 512),
     ([1, 0, 40], 0),
 ])
-@pytest.mark.parametrize("group,kv_heads", [(2, 8), (8, 4), (1, 2), (16, 1)])
-def test_decode_rows_of_a_mixed_step(native_lib, device, contexts, max_blocks, group, kv_heads):
+@pytest.mark.parametrize("group,kv_heads,exact", [(2, 8, False), (8, 4, False), (1, 2, False), (16, 1, False),
+                                                  (2, 8, True), (8, 2, True), (5, 1, True)])
+def test_decode_rows_of_a_mixed_step(native_lib, device, contexts, max_blocks, group, kv_heads, exact):
     q, k, v, kp, vp, table = _decode_rows(len(contexts) + max_blocks, contexts, max_blocks, group, kv_heads)
     rows = len(contexts)
     none = torch.zeros(0, dtype=torch.long, device=device)
     pools = kp.to(device), vp.to(device)
     out = data_plane.mixed_paged_attention(
         q.to(device), k.to(device), v.to(device), *pools, 0, 0, torch.zeros((0, 0), dtype=torch.long, device=device), none,
-        none, table.to(device), torch.tensor(contexts).to(device), torch.full((rows,), -1).to(device), SCALE).float().cpu()
+        none, table.to(device), torch.tensor(contexts).to(device), torch.full((rows,), -1).to(device), SCALE,
+        exact=exact).float().cpu()
     assert torch.equal(pools[0].cpu(), kp) and torch.equal(pools[1].cpu(), vp)
     for b, n in enumerate(contexts):
         if n == 0:
