@@ -35,6 +35,8 @@ __all__ = [
 
 
 def _require_gpu(name: str, tensor: torch.Tensor, device: torch.device | None = None) -> None:
+    if tensor.is_cuda and (device is None or tensor.device == device):
+        return
     if tensor.device.type != "cuda":
         raise RuntimeError(
             f"{name} is on {tensor.device}: the paged-KV data plane runs only on the GPU (no CPU fallback)"
@@ -49,7 +51,9 @@ def _require_index(name: str, tensor: torch.Tensor, ndim: int) -> None:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # The raw handle, without the Stream object that torch.cuda.current_stream() builds around it (0.1 us
+    # against 0.8; the small launches below are bound by this file: 22 us a decode call whose kernel takes 7).
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 _INDEX_CHECKS = os.environ.get("MI_CHECK_INDICES", "") == "1"
@@ -109,19 +113,24 @@ def reshape_and_cache(
     if pool0.ndim != 4:
         raise ValueError(f"pools must be [num_blocks, block_size, H_kv, D], got {tuple(pool0.shape)}")
     num_blocks, block_size, num_kv_heads, head_dim = pool0.shape
+    index, shape, dtype = pool0.get_device(), pool0.shape, pool0.dtype
     for name, tensors in (("key_pools", key_pools), ("value_pools", value_pools)):
         for t in tensors:
-            _require_gpu(name, t, device)
-            if t.shape != pool0.shape or t.dtype != pool0.dtype or not t.is_contiguous():
+            if index < 0 or t.get_device() != index:
+                _require_gpu(name, t, device)
+            if t.shape != shape or t.dtype is not dtype or not t.is_contiguous():
                 raise ValueError(f"{name}: every pool must be contiguous {tuple(pool0.shape)} {pool0.dtype}")
     k0, v0 = key_src[0], value_src[0]
     for name, tensors, ref in (("key_src", key_src, k0), ("value_src", value_src, v0)):
+        ref_shape, ref_stride = ref.shape, ref.stride()
         for t in tensors:
-            _require_gpu(name, t, device)
-            if t.ndim != 4 or t.shape[1] != num_kv_heads or t.shape[3] != head_dim or t.dtype != pool0.dtype:
+            if index < 0 or t.get_device() != index:
+                _require_gpu(name, t, device)
+            t_shape = t.shape
+            if len(t_shape) != 4 or t_shape[1] != num_kv_heads or t_shape[3] != head_dim or t.dtype is not dtype:
                 raise ValueError(f"{name} must be [B, {num_kv_heads}, L, {head_dim}] {pool0.dtype}, got "
                                  f"{tuple(t.shape)} {t.dtype}")
-            if t.stride() != ref.stride() or t.shape != ref.shape or t.stride(3) != 1:
+            if t.stride() != ref_stride or t_shape != ref_shape or ref_stride[3] != 1:
                 raise ValueError(f"{name}: all layers need the same shape and strides, with D contiguous")
     if k0.shape[:3] != v0.shape[:3]:
         raise ValueError("reshape_and_cache: key and value sources differ in shape")
@@ -386,29 +395,43 @@ def paged_decode_attention_fused(
     Returns ``out`` ``[B, Hq * 128]``.
     """
     device = key_pool.device
-    for name, t in (("q", q), ("k", k), ("v", v), ("q_weight", q_weight), ("k_weight", k_weight), ("cos", cos),
-                    ("sin", sin)):
-        _require_bf16_rows(name, t, device)
-    for name, t in (("key_pool", key_pool), ("value_pool", value_pool), ("block_tables", block_tables),
-                    ("context_lens", context_lens), ("slot_mapping", slot_mapping)):
-        _require_gpu(name, t, device)
+    bf16 = torch.bfloat16
+    # One chained comparison where all is well; the loops below name what is not.
+    if not (0 <= key_pool.get_device() == value_pool.get_device() == q.get_device() == k.get_device()
+            == v.get_device() == q_weight.get_device() == k_weight.get_device() == cos.get_device()
+            == sin.get_device() == block_tables.get_device() == context_lens.get_device()
+            == slot_mapping.get_device()
+            and q.dtype is k.dtype is v.dtype is q_weight.dtype is k_weight.dtype is cos.dtype is sin.dtype is bf16
+            and q.stride(-1) == k.stride(-1) == v.stride(-1) == q_weight.stride(-1) == k_weight.stride(-1)
+            == cos.stride(-1) == sin.stride(-1) == 1):
+        for name, t in (("q", q), ("k", k), ("v", v), ("q_weight", q_weight), ("k_weight", k_weight), ("cos", cos),
+                        ("sin", sin)):
+            _require_bf16_rows(name, t, device)
+        for name, t in (("key_pool", key_pool), ("value_pool", value_pool), ("block_tables", block_tables),
+                        ("context_lens", context_lens), ("slot_mapping", slot_mapping)):
+            _require_gpu(name, t, device)
     _require_index("block_tables", block_tables, 2)
     _require_index("context_lens", context_lens, 1)
     _require_index("slot_mapping", slot_mapping, 1)
-    if key_pool.dtype != torch.bfloat16 or value_pool.shape != key_pool.shape or value_pool.dtype != key_pool.dtype \
+    pool_shape = key_pool.shape
+    if key_pool.dtype is not bf16 or value_pool.shape != pool_shape or value_pool.dtype is not bf16 \
             or not key_pool.is_contiguous() or not value_pool.is_contiguous():
         raise ValueError("pools must be contiguous bf16 with identical shapes")
     head_dim = q_weight.shape[-1]
     batch = q.numel() // q.shape[-1]
-    q2, k2, v2 = q.reshape(batch, -1), k.reshape(batch, -1), v.reshape(batch, -1)
+    q2 = q if q.ndim == 2 else q.reshape(batch, -1)
+    k2 = k if k.ndim == 2 else k.reshape(batch, -1)
+    v2 = v if v.ndim == 2 else v.reshape(batch, -1)
     num_heads, num_kv_heads = q2.shape[1] // head_dim, k2.shape[1] // head_dim
-    cos2, sin2 = cos.reshape(batch, head_dim).contiguous(), sin.reshape(batch, head_dim).contiguous()
-    if v2.shape != k2.shape or k_weight.shape != q_weight.shape or key_pool.shape[2:] != (num_kv_heads, head_dim):
+    rows = (batch, head_dim)
+    cos2 = cos if cos.shape == rows and cos.is_contiguous() else cos.reshape(rows).contiguous()
+    sin2 = sin if sin.shape == rows and sin.is_contiguous() else sin.reshape(rows).contiguous()
+    if v2.shape != k2.shape or k_weight.shape != q_weight.shape or pool_shape[2:] != (num_kv_heads, head_dim):
         raise ValueError("q / k / v / weights / pools have inconsistent head sizes")
     if block_tables.shape[0] != batch or context_lens.shape[0] != batch or slot_mapping.shape[0] != batch:
         raise ValueError("block_tables / context_lens / slot_mapping batch differs from the tokens'")
-    _check_range("block_tables", block_tables, key_pool.shape[0])
-    _check_range("slot_mapping", slot_mapping, key_pool.shape[0] * key_pool.shape[1], allow_minus_one=True)
+    _check_range("block_tables", block_tables, pool_shape[0])
+    _check_range("slot_mapping", slot_mapping, pool_shape[0] * pool_shape[1], allow_minus_one=True)
     key_pool, value_pool, block_tables = _as_kernel_blocks(key_pool, value_pool, block_tables)
     num_blocks, block_size = key_pool.shape[:2]
     if block_tables.stride(1) != 1:
