@@ -39,7 +39,11 @@ class DeviceBlockTables:
 
     def sync(self) -> int:
         """Uploads the entries written since the last call (one copy of ``[2, n]`` int64 and one
-        scatter on the current stream); returns n."""
+        scatter on the current stream); returns n.
+
+        An entry written more than once since then (its row was freed and taken by another request
+        between two calls, as happens while steps pack their own tables) goes up once, with its last
+        id: the device scatter leaves either id of a repeated index."""
         rows, cols, ids = self.manager.take_deltas()
         n = int(rows.shape[0])
         if n == 0:
@@ -48,7 +52,11 @@ class DeviceBlockTables:
         if int(rows.max()) >= max_rows or int(cols.max()) >= width:
             raise ValueError(f"table entry ({int(rows.max())}, {int(cols.max())}) outside the device copy "
                              f"{tuple(self.tensor.shape)}")
-        packed = torch.from_numpy(np.stack((rows * width + cols, ids))).to(self.device)
+        flat = rows * width + cols
+        entries, last = np.unique(flat[::-1], return_index=True)  # of each entry its last write
+        if entries.shape[0] < n:
+            flat, ids, n = entries, ids[::-1][last], int(entries.shape[0])
+        packed = torch.from_numpy(np.stack((flat, ids))).to(self.device)
         self.tensor.view(-1).index_copy_(0, packed[0], packed[1])
         self.uploaded_entries += n
         return n

@@ -205,3 +205,33 @@ def test_device_block_tables_follow_the_allocator_by_deltas():
     assert small.allocate_slots(0, 16 * 5)
     with pytest.raises(ValueError, match="outside the device copy"):
         narrow.sync()
+
+
+def test_a_row_reused_between_syncs_uploads_each_entry_once(monkeypatch):
+    """A request's row is freed and taken by another before the next sync: both writes of an entry are in
+    the deltas, and the device scatter must not be given an index twice (it leaves either value)."""
+    import torch
+
+    from mini_infra_qwen3_amd.worker.block_tables import DeviceBlockTables
+
+    manager = KVCacheManager(block_size=4, num_blocks=64)
+    tables = DeviceBlockTables(manager, max_rows=4, max_blocks=8, device="cpu")
+    assert manager.allocate_slots(0, 9) and manager.allocate_slots(1, 5)
+    manager.free(0)
+    assert manager.allocate_slots(2, 17)  # row of request 0: columns 0-2 written again, 3-4 new
+    manager.free(2)
+    assert manager.allocate_slots(3, 6)   # columns 0-1 a third time
+    scattered = []
+    plain = torch.Tensor.index_copy_
+
+    def index_copy_(self, dim, index, source):
+        scattered.append(index.tolist())
+        return plain(self, dim, index, source)
+
+    monkeypatch.setattr(torch.Tensor, "index_copy_", index_copy_)
+    assert tables.sync() == 7 == tables.uploaded_entries  # 5 entries of the shared row, 2 of request 1
+    assert len(scattered) == 1 and len(set(scattered[0])) == len(scattered[0]) == 7
+    for r in (1, 3):
+        blocks = manager.block_table(r)
+        assert tables.tensor[manager.row_of(r), :len(blocks)].tolist() == blocks
+    assert (tables.tensor[:, :8].numpy() == manager.table_matrix[:4, :8]).all()
