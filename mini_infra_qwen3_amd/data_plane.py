@@ -419,9 +419,10 @@ def paged_decode_attention_fused(
         raise ValueError("pools must be contiguous bf16 with identical shapes")
     head_dim = q_weight.shape[-1]
     batch = q.numel() // q.shape[-1]
-    q2 = q if q.ndim == 2 else q.reshape(batch, -1)
-    k2 = k if k.ndim == 2 else k.reshape(batch, -1)
-    v2 = v if v.ndim == 2 else v.reshape(batch, -1)
+    # Rows in shape are taken as they are; any other layout is brought to one row per token, which a k or v of
+    # another token count does not survive (the head sizes below no longer fit).
+    in_rows = batch > 0 and q.ndim == k.ndim == v.ndim == 2 and k.shape[0] == v.shape[0] == batch
+    q2, k2, v2 = (q, k, v) if in_rows else (q.reshape(batch, -1), k.reshape(batch, -1), v.reshape(batch, -1))
     num_heads, num_kv_heads = q2.shape[1] // head_dim, k2.shape[1] // head_dim
     rows = (batch, head_dim)
     cos2 = cos if cos.shape == rows and cos.is_contiguous() else cos.reshape(rows).contiguous()
