@@ -160,15 +160,16 @@ int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, const void*
  * mi_paged_decode_attention_fused -- mi_qk_norm_rope's decode form (q/k RMSNorm + RoPE of the new
  * tokens, K/V rows into their slots: qwen3.py:182-217 with _apply_paged_kv_pool's append :282-283)
  * followed by mi_paged_decode_attention (qwen3.py:219-292), with the same results bit for bit.
- * Where the per-sequence kernels serve the launch (see mi_paged_decode_attention; projection rows,
- * weights and cos / sin 16-byte aligned) their workgroups rotate their own q heads and append their
- * own K/V head; otherwise it runs the two entry points, rotating q into q_scratch.  Without a
- * workspace they keep the sequences whole.
+ * Launches of at most one (sequence, KV head) per CU with max_blocks <= 512 (projection rows, weights
+ * and cos / sin 16-byte aligned) run the per-sequence kernels of mi_paged_decode_attention, whose
+ * workgroups rotate their own q heads and append their own K/V head; otherwise it runs the two entry
+ * points, rotating q into q_scratch.  Without a workspace they keep the sequences whole.
  * q: [batch] rows of num_heads * 128 (q_row_stride), k / v: rows of num_kv_heads * 128;
  * cos / sin: [batch, 128]; q_scratch: [batch, num_heads, 128] bf16 (always required).
  * The remaining arguments are those of mi_qk_norm_rope and mi_paged_decode_attention.  Each row's
  * slot must lie in one of its own blocks (decode packing puts it at position context - 1): in the
- * per-sequence form only the row's own workgroups are ordered after its append.
+ * per-sequence form only the row's own workgroups are ordered after its append.  Where it runs the two
+ * entry points, every row is.
  */
 int32_t mi_paged_decode_attention_fused(void* out, int64_t out_row_stride, const void* q, int64_t q_row_stride,
                                         const void* k, int64_t k_row_stride, const void* v, int64_t v_row_stride,

@@ -1440,11 +1440,15 @@ extern "C" int32_t mi_paged_decode_attention_fused(
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention_fused: pool too large");
   if (const int32_t rc = check_heads("mi_paged_decode_attention_fused", num_heads, num_kv_heads, head_dim, block_size))
     return rc;
+  // Rows may share blocks (two tokens of one sequence as two rows, one token apart): a launch of more pairs
+  // than CUs appends in a launch of its own, before any row reads.  Up to one pair per CU each row's slot has
+  // to be its own (the entry point's contract), and only its own workgroups put its rows in place.
+  const bool small = static_cast<int64_t>(batch) * num_kv_heads <= device_cus();
   // The prologue of the per-sequence kernel moves 16-byte pieces of the projection rows and tables.
   const bool pieces = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(q_weight) && aligned16(k_weight) &&
                       aligned16(cos) && aligned16(sin) && q_row_stride % 8 == 0 && k_row_stride % 8 == 0 &&
                       v_row_stride % 8 == 0;
-  if (!use_seq_path(batch, max_blocks, num_kv_heads) || max_blocks == 0 || !pieces) {
+  if (!small || !use_seq_path(batch, max_blocks, num_kv_heads) || max_blocks == 0 || !pieces) {
     // The append and q rotation in a launch of their own (large launches; rows of other alignments).
     int32_t rc = mi_qk_norm_rope(q_scratch, nullptr, nullptr, q, q_row_stride, k, k_row_stride, v, v_row_stride,
                                  q_weight, k_weight, cos, sin, batch, num_heads, num_kv_heads, head_dim, eps,

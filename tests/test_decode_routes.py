@@ -1,0 +1,32 @@
+"""Which kernels the decode entry points launch, on the CPU against a stand-in HIP runtime (no GPU): what the
+entry points promise about ordering and about the caller's workspace is a matter of the route."""
+
+import hip_standin
+
+CALLS = """
+P = 4096
+def attention(entry, batch, mb, ws=P, nbytes=1 << 30, heads=16, kv=8):
+    return getattr(lib, entry)(P, heads * 128, P, heads * 128, 128, P, P, 1000, P, max(mb, 1), mb, P, 1, batch, heads, kv, 128, 16,
+                               0.1, *(() if entry.endswith("noalloc") else (ws, nbytes)), None)
+def fused(entry, batch, mb, ws=P, nbytes=1 << 30, offset=0, heads=16, kv=8):
+    return getattr(lib, entry)(P, heads * 128, P + offset, 4096, P, 4096, P, 4096, P, P, P, P, 1e-6, P, 1, P, P, 1000, P,
+                               max(mb, 1), mb, P, 1, batch, heads, kv, 128, 16, 0.1, P, ws, nbytes, None)
+"""
+
+
+def test_a_fused_launch_of_more_pairs_than_cus_appends_before_it_attends():
+    """Rows that read each other's new token (one sequence as two rows) are ordered after the append there."""
+    routes = hip_standin.run(CALLS + """
+result = []
+for batch, kv in [(32, 8), (33, 8), (64, 8), (128, 8), (300, 8), (129, 2), (256, 1), (257, 1)]:
+    for mb in (4, 30, 72, 200, 512):
+        assert fused("mi_paged_decode_attention_fused", batch, mb, heads=2 * kv, kv=kv) == 0
+        result.append((batch * kv, [(l["kernel"], l["args"]) for l in launches()]))
+""")
+    for pairs, calls in routes:
+        names = [name for name, _ in calls]
+        fused = [name for name, args in calls if name in ("paged_decode_stripe_kernel", "paged_decode_parts_kernel") and args[2]]
+        if pairs <= 256:
+            assert names[0] in fused
+        else:
+            assert names[0].startswith("qk_norm_rope") and not fused, (pairs, names)

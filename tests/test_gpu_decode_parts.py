@@ -96,3 +96,22 @@ def test_fused_takes_rows_of_any_alignment(native_lib, device):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("rows,lo,hi", [(20, 40, 1100), (66, 1, 500), (40, 1000, 2500)])
+def test_rows_that_share_a_sequence_see_each_others_token(native_lib, device, rows, lo, hi):
+    """Each sequence as two rows, one token apart (the second row's context holds the first one's token), in
+    launches of more (row, KV head) pairs than CUs: the append comes before every row's attention."""
+    gen = torch.Generator().manual_seed(rows)
+    ctx = torch.randint(lo, hi, (rows,), generator=gen).tolist()
+    ctx = [n for m in ctx for n in (m, m + 1)]
+    kp, vp, tables, qkv, (qw, kw), cos, sin = _case(rows, ctx, max(-(-n // 16) for n in ctx), 2)
+    tables[0::2] = tables[1::2]  # one table per sequence
+    slots = torch.tensor([int(tables[b, (n - 1) // 16]) * 16 + (n - 1) % 16 for b, n in enumerate(ctx)])
+    kp, vp, tables, qkv, qw, kw, cos, sin, slots = [t.to(device) for t in (kp, vp, tables, qkv, qw, kw, cos, sin, slots)]
+    ctx_d = torch.tensor(ctx).to(device)
+    q, k, v = qkv.split((2048, 1024, 1024), dim=1)
+    kp2, vp2 = kp.clone(), vp.clone()
+    q_rot, _, _ = data_plane.qk_norm_rope(q, k, v, qw, kw, cos, sin, 1e-6, slot_mapping=slots, key_pool=kp2, value_pool=vp2)
+    want = data_plane.paged_decode_attention(q_rot.view(2 * rows, 16, 128), kp2, vp2, tables, ctx_d, SCALE)
+    out = data_plane.paged_decode_attention_fused(q, k, v, qw, kw, cos, sin, 1e-6, slots, kp, vp, tables, ctx_d, SCALE)
+    assert torch.equal(kp.view(torch.int16), kp2.view(torch.int16)) and torch.equal(vp.view(torch.int16), vp2.view(torch.int16))
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
