@@ -1353,15 +1353,16 @@ extern "C" int64_t mi_paged_decode_workspace_bytes(int32_t batch, int32_t max_bl
   return streams * 2 * num_heads * (head_dim + 2) * static_cast<int64_t>(sizeof(float));
 }
 
-extern "C" int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, const void* query,
-                                             int64_t query_row_stride, int64_t query_head_stride,
-                                             const void* key_pool, const void* value_pool, int64_t num_blocks,
-                                             const int64_t* block_tables, int64_t block_table_stride,
-                                             int32_t max_blocks, const int64_t* context_lens,
-                                             int64_t context_lens_stride, int32_t batch, int32_t num_heads,
-                                             int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
-                                             void* workspace, int64_t workspace_bytes, void* stream) {
-  using namespace mi;
+namespace mi {
+namespace {
+
+// mi_paged_decode_attention; bare: the launch needs no workspace and takes none.
+int32_t decode_attention(void* out, int64_t out_row_stride, const void* query, int64_t query_row_stride,
+                         int64_t query_head_stride, const void* key_pool, const void* value_pool, int64_t num_blocks,
+                         const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks,
+                         const int64_t* context_lens, int64_t context_lens_stride, int32_t batch, int32_t num_heads,
+                         int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale, void* workspace,
+                         int64_t workspace_bytes, bool bare, void* stream) {
   if (batch < 0 || max_blocks < 0 || num_blocks < 0)
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention: negative size");
   if (batch == 0) return ok();
@@ -1382,10 +1383,10 @@ extern "C" int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, 
 
   const int32_t streams = streams_for(batch, max_blocks, num_kv_heads);
   const int64_t need = mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size);
-  if (max_blocks > 0 && (!workspace || workspace_bytes < need))
+  if (!bare && max_blocks > 0 && (!workspace || workspace_bytes < need))
     return fail(MI_ERR_WORKSPACE, "mi_paged_decode_attention: workspace of %lld bytes needed, got %lld",
                 static_cast<long long>(need), static_cast<long long>(workspace_bytes));
-  if (max_blocks > 0 && !aligned16(workspace))
+  if (!bare && max_blocks > 0 && !aligned16(workspace))
     return fail(MI_ERR_UNSUPPORTED, "mi_paged_decode_attention: workspace must be 16-byte aligned");
   float* ws_acc = static_cast<float*>(workspace);
   float* ws_ml = ws_acc ? ws_acc + static_cast<int64_t>(streams) * 2 * num_heads * kHeadDim : nullptr;
@@ -1412,7 +1413,7 @@ extern "C" int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, 
     a.batch = nb;
     a.max_blocks = max_blocks;
     a.streams = streams;
-    if (seq_path) cut_sequences(a, num_kv_heads, true);
+    if (seq_path) cut_sequences(a, num_kv_heads, !bare);
     a.scale = scale;
     a.ws_acc = ws_acc;
     a.ws_ml = ws_ml;
@@ -1420,6 +1421,23 @@ extern "C" int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, 
     if (rc != MI_OK) return rc;
   }
   return ok();
+}
+
+}  // namespace
+}  // namespace mi
+
+extern "C" int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, const void* query,
+                                             int64_t query_row_stride, int64_t query_head_stride,
+                                             const void* key_pool, const void* value_pool, int64_t num_blocks,
+                                             const int64_t* block_tables, int64_t block_table_stride,
+                                             int32_t max_blocks, const int64_t* context_lens,
+                                             int64_t context_lens_stride, int32_t batch, int32_t num_heads,
+                                             int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
+                                             void* workspace, int64_t workspace_bytes, void* stream) {
+  return mi::decode_attention(out, out_row_stride, query, query_row_stride, query_head_stride, key_pool, value_pool,
+                              num_blocks, block_tables, block_table_stride, max_blocks, context_lens,
+                              context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size, scale,
+                              workspace, workspace_bytes, false, stream);
 }
 
 extern "C" int32_t mi_paged_decode_attention_fused(
@@ -1448,16 +1466,19 @@ extern "C" int32_t mi_paged_decode_attention_fused(
   const bool pieces = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(q_weight) && aligned16(k_weight) &&
                       aligned16(cos) && aligned16(sin) && q_row_stride % 8 == 0 && k_row_stride % 8 == 0 &&
                       v_row_stride % 8 == 0;
-  if (!small || !use_seq_path(batch, max_blocks, num_kv_heads) || max_blocks == 0 || !pieces) {
+  const int64_t need = mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size);
+  const bool room = workspace && workspace_bytes >= need && aligned16(workspace);
+  const bool sequences = small && use_seq_path(batch, max_blocks, num_kv_heads);  // the per-sequence kernels serve it
+  if (!sequences || !pieces) {
     // The append and q rotation in a launch of their own (large launches; rows of other alignments).
     int32_t rc = mi_qk_norm_rope(q_scratch, nullptr, nullptr, q, q_row_stride, k, k_row_stride, v, v_row_stride,
                                  q_weight, k_weight, cos, sin, batch, num_heads, num_kv_heads, head_dim, eps,
                                  slot_mapping, slot_stride, key_pool, value_pool, num_blocks * block_size, stream);
     if (rc != MI_OK) return rc;
-    return mi_paged_decode_attention(out, out_row_stride, q_scratch, static_cast<int64_t>(num_heads) * head_dim,
-                                     head_dim, key_pool, value_pool, num_blocks, block_tables, block_table_stride,
-                                     max_blocks, context_lens, context_lens_stride, batch, num_heads, num_kv_heads,
-                                     head_dim, block_size, scale, workspace, workspace_bytes, stream);
+    return decode_attention(out, out_row_stride, q_scratch, static_cast<int64_t>(num_heads) * head_dim, head_dim, key_pool,
+                            value_pool, num_blocks, block_tables, block_table_stride, max_blocks, context_lens,
+                            context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size, scale, workspace,
+                            workspace_bytes, sequences && !room, stream);
   }
   // The per-sequence kernel with the prologue.  Shape checks as in the two entry points.
   if (!out || !key_pool || !value_pool || !context_lens || !block_tables)
@@ -1480,8 +1501,6 @@ extern "C" int32_t mi_paged_decode_attention_fused(
   a.batch = batch;
   a.max_blocks = max_blocks;
   a.streams = 1;
-  const int64_t need = mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size);
-  const bool room = workspace && workspace_bytes >= need && aligned16(workspace);
   cut_sequences(a, num_kv_heads, room);
   if (room) {
     a.ws_acc = static_cast<float*>(workspace);

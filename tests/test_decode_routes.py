@@ -30,3 +30,20 @@ for batch, kv in [(32, 8), (33, 8), (64, 8), (128, 8), (300, 8), (129, 2), (256,
             assert names[0] in fused
         else:
             assert names[0].startswith("qk_norm_rope") and not fused, (pairs, names)
+
+
+def test_small_fused_launches_need_no_workspace_whatever_the_alignment_of_their_rows():
+    """Up to one (sequence, KV head) pair per CU and 512 table blocks: the sequences stay whole without one."""
+    routes = hip_standin.run(CALLS + """
+result = []
+for batch in (1, 8, 32):
+    for mb in (1, 30, 72, 200, 512):
+        for ws, nbytes in [(None, 0), (P, 16), (P + 8, 1 << 30)]:
+            for offset in (0, 2):
+                rc = fused("mi_paged_decode_attention_fused", batch, mb, ws, nbytes, offset)
+                result.append((offset, rc, [(l["kernel"], l["args"]) for l in launches()]))
+""")
+    for offset, rc, calls in routes:
+        assert rc == 0
+        assert [name for name, _ in calls] == (["qk_norm_rope_kernel"] if offset else []) + ["paged_decode_stripe_kernel"]
+        assert calls[-1][1] == [8, 2, 0 if offset else 1, 8]  # every stripe in one workgroup
