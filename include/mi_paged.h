@@ -138,11 +138,12 @@ int64_t mi_paged_decode_workspace_bytes(int32_t batch, int32_t max_blocks, int32
  * workspace: at least mi_paged_decode_workspace_bytes(...) bytes (may be null when
  *   max_blocks is 0).  The launch's blocks are cut into equal ranges, one per workgroup
  *   (and head group); sequences cut between ranges leave partials that a second, small
- *   launch merges (it also writes the zero rows).  Launches of at most one (sequence, KV
- *   head) per CU, or with batch * max_blocks * num_kv_heads <= 98304, with max_blocks <= 512 run
- *   the per-sequence kernels instead: one launch that leaves the workspace untouched when it
- *   keeps the sequences whole, else one that cuts them and the merge.  The environment variable
- *   MI_DECODE_PATH=stream or =seq forces either form where both apply.
+ *   launch merges (it also writes the zero rows).  Small launches, of at most one (sequence, KV
+ *   head) per CU with max_blocks <= 512, run a single per-sequence kernel instead, which leaves the
+ *   workspace untouched: calls that overlap may share one while all of them are small.  Launches
+ *   with batch * max_blocks * num_kv_heads <= 98304 and max_blocks <= 512 run per-sequence kernels
+ *   that cut the sequences, and the merge.  The environment variable MI_DECODE_PATH=stream or =seq
+ *   forces either form where both apply.
  * Specialised for head_dim 128, block_size 16, num_kv_heads in {1, 2, 4, 8} and GQA groups
  * num_heads / num_kv_heads in {1, 2, 4, 5, 8} (query head h reads KV head h / group, as
  * _repeat_key_value does, src/mini_infra/model/qwen3.py:147-156); other shapes return
@@ -163,7 +164,7 @@ int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, const void*
  * Launches of at most one (sequence, KV head) per CU with max_blocks <= 512 (projection rows, weights
  * and cos / sin 16-byte aligned) run the per-sequence kernels of mi_paged_decode_attention, whose
  * workgroups rotate their own q heads and append their own K/V head; otherwise it runs the two entry
- * points, rotating q into q_scratch.  Without a workspace they keep the sequences whole.
+ * points, rotating q into q_scratch.  Small launches neither need nor touch the workspace.
  * q: [batch] rows of num_heads * 128 (q_row_stride), k / v: rows of num_kv_heads * 128;
  * cos / sin: [batch, 128]; q_scratch: [batch, num_heads, 128] bf16 (always required).
  * The remaining arguments are those of mi_qk_norm_rope and mi_paged_decode_attention.  Each row's
@@ -181,6 +182,35 @@ int32_t mi_paged_decode_attention_fused(void* out, int64_t out_row_stride, const
                                         int64_t context_lens_stride, int32_t batch, int32_t num_heads,
                                         int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
                                         void* q_scratch, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
+ * mi_paged_decode_attention_spread, mi_paged_decode_attention_fused_spread -- the two entry points above for
+ * a workspace that the call has to itself: small launches may cut their sequences too, spreading each over
+ * more workgroups, with partials in the workspace and the merge launch.  Calls that overlap need workspaces
+ * of their own, whatever their size.  Results: tables of up to 128 blocks the same bits as the entry points
+ * above, longer ones summed in another order; the two agree bit for bit with each other.
+ * mi_paged_decode_spread_bytes: the workspace with which a small launch cuts its sequences; 0 where it does
+ * not, or where the launch is not small (the entry points above are then the same).
+ */
+int32_t mi_paged_decode_attention_spread(void* out, int64_t out_row_stride, const void* query,
+                                         int64_t query_row_stride, int64_t query_head_stride,
+                                         const void* key_pool, const void* value_pool, int64_t num_blocks,
+                                         const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks,
+                                         const int64_t* context_lens, int64_t context_lens_stride, int32_t batch,
+                                         int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                         float scale, void* workspace, int64_t workspace_bytes, void* stream);
+int32_t mi_paged_decode_attention_fused_spread(void* out, int64_t out_row_stride, const void* q, int64_t q_row_stride,
+                                               const void* k, int64_t k_row_stride, const void* v, int64_t v_row_stride,
+                                               const void* q_weight, const void* k_weight, const void* cos,
+                                               const void* sin, float eps, const int64_t* slot_mapping,
+                                               int64_t slot_stride, void* key_pool, void* value_pool, int64_t num_blocks,
+                                               const int64_t* block_tables, int64_t block_table_stride,
+                                               int32_t max_blocks, const int64_t* context_lens,
+                                               int64_t context_lens_stride, int32_t batch, int32_t num_heads,
+                                               int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
+                                               void* q_scratch, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t mi_paged_decode_spread_bytes(int32_t batch, int32_t max_blocks, int32_t num_heads, int32_t num_kv_heads,
+                                     int32_t head_dim, int32_t block_size);
 
 /*
  * mi_paged_decode_attention_noalloc -- mi_paged_decode_attention without a workspace argument: a

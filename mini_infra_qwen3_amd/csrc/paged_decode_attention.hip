@@ -1356,13 +1356,24 @@ extern "C" int64_t mi_paged_decode_workspace_bytes(int32_t batch, int32_t max_bl
 namespace mi {
 namespace {
 
-// mi_paged_decode_attention; bare: the launch needs no workspace and takes none.
+// Whose workspace a launch has.  kShared: the caller's, which other calls may use at the same time while all of
+// them are small (at most one (sequence, KV head) pair per CU), so small launches leave it untouched.
+// kOwn: this call's alone, so small launches may spread their sequences through it.  kNone: the launch is
+// small, needs none and takes none.
+enum class Workspace { kShared, kOwn, kNone };
+
+// Small launches, to which the promise of an untouched workspace applies.
+bool is_small(int32_t batch, int32_t num_kv_heads) {
+  return static_cast<int64_t>(batch) * num_kv_heads <= device_cus();
+}
+
+// mi_paged_decode_attention.
 int32_t decode_attention(void* out, int64_t out_row_stride, const void* query, int64_t query_row_stride,
                          int64_t query_head_stride, const void* key_pool, const void* value_pool, int64_t num_blocks,
                          const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks,
                          const int64_t* context_lens, int64_t context_lens_stride, int32_t batch, int32_t num_heads,
                          int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale, void* workspace,
-                         int64_t workspace_bytes, bool bare, void* stream) {
+                         int64_t workspace_bytes, Workspace use, void* stream) {
   if (batch < 0 || max_blocks < 0 || num_blocks < 0)
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention: negative size");
   if (batch == 0) return ok();
@@ -1383,16 +1394,17 @@ int32_t decode_attention(void* out, int64_t out_row_stride, const void* query, i
 
   const int32_t streams = streams_for(batch, max_blocks, num_kv_heads);
   const int64_t need = mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size);
-  if (!bare && max_blocks > 0 && (!workspace || workspace_bytes < need))
+  if (use != Workspace::kNone && max_blocks > 0 && (!workspace || workspace_bytes < need))
     return fail(MI_ERR_WORKSPACE, "mi_paged_decode_attention: workspace of %lld bytes needed, got %lld",
                 static_cast<long long>(need), static_cast<long long>(workspace_bytes));
-  if (!bare && max_blocks > 0 && !aligned16(workspace))
+  if (use != Workspace::kNone && max_blocks > 0 && !aligned16(workspace))
     return fail(MI_ERR_UNSUPPORTED, "mi_paged_decode_attention: workspace must be 16-byte aligned");
   float* ws_acc = static_cast<float*>(workspace);
   float* ws_ml = ws_acc ? ws_acc + static_cast<int64_t>(streams) * 2 * num_heads * kHeadDim : nullptr;
 
   hipStream_t s = as_stream(stream);
   const bool seq_path = use_seq_path(batch, max_blocks, num_kv_heads);
+  const bool cut = use == Workspace::kOwn || !is_small(batch, num_kv_heads);
   // Sequences go in slices of at most kMaxBatchPerLaunch (the per-workgroup prefix sum lives in
   // LDS); the slices reuse the workspace one after the other on the stream.
   for (int32_t b0 = 0; b0 < batch; b0 += kMaxBatchPerLaunch) {
@@ -1413,7 +1425,7 @@ int32_t decode_attention(void* out, int64_t out_row_stride, const void* query, i
     a.batch = nb;
     a.max_blocks = max_blocks;
     a.streams = streams;
-    if (seq_path) cut_sequences(a, num_kv_heads, !bare);
+    if (seq_path) cut_sequences(a, num_kv_heads, cut);
     a.scale = scale;
     a.ws_acc = ws_acc;
     a.ws_ml = ws_ml;
@@ -1437,17 +1449,47 @@ extern "C" int32_t mi_paged_decode_attention(void* out, int64_t out_row_stride, 
   return mi::decode_attention(out, out_row_stride, query, query_row_stride, query_head_stride, key_pool, value_pool,
                               num_blocks, block_tables, block_table_stride, max_blocks, context_lens,
                               context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size, scale,
-                              workspace, workspace_bytes, false, stream);
+                              workspace, workspace_bytes, mi::Workspace::kShared, stream);
 }
 
-extern "C" int32_t mi_paged_decode_attention_fused(
+extern "C" int32_t mi_paged_decode_attention_spread(void* out, int64_t out_row_stride, const void* query,
+                                                    int64_t query_row_stride, int64_t query_head_stride,
+                                                    const void* key_pool, const void* value_pool, int64_t num_blocks,
+                                                    const int64_t* block_tables, int64_t block_table_stride,
+                                                    int32_t max_blocks, const int64_t* context_lens,
+                                                    int64_t context_lens_stride, int32_t batch, int32_t num_heads,
+                                                    int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
+                                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  return mi::decode_attention(out, out_row_stride, query, query_row_stride, query_head_stride, key_pool, value_pool,
+                              num_blocks, block_tables, block_table_stride, max_blocks, context_lens,
+                              context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size, scale,
+                              workspace, workspace_bytes, mi::Workspace::kOwn, stream);
+}
+
+extern "C" int64_t mi_paged_decode_spread_bytes(int32_t batch, int32_t max_blocks, int32_t num_heads,
+                                                int32_t num_kv_heads, int32_t head_dim, int32_t block_size) {
+  using namespace mi;
+  const int64_t need = mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size);
+  if (need == 0 || !is_small(batch, num_kv_heads) || !use_seq_path(batch, max_blocks, num_kv_heads)) return 0;
+  DecodeArgs a{};
+  a.batch = batch;
+  a.max_blocks = max_blocks;
+  cut_sequences(a, num_kv_heads, true);
+  return a.splits > 1 ? need : 0;
+}
+
+namespace mi {
+namespace {
+
+// mi_paged_decode_attention_fused.
+int32_t decode_attention_fused(
     void* out, int64_t out_row_stride, const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride,
     const void* v, int64_t v_row_stride, const void* q_weight, const void* k_weight, const void* cos, const void* sin,
     float eps, const int64_t* slot_mapping, int64_t slot_stride, void* key_pool, void* value_pool, int64_t num_blocks,
     const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks, const int64_t* context_lens,
     int64_t context_lens_stride, int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
-    int32_t block_size, float scale, void* q_scratch, void* workspace, int64_t workspace_bytes, void* stream) {
-  using namespace mi;
+    int32_t block_size, float scale, void* q_scratch, void* workspace, int64_t workspace_bytes, Workspace use,
+    void* stream) {
   if (batch < 0 || max_blocks < 0 || num_blocks < 0)
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention_fused: negative size");
   if (batch == 0) return ok();
@@ -1461,13 +1503,14 @@ extern "C" int32_t mi_paged_decode_attention_fused(
   // Rows may share blocks (two tokens of one sequence as two rows, one token apart): a launch of more pairs
   // than CUs appends in a launch of its own, before any row reads.  Up to one pair per CU each row's slot has
   // to be its own (the entry point's contract), and only its own workgroups put its rows in place.
-  const bool small = static_cast<int64_t>(batch) * num_kv_heads <= device_cus();
+  const bool small = is_small(batch, num_kv_heads);
   // The prologue of the per-sequence kernel moves 16-byte pieces of the projection rows and tables.
   const bool pieces = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(q_weight) && aligned16(k_weight) &&
                       aligned16(cos) && aligned16(sin) && q_row_stride % 8 == 0 && k_row_stride % 8 == 0 &&
                       v_row_stride % 8 == 0;
   const int64_t need = mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size);
-  const bool room = workspace && workspace_bytes >= need && aligned16(workspace);
+  // Where a small launch may cut its sequences; without that they stay whole.
+  const bool room = use == Workspace::kOwn && workspace && workspace_bytes >= need && aligned16(workspace);
   const bool sequences = small && use_seq_path(batch, max_blocks, num_kv_heads);  // the per-sequence kernels serve it
   if (!sequences || !pieces) {
     // The append and q rotation in a launch of their own (large launches; rows of other alignments).
@@ -1478,7 +1521,7 @@ extern "C" int32_t mi_paged_decode_attention_fused(
     return decode_attention(out, out_row_stride, q_scratch, static_cast<int64_t>(num_heads) * head_dim, head_dim, key_pool,
                             value_pool, num_blocks, block_tables, block_table_stride, max_blocks, context_lens,
                             context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size, scale, workspace,
-                            workspace_bytes, sequences && !room, stream);
+                            workspace_bytes, sequences && !room ? Workspace::kNone : use, stream);
   }
   // The per-sequence kernel with the prologue.  Shape checks as in the two entry points.
   if (!out || !key_pool || !value_pool || !context_lens || !block_tables)
@@ -1522,6 +1565,37 @@ extern "C" int32_t mi_paged_decode_attention_fused(
   a.num_slots = num_blocks * kBlockSize;
   a.eps = eps;
   return launch_for_heads<true>(a, num_heads, num_kv_heads, true, as_stream(stream));
+}
+
+}  // namespace
+}  // namespace mi
+
+extern "C" int32_t mi_paged_decode_attention_fused(
+    void* out, int64_t out_row_stride, const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride,
+    const void* v, int64_t v_row_stride, const void* q_weight, const void* k_weight, const void* cos, const void* sin,
+    float eps, const int64_t* slot_mapping, int64_t slot_stride, void* key_pool, void* value_pool, int64_t num_blocks,
+    const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks, const int64_t* context_lens,
+    int64_t context_lens_stride, int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+    int32_t block_size, float scale, void* q_scratch, void* workspace, int64_t workspace_bytes, void* stream) {
+  return mi::decode_attention_fused(
+      out, out_row_stride, q, q_row_stride, k, k_row_stride, v, v_row_stride, q_weight, k_weight, cos, sin, eps,
+      slot_mapping, slot_stride, key_pool, value_pool, num_blocks, block_tables, block_table_stride, max_blocks,
+      context_lens, context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size, scale, q_scratch,
+      workspace, workspace_bytes, mi::Workspace::kShared, stream);
+}
+
+extern "C" int32_t mi_paged_decode_attention_fused_spread(
+    void* out, int64_t out_row_stride, const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride,
+    const void* v, int64_t v_row_stride, const void* q_weight, const void* k_weight, const void* cos, const void* sin,
+    float eps, const int64_t* slot_mapping, int64_t slot_stride, void* key_pool, void* value_pool, int64_t num_blocks,
+    const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks, const int64_t* context_lens,
+    int64_t context_lens_stride, int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+    int32_t block_size, float scale, void* q_scratch, void* workspace, int64_t workspace_bytes, void* stream) {
+  return mi::decode_attention_fused(
+      out, out_row_stride, q, q_row_stride, k, k_row_stride, v, v_row_stride, q_weight, k_weight, cos, sin, eps,
+      slot_mapping, slot_stride, key_pool, value_pool, num_blocks, block_tables, block_table_stride, max_blocks,
+      context_lens, context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size, scale, q_scratch,
+      workspace, workspace_bytes, mi::Workspace::kOwn, stream);
 }
 
 // ---- The no-allocation variant.  The stream kernel's cut-sequence partials go to `scratch`, a

@@ -264,6 +264,24 @@ def paged_decode_workspace_bytes(batch: int, max_blocks: int, num_heads: int, he
                                                                         block_size))
 
 
+def _decode_workspace(lib, workspace: torch.Tensor | None, batch: int, max_blocks: int, num_heads: int, num_kv_heads: int,
+                      head_dim: int, block_size: int, device: torch.device) -> tuple[bool, torch.Tensor | None]:
+    """(spread, workspace) of a bandwidth decode launch.  A small launch that can cut its sequences gets a
+    buffer of this call's own (``spread``): the caller's may be in use by another small launch on another
+    stream.  Others get ``workspace``, or a new buffer when it is missing or too small; None when the
+    launch needs none.  The caller keeps the buffer until the launch is enqueued."""
+    need = lib.mi_paged_decode_spread_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size)
+    if need > 0:
+        return True, torch.empty(need, dtype=torch.uint8, device=device)
+    need = lib.mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size)
+    if need <= 0:
+        return False, None
+    if workspace is None or workspace.numel() * workspace.element_size() < need:
+        return False, torch.empty(need, dtype=torch.uint8, device=device)
+    _require_gpu("workspace", workspace, device)
+    return False, workspace
+
+
 def paged_decode_exact_workspace_bytes(batch: int, max_blocks: int, num_heads: int, num_kv_heads: int,
                                        block_size: int = KERNEL_BLOCK_SIZE) -> int:
     """Workspace of the reference-numerics decode's split form (0: the launch runs unsplit)."""
@@ -300,7 +318,8 @@ def paged_decode_attention(
     contiguous, block_size 16 or a multiple of it; block_tables ``[B, max_blocks]`` int64
     (null-padded); context_lens ``[B]`` int64 (includes the new token).  Returns ``out``
     ``[B, H * D]`` bf16.  ``workspace`` (optional, uint8, reused across calls) holds the
-    split-context partials; it is allocated here when missing or too small.  ``exact``: the
+    split-context partials; it is allocated here when missing or too small, and small launches (one
+    (sequence, KV head) pair per CU at most) leave the caller's untouched.  ``exact``: the
     reference-numerics kernel (``mi_paged_decode_attention_exact``: the reference's rounding
     points with exact sums), whose split form for small batches uses the workspace the same way.
     """
@@ -347,14 +366,9 @@ def paged_decode_attention(
             head_dim, block_size, float(scale), ws_ptr, ws_bytes, stream)
         _native.check(rc, "mi_paged_decode_attention_exact")
         return out
-    need = paged_decode_workspace_bytes(batch, max_blocks, num_heads, head_dim, block_size, num_kv_heads)
-    ws_ptr, ws_bytes = None, 0
-    if need > 0:
-        if workspace is None or workspace.numel() * workspace.element_size() < need:
-            workspace = torch.empty(need, dtype=torch.uint8, device=device)
-        _require_gpu("workspace", workspace, device)
-        ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    rc = lib.mi_paged_decode_attention(
+    spread, ws = _decode_workspace(lib, workspace, batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size, device)
+    ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel() * ws.element_size())
+    rc = (lib.mi_paged_decode_attention_spread if spread else lib.mi_paged_decode_attention)(
         out.data_ptr(), out.stride(0),
         query.data_ptr(), query.stride(0), query.stride(1),
         key_pool.data_ptr(), value_pool.data_ptr(), num_blocks,
@@ -458,14 +472,10 @@ def paged_decode_attention_fused(
         _native.check(rc, "mi_paged_decode_attention_exact")
         return out
     q_scratch = torch.empty((batch, num_heads, head_dim), dtype=torch.bfloat16, device=device)
-    need = paged_decode_workspace_bytes(batch, max_blocks, num_heads, head_dim, block_size, num_kv_heads)
-    ws_ptr, ws_bytes = None, 0
-    if need > 0:
-        if workspace is None or workspace.numel() * workspace.element_size() < need:
-            workspace = torch.empty(need, dtype=torch.uint8, device=device)
-        _require_gpu("workspace", workspace, device)
-        ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    rc = _native.load().mi_paged_decode_attention_fused(
+    lib = _native.load()
+    spread, ws = _decode_workspace(lib, workspace, batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size, device)
+    ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel() * ws.element_size())
+    rc = (lib.mi_paged_decode_attention_fused_spread if spread else lib.mi_paged_decode_attention_fused)(
         out.data_ptr(), out.stride(0), q2.data_ptr(), q2.stride(0), k2.data_ptr(), k2.stride(0), v2.data_ptr(),
         v2.stride(0), q_weight.data_ptr(), k_weight.data_ptr(), cos2.data_ptr(), sin2.data_ptr(), float(eps),
         slot_mapping.data_ptr(), slot_mapping.stride(0) if batch > 1 else 1, key_pool.data_ptr(), value_pool.data_ptr(),

@@ -47,3 +47,31 @@ for batch in (1, 8, 32):
         assert rc == 0
         assert [name for name, _ in calls] == (["qk_norm_rope_kernel"] if offset else []) + ["paged_decode_stripe_kernel"]
         assert calls[-1][1] == [8, 2, 0 if offset else 1, 8]  # every stripe in one workgroup
+
+
+def test_small_launches_leave_the_callers_workspace_untouched():
+    """Calls that overlap on two streams may share one workspace while all of them are small: no partials, no
+    merge.  The spread entry points cut the sequences (their workspace is the call's own), and
+    mi_paged_decode_spread_bytes says where."""
+    routes = hip_standin.run(CALLS + """
+result = []
+for batch, kv in [(1, 8), (8, 8), (32, 8), (128, 2), (256, 1), (33, 8), (96, 8)]:
+    for mb in (1, 30, 64, 128, 129, 512, 513):
+        for fn, entry in ((attention, "mi_paged_decode_attention"), (fused, "mi_paged_decode_attention_fused"),
+                          (attention, "mi_paged_decode_attention_noalloc"), (attention, "mi_paged_decode_attention_spread"),
+                          (fused, "mi_paged_decode_attention_fused_spread")):
+            rc = fn(entry, batch, mb, heads=2 * kv, kv=kv)
+            names = [l["kernel"] for l in launches()]
+            result.append((entry, batch * kv, mb, rc, names, lib.mi_paged_decode_spread_bytes(batch, mb, 2 * kv, kv, 128, 16),
+                           lib.mi_paged_decode_workspace_bytes(batch, mb, 2 * kv, kv, 128, 16)))
+""")
+    for entry, pairs, mb, rc, names, spread, need in routes:
+        assert rc == 0 or (rc == -3 and entry.endswith("noalloc") and need > 8 << 20)
+        small = pairs <= 256 and mb <= 512
+        assert spread in ((0, need) if small else (0,))
+        if small and entry.endswith("spread"):
+            merged = ["paged_decode_stripe_merge_kernel"] if mb <= 128 else ["paged_decode_merge_kernel"]
+            assert names[1:] == (merged if spread else [])
+            assert (mb >= 129) <= (spread > 0)
+        elif small:
+            assert names == ["paged_decode_stripe_kernel"]

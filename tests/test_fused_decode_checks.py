@@ -20,7 +20,7 @@ class Recorder:
     def __getattr__(self, name):
         def entry(*args):
             self.calls.append(name)
-            return 4096 if name.endswith("_bytes") else _native.MI_OK
+            return 4096 if name.endswith("workspace_bytes") else _native.MI_OK
 
         return entry
 

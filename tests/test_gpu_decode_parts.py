@@ -115,3 +115,25 @@ def test_rows_that_share_a_sequence_see_each_others_token(native_lib, device, ro
     out = data_plane.paged_decode_attention_fused(q, k, v, qw, kw, cos, sin, 1e-6, slots, kp, vp, tables, ctx_d, SCALE)
     assert torch.equal(kp.view(torch.int16), kp2.view(torch.int16)) and torch.equal(vp.view(torch.int16), vp2.view(torch.int16))
     assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("width,ctx", [(30, [480, 3, 0]), (72, [1150, 17, 600, 1]), (200, [3200, 129]), (512, [8192, 1, 0, 700])])
+def test_small_launches_leave_the_callers_workspace_untouched(native_lib, device, width, ctx):
+    """Through the C ABI with a filled workspace, and through the Python layer with the same one; spread, tables
+    of up to 128 blocks have the same bits, longer ones agree within the tolerance."""
+    kp, vp, tables, qkv, _, _, _ = _case(width, ctx, width, 2)
+    q = qkv[:, :2048].reshape(len(ctx), 16, 128).contiguous().to(device)
+    kp, vp, tables, ctx_d = kp.to(device), vp.to(device), tables.to(device), torch.tensor(ctx).to(device)
+    need = native_lib.mi_paged_decode_workspace_bytes(len(ctx), width, 16, 8, 128, 16)
+    ws = torch.full((need,), 171, dtype=torch.uint8, device=device)
+    out = torch.empty((len(ctx), 2048), dtype=torch.bfloat16, device=device)
+    rc = native_lib.mi_paged_decode_attention(
+        out.data_ptr(), 2048, q.data_ptr(), 2048, 128, kp.data_ptr(), vp.data_ptr(), kp.shape[0], tables.data_ptr(), width,
+        width, ctx_d.data_ptr(), 1, len(ctx), 16, 8, 128, 16, SCALE, ws.data_ptr(), need,
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    spread = data_plane.paged_decode_attention(q, kp, vp, tables, ctx_d, SCALE, workspace=ws)
+    assert (ws == 171).all()
+    if width <= 128:
+        assert torch.equal(out.view(torch.int16), spread.view(torch.int16))
+    assert (out.float() - spread.float()).abs().max().item() <= TOL
