@@ -75,3 +75,21 @@ for batch, kv in [(1, 8), (8, 8), (32, 8), (128, 2), (256, 1), (33, 8), (96, 8)]
             assert (mb >= 129) <= (spread > 0)
         elif small:
             assert names == ["paged_decode_stripe_kernel"]
+
+
+def test_many_sequences_are_merged_by_one_workgroup_each():
+    """The stream form's merge: a workgroup per sequence where a sequence spans under two ranges, else one per
+    (sequence, KV head)."""
+    routes = hip_standin.run(CALLS + """
+result = []
+for batch, kv in [(64, 8), (128, 8), (129, 8), (512, 8), (4096, 8), (512, 2), (513, 2), (4500, 8)]:
+    assert attention("mi_paged_decode_attention", batch, 600, heads=2 * kv, kv=kv) == 0
+    result.append((batch, kv, [(l["kernel"], l["args"], l["grid"], l["block"]) for l in launches()]))
+""")
+    for batch, kv, calls in routes:
+        for at, rows in enumerate([min(batch, 4096), batch - 4096] if batch > 4096 else [batch]):
+            name, args, grid, block = calls[2 * at + 1]
+            if (1024 if kv == 2 else 256) < 2 * rows:
+                assert (name, args, grid, block) == ("paged_decode_merge_rows_kernel", [2 * kv], [rows, 1, 1], 256)
+            else:
+                assert (name, args, grid) == ("paged_decode_merge_kernel", [kv, 2, 0], [rows, kv, 1])

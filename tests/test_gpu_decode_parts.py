@@ -137,3 +137,26 @@ def test_small_launches_leave_the_callers_workspace_untouched(native_lib, device
     if width <= 128:
         assert torch.equal(out.view(torch.int16), spread.view(torch.int16))
     assert (out.float() - spread.float()).abs().max().item() <= TOL
+
+
+@pytest.mark.parametrize("batch,kv_heads,group", [(129, 8, 1), (300, 8, 2), (200, 8, 8), (520, 2, 2), (1025, 1, 5)])
+def test_merge_of_many_sequences(native_lib, device, monkeypatch, batch, kv_heads, group):
+    """More sequences than half the block ranges (a merge workgroup per sequence): empty, one-token and
+    two-block contexts among longer ones, one cut into many ranges.  Against the per-sequence kernels, which
+    other tests hold against the oracle."""
+    gen = torch.Generator(device=device).manual_seed(batch)
+    ctx = torch.randint(0, 300, (batch,), generator=gen, device=device)
+    ctx[::7] = torch.tensor([0, 1, 16, 17, 31, 32, 33], device=device).repeat(-(-len(ctx[::7]) // 7))[:len(ctx[::7])]
+    ctx[batch // 2] = 8000
+    width = 512
+    num_blocks = 3000
+    tables = torch.randint(1, num_blocks, (batch, width), generator=gen, device=device)
+    kp, vp = (torch.randn(num_blocks, 16, kv_heads, 128, generator=gen, device=device).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(batch, group * kv_heads, 128, generator=gen, device=device).to(torch.bfloat16)
+    outs = []
+    for path in ("stream", "seq"):
+        monkeypatch.setenv("MI_DECODE_PATH", path)
+        out = torch.full((batch, group * kv_heads * 128), float("nan"), dtype=torch.bfloat16, device=device)
+        outs.append(data_plane.paged_decode_attention(q, kp, vp, tables, ctx, SCALE, out=out).float())
+    assert (outs[0] - outs[1]).abs().max().item() <= TOL  # NaN (a row not written) fails too
+    assert not outs[0][ctx == 0].any()
