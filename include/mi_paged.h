@@ -141,9 +141,9 @@ int64_t mi_paged_decode_workspace_bytes(int32_t batch, int32_t max_blocks, int32
  *   launch merges (it also writes the zero rows).  Small launches, of at most one (sequence, KV
  *   head) per CU with max_blocks <= 512, run a single per-sequence kernel instead, which leaves the
  *   workspace untouched: calls that overlap may share one while all of them are small.  Launches
- *   with batch * max_blocks * num_kv_heads <= 98304 and max_blocks <= 512 run per-sequence kernels
- *   that cut the sequences, and the merge.  The environment variable MI_DECODE_PATH=stream or =seq
- *   forces either form where both apply.
+ *   of fewer than six (sequence, KV head) pairs per CU with batch * max_blocks * num_kv_heads <=
+ *   98304 and max_blocks <= 512 run per-sequence kernels that may cut the sequences, and the merge.
+ *   The environment variable MI_DECODE_PATH=stream or =seq forces either form where both apply.
  * Specialised for head_dim 128, block_size 16, num_kv_heads in {1, 2, 4, 8} and GQA groups
  * num_heads / num_kv_heads in {1, 2, 4, 5, 8} (query head h reads KV head h / group, as
  * _repeat_key_value does, src/mini_infra/model/qwen3.py:147-156); other shapes return

@@ -1329,13 +1329,14 @@ void cut_sequences(DecodeArgs& a, int32_t num_kv_heads, bool has_workspace) {
   a.splits = (a.max_blocks + a.part_blocks - 1) / a.part_blocks;
 }
 
-// The per-sequence kernel serves launches of at most one (sequence, KV head) pair per CU, and larger
-// ones while their tables hold no more than kSeqWork (block, KV head) pairs; beyond that the stream
-// kernel's equal ranges win.  Measured, us per layer with the prologue, per-sequence / stream: 40 and 64
-// sequences U[32, 1150] 25.4 / 29.9 and 39.2 / 43.6, 128 of U[32, 400] 28.1 / 35.5, 128 of U[32, 1150]
-// (73,728 pairs) 56-58 / 62; 40 lognormal to 8192 with 5 heads per KV head (163,840 pairs) 112 / 94, 100
-// of them with 2 264 / 216.  MI_DECODE_PATH=stream or =seq (environment) forces one kernel where both
-// apply.
+// The per-sequence kernels serve launches of at most one (sequence, KV head) pair per CU, and larger ones while
+// each sequence can be cut in two (fewer than kPartGroupsPerCu pairs per CU) and their tables hold no more
+// than kSeqWork (block, KV head) pairs; beyond that the stream kernel's equal ranges win.  Measured, us per
+// layer without the prologue, per-sequence / stream: 64 sequences of U[1, 64] 7.4 / 21.7, of U[1, 700] 25.5 / 26.2,
+// 128 of U[1, 300] 22.4 / 25.1, 190 of U[1, 700] 58 / 62; uncut, with eight stripes in a workgroup: 256 of U[1, 420]
+// 53 / 50.5, 512 of U[32, 300] 86 / 74, 1024 of U[32, 190] 131 / 103, 4096 of U[1, 48] 342 / 163; 40 lognormal to 8192
+// with 5 heads per KV head (163,840 pairs) 112 / 94, 100 of them with 2 264 / 216.  MI_DECODE_PATH=stream or
+// =seq (environment) forces one form where both apply.
 constexpr int64_t kSeqWork = 98304;
 bool use_seq_path(int32_t batch, int32_t max_blocks, int32_t num_kv_heads) {
   if (max_blocks <= 0 || max_blocks > kSeqMaxBlocks) return false;
@@ -1343,7 +1344,8 @@ bool use_seq_path(int32_t batch, int32_t max_blocks, int32_t num_kv_heads) {
   if (forced && strcmp(forced, "stream") == 0) return false;
   if (forced && strcmp(forced, "seq") == 0) return true;
   const int64_t pairs = static_cast<int64_t>(batch) * num_kv_heads;
-  return pairs <= device_cus() || pairs * max_blocks <= kSeqWork;
+  const int64_t cus = device_cus();
+  return pairs <= cus || (pairs < cus * kPartGroupsPerCu && pairs * max_blocks <= kSeqWork);
 }
 
 template <int kKvHeads, int kG, bool kFused>

@@ -93,3 +93,18 @@ for batch, kv in [(64, 8), (128, 8), (129, 8), (512, 8), (4096, 8), (512, 2), (5
                 assert (name, args, grid, block) == ("paged_decode_merge_rows_kernel", [2 * kv], [rows, 1, 1], 256)
             else:
                 assert (name, args, grid) == ("paged_decode_merge_kernel", [kv, 2, 0], [rows, kv, 1])
+
+
+def test_sequences_of_large_launches_are_cut_or_streamed():
+    """Past one pair per CU the per-sequence kernels take a launch only where they can cut its sequences in two;
+    the workgroup of eight stripes per (sequence, KV head) does not serve thousands of short sequences."""
+    routes = hip_standin.run(CALLS + """
+result = []
+for batch, kv in [(33, 8), (64, 8), (191, 8), (192, 8), (256, 8), (512, 8), (4096, 8), (767, 2), (768, 2), (1535, 1), (1536, 1)]:
+    for mb in (1, 8, 19, 44, 72, 300):
+        assert attention("mi_paged_decode_attention", batch, mb, heads=2 * kv, kv=kv) == 0
+        result.append((batch * kv, mb, launches()[0]["kernel"]))
+""")
+    for pairs, mb, kernel in routes:
+        per_sequence = pairs < 6 * 256 and pairs * mb <= 98304
+        assert (kernel != "paged_decode_kernel") == per_sequence, (pairs, mb, kernel)
