@@ -766,35 +766,61 @@ PrefillArgs rows_args(int32_t batch, int32_t padded_len, int32_t num_heads, int3
 
 enum class Form { kWide, kHalf, kHalfSplit, kNarrow };
 
+// Whether a row's history table fits beside `tile_bytes` of K/V tiles in LDS.
+bool table_fits(int tile_bytes, int32_t max_history_blocks) {
+  return tile_bytes + static_cast<int64_t>(sizeof(int)) * max_history_blocks <= kLdsPerGroup;
+}
+
 #ifndef MI_PREFILL_FORM
 #define MI_PREFILL_FORM -1
 #endif
-#ifndef MI_PREFILL_T1
-#define MI_PREFILL_T1 128
-#define MI_PREFILL_T2 248
-#define MI_PREFILL_T3 512
-#endif
-// Which workgroup shape takes a launch of `batch` chunk rows: by the workgroups it would have in the wide
-// one (80 of them occupied 80 CUs for 11 serial key tiles of 2 us).  Measured, us, wide / half / half split /
-// narrow (16 query, 8 KV heads):
-//   1 x 60 behind 4000 tokens           8 workgroups   143 / 111 /  90 /  65
-//   1 x 1000                           64               44 /  35 /  29 /  22
-//   2 x 250-700                        80               27 /  23 /  21 /  16
-//   1 x 2048 behind 2000              128              114 /  86 /  72 /  82
-//   2 x 700-1400                      160               59 /  46 /  37 /  40
-//   3 x 1200                          240               51 /  50 /  48 /  53
-//   2 x 2048 behind 3000              256              144 / 154 / 153 / 214
-//   3 x 1024-2048, none / 5000        360          72 / 327 | 63 / 282 | 72 / 290 | 82 / 346
-//   4 x 2048 behind 10240             512              658 / 679 / 762 / 1135
+// Which workgroup shape takes a launch of `batch` chunk rows: by the workgroups it would have in the narrow and the
+// wide shape, and by whether its query tiles see about as many keys each (history tables next to the
+// chunk's length) or the later ones more, so that light tiles fill the last round of a finer cut.
+// Measured, us, wide / half / half split / narrow (16 query, 8 KV heads; rows x queries behind tokens of
+// history, and the workgroups that decide):
+//   narrow: one round of its workgroups (cus; 11/8 of that without much history)
+//     1 x 60 behind 4000     16 narrow       147 / 115 /  85 /  57
+//     3 x 300               240               20 /  16 /  17 /  13
+//     1 x 1000              256               46 /  35 /  29 /  22
+//     2 x 700               352               33 /  27 /  24 /  19
+//   half: short rows without history
+//     15 x 128              120 wide          17 /  12 /  14 /  17
+//     64 x 128              512               38 /  31 /  47 /  58
+//     40 x 256              640               54 /  40 /  62 /  79
+//   half split: up to half of cus wide workgroups, one round of its own
+//     3 x 450                96               28 /  21 /  19 /  20
+//     16 x 128 behind 1000  128               49 /  37 /  35 /  44
+//     1 x 2048 behind 2000  128              127 /  94 /  83 /  86
+//   up to cus: wide with history, else half split for long rows, half for shorter ones
+//     20 x 128 behind 2000  160               81 /  83 /  96 /  99
+//     2 x 1792 behind 4000  224              179 / 186 / 186 / 233
+//     3 x 700               144               36 /  30 /  26 /  30
+//     1 x 4096              256              128 / 103 /  94 / 117
+//     5 x 640               200               34 /  31 /  33 /  38
+//   half: a second wide round at most 9/16 full (400)
+//     3 x 1408 behind 6000  264              370 / 320 / 332 / 380
+//     3 x 2048              384               88 /  81 /  97 / 106
+//     25 x 256 behind 2000  400              165 / 162 / 194 / 235
+//   wide beyond
+//     4 x 1664              416               66 /  82 /  81 / 105
+//     4 x 1900 behind 1000  480              142 / 163 / 165 / 213
+//     4 x 2048 behind 10240 512              729 / 750 / 801 / 1025
 Form form_for(int32_t batch, int32_t padded_len, int32_t num_heads, int32_t num_kv_heads, int32_t max_history_blocks) {
   if (MI_PREFILL_FORM >= 0) return static_cast<Form>(MI_PREFILL_FORM);
+  static_assert(Narrow::kLdsBytes == HalfSplit::kLdsBytes, "one limit");
+  const int64_t cus = device_cus();
   const int64_t pairs = static_cast<int64_t>(num_kv_heads) * ((num_heads / num_kv_heads + kGroup - 1) / kGroup) * batch;
   const int64_t wide = pairs * ((padded_len + Wide::kQTile - 1) / Wide::kQTile);
-  if (wide >= MI_PREFILL_T3 || (wide >= MI_PREFILL_T2 && wide <= 256)) return Form::kWide;
-  static_assert(Narrow::kLdsBytes == HalfSplit::kLdsBytes, "one limit");
-  const bool split_fits = Narrow::kLdsBytes + sizeof(int) * static_cast<size_t>(max_history_blocks) <= kLdsPerGroup;
-  if (wide >= MI_PREFILL_T2 || !split_fits) return Form::kHalf;
-  return wide >= MI_PREFILL_T1 ? Form::kHalfSplit : Form::kNarrow;
+  const int64_t narrow = pairs * ((padded_len + Narrow::kQTile - 1) / Narrow::kQTile);
+  const int64_t history = static_cast<int64_t>(max_history_blocks) * kBlockSize;
+  const bool split_fits = table_fits(Narrow::kLdsBytes, max_history_blocks);
+  if (split_fits && 8 * narrow <= (2 * history >= padded_len ? 8 : 11) * cus) return Form::kNarrow;
+  if (history == 0 && padded_len <= 256) return Form::kHalf;
+  if (2 * wide <= cus) return split_fits ? Form::kHalfSplit : Form::kHalf;
+  if (wide <= cus && history >= padded_len) return Form::kWide;
+  if (wide <= cus) return padded_len > 640 && split_fits ? Form::kHalfSplit : Form::kHalf;
+  return 16 * wide <= 25 * cus ? Form::kHalf : Form::kWide;
 }
 
 int q_tile_of(Form f) {
@@ -980,9 +1006,9 @@ extern "C" int32_t mi_mixed_paged_attention(
     a.num_blocks = num_blocks;
   };
   PrefillArgs a0{}, a1{};
-  const int32_t hist = std::max(chunks ? max_history_blocks : 0, decode_rows > 0 ? max_blocks : 0);
-  // Decode rows alone: the shape whose LDS lets two workgroups share a CU.
-  Form form = !chunks ? Form::kWide : form_for(chunks ? prefill_rows : 0, prefill_width, num_heads, num_kv_heads, hist);
+  // The chunk rows' shape is the one mi_chunked_prefill_attention gives them (with the same bits: the wide shape sums
+  // in the half one's order).  Decode rows alone: the wide shape, two workgroups of which share a CU.
+  Form form = chunks ? form_for(prefill_rows, prefill_width, num_heads, num_kv_heads, max_history_blocks) : Form::kWide;
   if (form == Form::kHalf && decode_rows > 0) form = Form::kWide;  // decode rows take eight wavefronts
   const int q_tile = q_tile_of(form);
   if (chunks) {
@@ -1009,16 +1035,25 @@ extern "C" int32_t mi_mixed_paged_attention(
     a1.decode_rows = 1;
     a1.slot_mapping = slot_mapping;
     a1.slot_stride = slot_stride;
-    // Block by block where the workgroup has kStripes wavefronts, the table has blocks and their ids fit its
-    // lanes; otherwise one-query tiles.
-    a1.stripes = form != Form::kHalf && max_blocks >= 1 && max_blocks <= kRowMaxBlocks && a1.group <= kRowMaxGroup;
+    // Block by block where the table has blocks and their ids fit a wavefront's lanes; otherwise one-query tiles.
+    a1.stripes = max_blocks >= 1 && max_blocks <= kRowMaxBlocks && a1.group <= kRowMaxGroup;
     if (a1.stripes) a1.groups = decode_rows * num_kv_heads;
   }
   ZeroRows z{};
   if (ragged) {
     rc = zero_rows(z, name, out, out_tok_stride, num_heads * head_dim, chunk_first, chunk_lens, lens_stride,
-                   chunks ? prefill_rows : 0, prefill_width, chunk_tokens, Wide::kThreads);
+                   chunks ? prefill_rows : 0, prefill_width, chunk_tokens);
     if (rc != MI_OK) return rc;
   }
-  return launch_form(form, name, a0, a1, z, num_kv_heads, hist, stream);
+  const int32_t chunk_hist = chunks ? max_history_blocks : 0;
+  const int32_t decode_hist = decode_rows > 0 ? max_blocks : 0;
+  if (q_tile != Wide::kQTile && !table_fits(Narrow::kLdsBytes, decode_hist)) {
+    // Decode tables too long for the split shapes' LDS: those rows in a launch of their own, with the wide shape.
+    if (decode_hist > kMaxHistoryBlocks)
+      return fail(MI_ERR_UNSUPPORTED, "%s: history of %d blocks exceeds %d", name, decode_hist, kMaxHistoryBlocks);
+    rc = launch_form(form, name, a0, PrefillArgs{}, z, num_kv_heads, chunk_hist, stream);
+    if (rc != MI_OK) return rc;
+    return launch_form(Form::kWide, name, PrefillArgs{}, a1, ZeroRows{}, num_kv_heads, decode_hist, stream);
+  }
+  return launch_form(form, name, a0, a1, z, num_kv_heads, std::max(chunk_hist, decode_hist), stream);
 }

@@ -1605,8 +1605,9 @@ extern "C" int32_t mi_mixed_paged_attention_exact(
   ZeroRows z{};
   if (ragged) {
     if (const int32_t rc = zero_rows(z, what, out, out_tok_stride, num_heads * head_dim, chunk_first, chunk_lens, lens_stride,
-                                     chunks ? prefill_rows : 0, prefill_width, chunk_tokens, kPfThreads))
+                                     chunks ? prefill_rows : 0, prefill_width, chunk_tokens))
       return rc;
+    z.groups = static_cast<int32_t>((z.tokens + kPfThreads - 1) / kPfThreads);
   }
   const int32_t rc = dispatch_exact_prefill(a0, a1, z, group, what, as_stream(stream));
   return rc == MI_OK ? ok() : rc;

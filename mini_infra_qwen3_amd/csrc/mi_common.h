@@ -198,7 +198,7 @@ struct ZeroRows {
   int64_t lens_stride;
   int64_t tokens;
   int32_t rows, width, row_elems;
-  int32_t groups;      // workgroups: ceil(tokens / threads)
+  int32_t groups;      // workgroups: ceil(tokens / threads of the launch), set by it
 };
 // Workgroup `group` of them: one token per thread, the chunk rows read 64 at a time by each wavefront.
 __device__ __forceinline__ void zero_uncovered_rows(const ZeroRows& z, int group, int threads) {
@@ -225,14 +225,13 @@ __device__ __forceinline__ void zero_uncovered_rows(const ZeroRows& z, int group
     for (int i = lane; i < z.row_elems / 8; i += 64) *reinterpret_cast<u32x4*>(out + 8 * i) = u32x4{0u, 0u, 0u, 0u};
   }
 }
-// Fills z for a launch of `threads` per workgroup; groups 0 when there is nothing to cover.
+// Fills z but for its groups; no tokens when there is nothing to cover.
 inline int32_t zero_rows(ZeroRows& z, const char* what, void* out, int64_t out_tok_stride, int32_t row_elems,
                          const int64_t* first, const int64_t* lens, int64_t lens_stride, int32_t rows, int32_t width,
-                         int64_t tokens, int threads) {
+                         int64_t tokens) {
   if (tokens <= 0) return MI_OK;
   if (tokens > 0x7fffffff) return fail(MI_ERR_UNSUPPORTED, "%s: more than 2^31 - 1 chunk tokens", what);
-  z = ZeroRows{static_cast<uint16_t*>(out), out_tok_stride, first, lens, lens_stride, tokens, rows, width, row_elems,
-               static_cast<int32_t>((tokens + threads - 1) / threads)};
+  z = ZeroRows{static_cast<uint16_t*>(out), out_tok_stride, first, lens, lens_stride, tokens, rows, width, row_elems, 0};
   return MI_OK;
 }
 

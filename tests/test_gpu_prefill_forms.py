@@ -29,17 +29,22 @@ def _chunk_case(seed, starts, lens, kv_heads, group):
     return q, k, v, kp, vp, hist
 
 
-# Wide-shape workgroups (rows x head pairs x 128-query tiles) decide: below 128 the 32-query split shape,
-# to 247 the 64-query split shape, 248 to 256 and from 512 the wide one, between them the 64-query one.
+# The launch's size and the history's length decide (tests/test_prefill_routes.py holds the rule): narrow is 32
+# queries with split keys, half split 64 with split keys, half 64, wide 128.
 @pytest.mark.parametrize("starts,lens,kv_heads,group", [
-    ([0], [1], 8, 2),                              # 8: one query, one key, the second key half idle
-    ([64, 0], [33, 32], 8, 2),                     # 16: one past a 32-query tile
-    ([129, 63, 1], [65, 64, 31], 8, 5),            # 72: odd group, an odd number of key tiles
-    ([0] * 15, [130 - i for i in range(15)], 4, 2),          # 120: the last below 128
-    ([0, 70] * 8, [129 + i for i in range(16)], 4, 2),       # 128: 64-query tiles with split keys
-    ([17] * 31, [97 + i for i in range(31)], 8, 2),          # 248: wide
-    ([0] * 11, [257 + i for i in range(11)], 8, 2),          # 264: 64-query tiles
-    ([0] * 64, [1 + i for i in range(64)], 8, 2),            # 512: wide
+    ([0], [1], 8, 2),                              # narrow: one query, one key, the second key half idle
+    ([64, 0], [33, 32], 8, 2),                     # narrow: one past a 32-query tile
+    ([129, 63, 1], [65, 64, 31], 8, 5),            # narrow: odd group, an odd number of key tiles
+    ([0] * 15, [130 - i for i in range(15)], 4, 2),          # narrow, more workgroups than CUs
+    ([0, 70] * 8, [129 + i for i in range(16)], 4, 2),       # half split
+    ([17] * 31, [97 + i for i in range(31)], 8, 2),          # half
+    ([0] * 11, [257 + i for i in range(11)], 8, 2),          # half
+    ([0] * 64, [1 + i for i in range(64)], 8, 2),            # half
+    ([0, 0], [600, 513], 8, 2),                              # narrow: eleven key tiles, the halves uneven
+    ([600, 70], [513, 450], 8, 2),                           # half split: history as long as the chunk
+    ([0, 65], [1100, 1025], 8, 2),                           # half split: long rows
+    ([140] * 20, [128 - i for i in range(20)], 8, 2),        # wide: history as long as the chunk
+    ([1] * 26, [256 - i for i in range(26)], 8, 2),          # wide
 ])
 def test_shapes_match_oracle(native_lib, device, starts, lens, kv_heads, group):
     q, k, v, kp, vp, hist = _chunk_case(len(lens) + sum(lens), starts, lens, kv_heads, group)
@@ -122,3 +127,30 @@ def test_uncovered_tokens_of_many_rows(native_lib, device):
             chunk_first=first.to(device), chunk_tokens=tokens).cpu()
         assert not out[~covered].any()
         assert (out[covered].float().abs().sum(1) > 0).all() and torch.isfinite(out[covered].float()).all()
+
+
+@pytest.mark.parametrize("starts,lens", [([0], [300]), ([700, 513], [513, 600]), ([0, 0], [1100, 1025])])
+@pytest.mark.parametrize("max_blocks", [40, 8192, 8193])
+def test_chunk_rows_of_a_mixed_step_have_the_bits_of_a_prefill(native_lib, device, starts, lens, max_blocks):
+    """Whatever shape the chunk rows take, and however wide the decode rows' table is beside them (8193 blocks no
+    longer fit the split shapes' LDS)."""
+    q, k, v, kp, vp, hist = _chunk_case(sum(lens), starts, lens, 8, 2)
+    rows, width = len(lens), max(lens)
+    gen = torch.Generator().manual_seed(max_blocks)
+    dec = 3
+    dq, dk, dv = (torch.randn(dec, h, 128, generator=gen).to(torch.bfloat16) for h in (16, 8, 8))
+    table = torch.randint(1, kp.shape[0], (dec, max_blocks), generator=gen)
+    flat = [torch.cat((t.transpose(1, 2).reshape(rows * width, t.shape[1], 128), d)).to(device)
+            for t, d in ((q, dq), (k, dk), (v, dv))]
+    kp, vp, hist = kp.to(device), vp.to(device), hist.to(device)
+    starts, lens = torch.tensor(starts, device=device), torch.tensor(lens, device=device)
+    want = data_plane.chunked_prefill_attention(q.to(device), k.to(device), v.to(device), kp, vp, hist, starts, lens, SCALE)
+    got = data_plane.mixed_paged_attention(
+        *flat, kp, vp, rows, width, hist, starts, lens, table.to(device), torch.tensor([33, 1, 600]).to(device),
+        torch.full((dec,), -1).to(device), SCALE)
+    assert torch.equal(got[:rows * width].view(torch.int16), want.view(rows * width, -1).view(torch.int16))
+    # The decode rows against the same rows beside a table that holds their contexts and no more.
+    alone = data_plane.mixed_paged_attention(
+        *(t[rows * width:] for t in flat), kp, vp, 0, 0, hist[:0], starts[:0], lens[:0], table[:, :40].to(device),
+        torch.tensor([33, 1, 600]).to(device), torch.full((dec,), -1).to(device), SCALE)
+    assert (got[rows * width:].float() - alone.float()).abs().max().item() <= TOL

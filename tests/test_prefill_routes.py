@@ -1,0 +1,74 @@
+"""Which workgroup shapes the prefill and mixed entry points launch, on the CPU against a stand-in HIP runtime (no
+GPU, 256 CUs)."""
+
+import hip_standin
+
+CALLS = """
+P = 4096
+def prefill(rows, width, hist, group=2, kv=8):
+    heads = group * kv
+    return lib.mi_chunked_prefill_attention(P, width * heads * 128, heads * 128, P, width * heads * 128, 128, heads * 128,
+                                            P, width * kv * 128, 128, kv * 128, P, width * kv * 128, 128, kv * 128, P, P, 100, P,
+                                            max(hist, 1), hist, P, P, 1, rows, width, heads, kv, 128, 16, 0.1, None)
+def mixed(rows, width, hist, decode_rows, mb, group=2, kv=8, exact="", first=None, tokens=0):
+    heads = group * kv
+    return getattr(lib, "mi_mixed_paged_attention" + exact)(
+        P, heads * 128, P, heads * 128, 128, P, kv * 128, 128, P, kv * 128, 128, P, P, 100, rows, width, tokens, first, P,
+        max(hist, 1), hist, P, P, 1, decode_rows, P, max(mb, 1), mb, P, 1, P, 1, heads, kv, 128, 16, 0.1, None)
+def shapes():
+    return [(l["args"], l["grid"][0], l["block"], l["lds"]) for l in launches()]
+"""
+WIDE, HALF, HALF_SPLIT, NARROW = [2, 4, 1], [2, 2, 1], [2, 2, 2], [1, 2, 2]
+
+
+def test_prefill_shapes_by_launch_size_and_history():
+    cases = [
+        # narrow: one round of its workgroups, or 11/8 of one without much history
+        (1, 1, 0, 2, NARROW), (1, 1024, 0, 2, NARROW), (1, 60, 250, 2, NARROW), (8, 128, 8, 2, NARROW),
+        (1, 1025, 33, 2, HALF_SPLIT), (1, 1025, 32, 2, NARROW), (2, 704, 0, 2, NARROW), (2, 705, 0, 2, HALF_SPLIT),
+        # short rows without history: half
+        (9, 128, 0, 2, NARROW), (12, 128, 0, 2, HALF), (16, 256, 0, 2, HALF), (64, 128, 0, 2, HALF), (100, 256, 0, 2, HALF),
+        # up to half of the CUs in wide workgroups: half split
+        (12, 128, 1, 2, HALF_SPLIT), (16, 128, 8, 2, HALF_SPLIT), (5, 257, 0, 2, HALF_SPLIT), (1, 2048, 0, 2, HALF_SPLIT),
+        # up to all of them: wide with history, else half split for long rows
+        (17, 128, 8, 2, WIDE), (17, 128, 7, 2, HALF), (2, 1152, 0, 2, HALF_SPLIT), (2, 1152, 72, 2, WIDE), (4, 640, 0, 2, HALF),
+        (4, 641, 0, 2, HALF_SPLIT), (1, 4096, 0, 2, HALF_SPLIT), (32, 128, 8, 2, WIDE),
+        # a second wide round up to 9/16 full: half; beyond: wide
+        (33, 128, 300, 2, HALF), (50, 128, 300, 2, HALF), (51, 128, 300, 2, WIDE), (25, 257, 0, 2, WIDE), (64, 128, 1, 2, WIDE),
+        # the table beside split tiles in LDS
+        (1, 60, 8192, 2, NARROW), (1, 60, 8193, 2, HALF), (4, 2048, 640, 2, WIDE), (2, 700, 0, 5, HALF),
+    ]
+    got = hip_standin.run(CALLS + f"""
+result = []
+for rows, width, hist, group in {[c[:4] for c in cases]}:
+    assert prefill(rows, width, hist, group) == 0
+    result.append(shapes())
+""")
+    for (rows, width, hist, group, want), launches in zip(cases, got):
+        (args, grid, block, lds), = launches
+        assert args[1:] == want, (rows, width, hist, group, args)
+        tile = 16 * args[1] * args[2]
+        assert grid == 8 * ((group + 1) // 2) * rows * -(-width // tile) and lds <= 160 * 1024
+        assert block == 64 * 2 * args[2] * args[3]
+
+
+def test_mixed_chunk_rows_take_the_shape_of_a_prefill():
+    """The same order of sums (the wide shape sums as the half one does), whatever the decode rows' table."""
+    got = hip_standin.run(CALLS + """
+result = []
+for rows, width, hist in [(1, 300, 0), (1, 700, 40), (2, 700, 0), (2, 700, 50), (2, 1200, 0), (4, 640, 0), (33, 128, 0), (4, 2048, 640)]:
+    assert prefill(rows, width, hist) == 0
+    alone = shapes()
+    for mb in (0, 72, 512, 8192, 8193, 16384):
+        assert mixed(rows, width, hist, 7, mb) == 0
+        result.append((mb, alone[0], shapes()))
+    assert mixed(rows, width, hist, 7, 16385) == -2 and not launches()  # refused before any launch
+""")
+    for mb, (want, _, _, _), launches in got:
+        split = want[3] == 2
+        args = [l[0] for l in launches]
+        assert args[0][3] == want[3] and (args[0] == want if split else args[0][1:] == WIDE)
+        assert all(l[3] <= 160 * 1024 for l in launches)
+        assert len(launches) == (2 if split and mb > 8192 else 1)
+        if len(launches) == 2:
+            assert args[1][1:] == WIDE
