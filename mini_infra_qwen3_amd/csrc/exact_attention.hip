@@ -1233,6 +1233,12 @@ int32_t dispatch_exact_decode(const ExactDecodeArgs& a, int32_t batch, int group
   }
 }
 
+int32_t check_exact_groups(const ExactPrefillArgs& a0, const ExactPrefillArgs& a1, const ZeroRows& z, const char* what) {
+  if (a0.groups < 0 || a1.groups < 0 || static_cast<int64_t>(a0.groups) + a1.groups + z.groups > 0x3fffffff)
+    return fail(MI_ERR_UNSUPPORTED, "%s: too many workgroups", what);
+  return MI_OK;
+}
+
 template <int kG, bool kCached>
 int32_t launch_exact_prefill(const ExactPrefillArgs& a0, const ExactPrefillArgs& a1, const ZeroRows& z, const char* what,
                              hipStream_t s) {
@@ -1240,8 +1246,7 @@ int32_t launch_exact_prefill(const ExactPrefillArgs& a0, const ExactPrefillArgs&
   static int32_t attr_rc = MI_OK;
   std::call_once(once, [] { attr_rc = allow_lds(exact_prefill_kernel<kG, kCached>, kPfLdsBytes, "exact_prefill_kernel"); });
   if (attr_rc != MI_OK) return attr_rc;
-  if (a0.groups < 0 || a1.groups < 0 || static_cast<int64_t>(a0.groups) + a1.groups + z.groups > 0x3fffffff)
-    return fail(MI_ERR_UNSUPPORTED, "%s: too many workgroups", what);
+  if (const int32_t rc = check_exact_groups(a0, a1, z, what)) return rc;
   const int groups = a0.groups + a1.groups + z.groups;
   if (groups == 0) return ok();
   const size_t lds = static_cast<size_t>(kPfRedBytes) +
@@ -1549,6 +1554,15 @@ extern "C" int32_t mi_mixed_paged_attention_exact(
   } else {
     a0.kv_heads = num_kv_heads;
   }
+  ZeroRows z{};
+  if (ragged) {
+    if (const int32_t rc = zero_rows(z, what, out, out_tok_stride, num_heads * head_dim, chunk_first, chunk_lens, lens_stride,
+                                     chunks ? prefill_rows : 0, prefill_width, chunk_tokens))
+      return rc;
+    z.groups = static_cast<int32_t>((z.tokens + kPfThreads - 1) / kPfThreads);
+  }
+  // Before any launch: the decode rows may go in one of their own, which appends to the pool.
+  if (const int32_t rc = check_exact_groups(a0, ExactPrefillArgs{}, z, what)) return rc;
   // Decode rows: one-token chunks at the D tokens after the chunk rows, whose history is the
   // context minus the token (the block table), appending each row's rotated K/V to its slot.
   const int group = num_heads / num_kv_heads;
@@ -1601,13 +1615,6 @@ extern "C" int32_t mi_mixed_paged_attention_exact(
       if (const int32_t rc = dispatch_exact_decode<false, true>(d, decode_rows, group, what, as_stream(stream))) return rc;
       a1.groups = 0;
     }
-  }
-  ZeroRows z{};
-  if (ragged) {
-    if (const int32_t rc = zero_rows(z, what, out, out_tok_stride, num_heads * head_dim, chunk_first, chunk_lens, lens_stride,
-                                     chunks ? prefill_rows : 0, prefill_width, chunk_tokens))
-      return rc;
-    z.groups = static_cast<int32_t>((z.tokens + kPfThreads - 1) / kPfThreads);
   }
   const int32_t rc = dispatch_exact_prefill(a0, a1, z, group, what, as_stream(stream));
   return rc == MI_OK ? ok() : rc;

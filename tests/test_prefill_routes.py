@@ -72,3 +72,16 @@ for rows, width, hist in [(1, 300, 0), (1, 700, 40), (2, 700, 0), (2, 700, 50), 
         assert len(launches) == (2 if split and mb > 8192 else 1)
         if len(launches) == 2:
             assert args[1][1:] == WIDE
+
+
+def test_refused_mixed_steps_launch_nothing():
+    """The decode rows append to the pool: a step that a size check refuses must not have run them."""
+    got = hip_standin.run(CALLS + """
+result = []
+for exact in ("", "_exact"):
+    for rows, width, first, tokens in [(1, 64, P, 1 << 31), (65535, 1 << 20, None, 0), (65535, 1 << 20, P, 4096)]:
+        result.append((exact, mixed(rows, width, 4, 3, 20, exact=exact, first=first, tokens=tokens), len(launches())))
+    assert mixed(1, 64, 4, 3, 20, exact=exact, first=P, tokens=100) == 0 and launches()
+""")
+    for exact, rc, count in got:
+        assert (rc, count) == (-2, 0), exact
