@@ -884,8 +884,8 @@ __device__ __forceinline__ double bf16_at(const u32x4 v, int e) {
 }
 
 // One launch serves the chunk rows of a0 after, in the first a1.groups workgroups, a mixed step's decode
-// rows where they have no table (as one-token chunks; with a table the decode body takes them in a launch of
-// its own).  The sums are exact, so both give the same bits.
+// rows where they are few and short, or have no table, as one-token chunks; else the decode body takes them in
+// a launch of its own.  The sums are exact, so both give the same bits.
 // The last z.groups workgroups write zero rows.  Three wavefronts per SIMD: two rows of 500-1024 tokens took
 // 87.2 us, 92.4 with the registers of four (8 bytes of them spilled).
 template <int kG, bool kCached>
@@ -1580,11 +1580,18 @@ extern "C" int32_t mi_mixed_paged_attention_exact(
     a1.slot_mapping = slot_mapping;
     a1.slot_stride = slot_stride;
     exact_rows(a1, decode_rows, 1, num_heads, num_kv_heads, static_cast<int64_t>(max_blocks) * kBlockSize + 1, scale);
-    if (max_blocks > 0) {
-      // Tables with blocks: the decode body, in a launch of its own.  As one-token chunks beside the chunk
-      // rows a decode row was the launch's longest chain (four wavefronts, 2 of 16 matrix columns in use):
-      // one chunk of 400-650 tokens with 7 decode rows 110 -> 76 us, one of 60-120 with 16 103 -> 39.  Inside
-      // the chunk kernel the decode body's registers (224) would halve the chunk rows' wavefronts.
+    // As one-token chunks (four wavefronts, 2 of 16 matrix columns in use) beside the chunk rows, or through the
+    // decode body in a launch of its own; inside the chunk kernel the decode body's registers (224) would
+    // halve the chunk rows' wavefronts.  Beside the chunk rows where they are few and their tables hold hardly
+    // more keys than a chunk row sees: 128 more make the launch's longest chain as much longer as a launch of
+    // their own costs.  Measured, us, beside / own launch: one chunk of 96 tokens behind 300 with 1 row of 100-200
+    // tokens 35 / 45, of 64 with 4 of 20-60 11 / 18, of 300 with 16 of 100-300 34 / 39, of 2048 with 8 to 1150 429 / 447;
+    // one of 400-650 with 7 to 1150 86 / 81, of 60-120 with 16 to 1150 101 / 47, of 24 with 1 of 300-400 36 / 24, two of
+    // 1024 with 64 to 1000 271 / 265, three of 1024 with 200 to 600 441 / 426.
+    const bool beside = chunks && static_cast<int64_t>(max_blocks - max_history_blocks) * kBlockSize <= prefill_width + 128 &&
+                        2 * static_cast<int64_t>(decode_rows) * num_kv_heads <= device_cus() &&
+                        (a1.cache_tiles > 0 || a0.cache_tiles == 0);  // the cached form is off where either set's is
+    if (max_blocks > 0 && !beside) {
       ExactDecodeArgs d{};
       d.out = a1.out;
       d.out_row = a1.out_row;

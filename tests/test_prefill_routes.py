@@ -85,3 +85,35 @@ for exact in ("", "_exact"):
 """)
     for exact, rc, count in got:
         assert (rc, count) == (-2, 0), exact
+
+
+def test_exact_decode_rows_go_beside_the_chunk_rows_where_they_are_few_and_short():
+    """One launch where a decode row's table holds at most 128 keys more than a chunk row sees and the rows fill at most
+    half the CUs; else the decode body in a launch of its own, first."""
+    got = hip_standin.run(CALLS + """
+result = []
+for width, hist, decode_rows, mb in [(96, 19, 1, 13), (96, 19, 1, 33), (96, 19, 1, 34), (97, 0, 16, 14), (97, 0, 16, 15), (97, 0, 17, 6),
+                                     (650, 0, 7, 72), (2048, 0, 8, 136), (2048, 0, 8, 137), (64, 4, 3, 0), (0, 0, 3, 20)]:
+    assert mixed(1 if width else 0, width, hist, decode_rows, mb, exact="_exact") == 0
+    result.append((16 * mb <= 16 * hist + width + 128 and decode_rows <= 16 or mb == 0, bool(width),
+                   [(l["kernel"], l["args"]) for l in launches()]))
+# A score cache that the decode rows' tables outgrow: the chunk rows keep theirs.
+for mb in range(1, 400):
+    assert mixed(1, 16 * mb, 0, 1, mb + 8, exact="_exact") == 0 and prefill_exact(1, 16 * mb) == 0
+    calls = launches()
+    result.append((None, True, [(l["kernel"], l["args"]) for l in calls]))
+""".replace("result = []", """
+def prefill_exact(rows, width, group=2, kv=8):
+    heads = group * kv
+    return lib.mi_chunked_prefill_attention_exact(P, width * heads * 128, heads * 128, P, width * heads * 128, 128, heads * 128,
+                                                  P, width * kv * 128, 128, kv * 128, P, width * kv * 128, 128, kv * 128, P, P, 100,
+                                                  P, 1, 0, P, P, 1, rows, width, heads, kv, 128, 16, 0.1, None)
+result = []"""))
+    for beside, chunks, calls in got:
+        kernels = [name for name, _ in calls]
+        if beside is None:
+            assert calls[-2] == calls[-1]  # the chunk rows' kernel, cached or not, as without decode rows
+        elif not chunks:
+            assert kernels == ["exact_decode_kernel"]
+        else:
+            assert kernels == (["exact_prefill_kernel"] if beside else ["exact_decode_kernel", "exact_prefill_kernel"])
