@@ -45,7 +45,6 @@
 //    together in 3.
 #include <algorithm>
 #include <initializer_list>
-#include <mutex>
 
 #include "decode_block.h"
 
@@ -830,19 +829,7 @@ int q_tile_of(Form f) {
 template <int kKvHeads, typename S>
 int32_t launch_shape(const char* name, const PrefillArgs& a0, const PrefillArgs& a1, const ZeroRows& z, int groups,
                      int32_t max_history_blocks, hipStream_t s) {
-  // Dynamic LDS above 64 KiB must be allowed per kernel and device (gfx950 has 160 KiB per workgroup).
-  constexpr int kMaxDevices = 64;
-  static std::once_flag once[kMaxDevices];
-  static hipError_t errs[kMaxDevices] = {};
-  int dev = 0;
-  if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess || dev < 0 || dev >= kMaxDevices)
-    return fail(MI_ERR_DEVICE, "%s: device %d: %s", name, dev, hipGetErrorString(e));
-  std::call_once(once[dev], [dev] {
-    errs[dev] = hipFuncSetAttribute(reinterpret_cast<const void*>(chunked_prefill_kernel<kKvHeads, S>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerGroup);
-  });
-  if (errs[dev] != hipSuccess)
-    return fail(MI_ERR_DEVICE, "%s: hipFuncSetAttribute: %s", name, hipGetErrorString(errs[dev]));
+  if (const int32_t rc = allow_lds<&chunked_prefill_kernel<kKvHeads, S>>(kLdsPerGroup, name)) return rc;
   const size_t lds = S::kLdsBytes + sizeof(int) * static_cast<size_t>(max_history_blocks > 0 ? max_history_blocks : 1);
   chunked_prefill_kernel<kKvHeads, S><<<groups, S::kThreads, lds, s>>>(a0, a1, z);
   return check_launch(name);

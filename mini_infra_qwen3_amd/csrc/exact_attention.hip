@@ -41,7 +41,6 @@
 // wavefronts splitting the keys; the layout is described at the kernel.
 #include <algorithm>
 #include <math.h>
-#include <mutex>
 
 #include "mi_common.h"
 
@@ -1142,24 +1141,10 @@ __global__ __launch_bounds__(kPfThreads, 3) void exact_prefill_kernel(const Exac
 // ------------------------------------------------------------------------- host ---
 bool group_ok(int g) { return g == 1 || g == 2 || g == 4 || g == 5 || g == 8; }
 
-template <typename Kernel>
-int32_t allow_lds(Kernel kernel, int bytes, const char* what) {
-  // Dynamic LDS above 64 KiB must be allowed per kernel (gfx950 has 160 KiB per workgroup).
-  const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (err != hipSuccess) return fail(MI_ERR_DEVICE, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(err));
-  return MI_OK;
-}
-
 template <int kG, bool kPrologue, bool kToken>
 int32_t launch_exact_decode(const ExactDecodeArgs& a, int32_t batch, const char* what, hipStream_t s) {
-  static std::once_flag once;
-  static int32_t attr_rc = MI_OK;
   using Lds = DecodeLds<kG, kDecWaves>;
-  std::call_once(once, [] {
-    attr_rc = allow_lds(exact_decode_kernel<kG, kPrologue, kToken>, Lds::kFixed + kDecCacheBytes, "exact_decode_kernel");
-  });
-  if (attr_rc != MI_OK) return attr_rc;
+  if (const int32_t rc = allow_lds<&exact_decode_kernel<kG, kPrologue, kToken>>(Lds::kFixed + kDecCacheBytes, what)) return rc;
   const size_t lds = Lds::kFixed + static_cast<size_t>(a.cache_tokens) * kG * sizeof(uint16_t);
   exact_decode_kernel<kG, kPrologue, kToken><<<dim3(batch, a.kv_heads), kDecThreads, lds, s>>>(a);
   return check_launch(what);
@@ -1242,10 +1227,7 @@ int32_t check_exact_groups(const ExactPrefillArgs& a0, const ExactPrefillArgs& a
 template <int kG, bool kCached>
 int32_t launch_exact_prefill(const ExactPrefillArgs& a0, const ExactPrefillArgs& a1, const ZeroRows& z, const char* what,
                              hipStream_t s) {
-  static std::once_flag once;
-  static int32_t attr_rc = MI_OK;
-  std::call_once(once, [] { attr_rc = allow_lds(exact_prefill_kernel<kG, kCached>, kPfLdsBytes, "exact_prefill_kernel"); });
-  if (attr_rc != MI_OK) return attr_rc;
+  if (const int32_t rc = allow_lds<&exact_prefill_kernel<kG, kCached>>(kPfLdsBytes, what)) return rc;
   if (const int32_t rc = check_exact_groups(a0, a1, z, what)) return rc;
   const int groups = a0.groups + a1.groups + z.groups;
   if (groups == 0) return ok();

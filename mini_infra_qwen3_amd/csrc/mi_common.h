@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "../../include/mi_paged.h"
 
 namespace mi {
@@ -83,6 +85,24 @@ inline int device_cus() {
     cached[dev] = cus;
   }
   return cached[dev];
+}
+
+// Dynamic LDS above 64 KiB must be allowed per kernel and device (gfx950 has 160 KiB per workgroup): set at the
+// kernel's first launch on each device.
+template <auto kKernel>
+int32_t allow_lds(int bytes, const char* what) {
+  constexpr int kMaxDevices = 64;
+  static std::once_flag once[kMaxDevices];
+  static hipError_t errs[kMaxDevices] = {};
+  int dev = 0;
+  if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess || dev < 0 || dev >= kMaxDevices)
+    return fail(MI_ERR_DEVICE, "%s: device %d: %s", what, dev, hipGetErrorString(e));
+  std::call_once(once[dev], [&] {
+    errs[dev] = hipFuncSetAttribute(reinterpret_cast<const void*>(kKernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  });
+  if (errs[dev] != hipSuccess)
+    return fail(MI_ERR_DEVICE, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(errs[dev]));
+  return MI_OK;
 }
 
 // Workgroups are handed out round-robin to this many XCDs (accelerator complex dies), each with
