@@ -142,7 +142,8 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t l
 // A decode row of a mixed step (its single new token) by one workgroup of kStripes wavefronts per KV head,
 // with the arithmetic of the decode kernels: stripe v attends blocks v, v + kStripes, ... of the history
 // and the token, whose K and V rows (not yet in the pool, and appended here) are put in place of what its
-// position's slot held.  As a one-query tile a row took 2 us per 64 keys, and the longest decode context
+// position's slot held, with zeros after them: the rest of that block was never part of the row, and an infinity or
+// NaN among it would survive the product with a weight of zero.  As a one-query tile a row took 2 us per 64 keys, and the longest decode context
 // was the longest chain of the launch.
 constexpr int kRowDepth = 3;                             // blocks of a stripe in registers
 constexpr int kRowStageElems = kBlockSize * kKStageRow;  // a wavefront's K staging; its output rows overlay it
@@ -218,7 +219,7 @@ __device__ __forceinline__ void decode_row(const PrefillArgs& a, const int unit,
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           kbuf[s][e] = 4 * e + r == t ? k_new : kbuf[s][e];
-          vbuf[s][e] = 4 * r + e == t ? v_new : vbuf[s][e];
+          vbuf[s][e] = 4 * r + e < t ? vbuf[s][e] : 4 * r + e == t ? v_new : u32x4{};
         }
       }
       attend_block_mfma(ms, qf, kbuf[s], vbuf[s], s_kst + w * kRowStageElems, a.scale, (w + kStripes * i) * kBlockSize,

@@ -276,7 +276,9 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
       for (int t = 0; t < 4; ++t) buf[q][t] = *reinterpret_cast<const u32x4*>(p + 4 * t * row_elems);
     }
   };
-  // The token's row (its 8 dims of this lane) in place of its position in the last block.
+  // The token's row (its 8 dims of this lane) in place of its position in the last block, and zeros after it: what
+  // the pool holds there was never part of the row (a block just handed out, or the table's last one again),
+  // and an infinity or NaN among it would survive the product with a weight of zero.
   u32x4 k_tok{}, v_tok{};
   if constexpr (kToken) {
     k_tok = *reinterpret_cast<const u32x4*>(a.k_new + b * a.k_row + g * a.k_head + 8 * dl);
@@ -287,7 +289,7 @@ __device__ void exact_decode_body(const ExactDecodeArgs& a, const int b, const i
       if (w + kDecWaves * i != nblk - 1) return;  // wave-uniform
       const int at = (n - 1) % kBlockSize;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) buf[t] = 4 * t + r == at ? row : buf[t];
+      for (int t = 0; t < 4; ++t) buf[t] = 4 * t + r < at ? buf[t] : 4 * t + r == at ? row : u32x4{};
     }
   };
   // Scores of the lane row's 4 tokens of block i against the kG queries (equal in the 16 lanes of

@@ -154,3 +154,30 @@ def test_chunk_rows_of_a_mixed_step_have_the_bits_of_a_prefill(native_lib, devic
         *(t[rows * width:] for t in flat), kp, vp, 0, 0, hist[:0], starts[:0], lens[:0], table[:, :40].to(device),
         torch.tensor([33, 1, 600]).to(device), torch.full((dec,), -1).to(device), SCALE)
     assert (got[rows * width:].float() - alone.float()).abs().max().item() <= TOL
+
+
+@pytest.mark.parametrize("max_blocks", [5, 512])
+@pytest.mark.parametrize("group,kv_heads,exact", [(2, 8, False), (8, 2, False), (2, 8, True), (5, 1, True)])
+def test_decode_rows_of_a_mixed_step_do_not_see_what_lies_past_their_history(native_lib, device, max_blocks, group, kv_heads,
+                                                                             exact):
+    """NaN in every pool row that no history holds: the rest of a block just handed out (histories that end on a
+    block), and the table's end (the token comes after the 80 positions it holds)."""
+    contexts = [1, 17, 33, 65, 81, 100, 2, 48] if max_blocks == 5 else [1, 17, 4097, 8177]
+    q, k, v, kp, vp, table = _decode_rows(7, contexts, max_blocks, group, kv_heads)
+    rows = len(contexts)
+    clean_k, clean_v = kp.clone(), vp.clone()
+    kp.fill_(float("nan")), vp.fill_(float("nan"))
+    for b, n in enumerate(contexts):
+        nh = min(n - 1, 16 * max_blocks)
+        for pool, clean in ((kp, clean_k), (vp, clean_v)):
+            pool.view(-1, kv_heads, 128)[(table[b, :, None] * 16 + torch.arange(16)).view(-1)[:nh]] = \
+                clean.view(-1, kv_heads, 128)[(table[b, :, None] * 16 + torch.arange(16)).view(-1)[:nh]]
+    ends = [b for b, n in enumerate(contexts) if min(n - 1, 16 * max_blocks) % 16 == 0]
+    none = torch.zeros(0, dtype=torch.long, device=device)
+    outs = []
+    for pools in ((kp, vp), (clean_k, clean_v)):
+        outs.append(data_plane.mixed_paged_attention(
+            q.to(device), k.to(device), v.to(device), pools[0].to(device), pools[1].to(device), 0, 0,
+            torch.zeros((0, 0), dtype=torch.long, device=device), none, none, table.to(device),
+            torch.tensor(contexts).to(device), torch.full((rows,), -1).to(device), SCALE, exact=exact).cpu())
+    assert len(ends) >= 4 and torch.equal(outs[0][ends], outs[1][ends])
