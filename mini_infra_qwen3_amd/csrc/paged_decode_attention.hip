@@ -1000,6 +1000,10 @@ __global__ __launch_bounds__(64 * kPartWaves, 3) void paged_decode_parts_kernel(
     stage_pair(kb, kst, lane);
     const bf16x8 pa = pair_probs(ms, qf, kst, scale, tok_base(cnt - 1), tok_end, lane);
     patch_values(cnt - 1);
+    if (lo + 2 * (w + kPartWaves * (cnt - 1)) + 1 >= hi) {  // wave-uniform: the second block repeats the first
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vb[1][i] = u32x4{};       // its weights are zero, but an infinite value is not
+    }
     pair_values(ms, pa, vb);
   }
 

@@ -160,3 +160,23 @@ def test_merge_of_many_sequences(native_lib, device, monkeypatch, batch, kv_head
         outs.append(data_plane.paged_decode_attention(q, kp, vp, tables, ctx, SCALE, out=out).float())
     assert (outs[0] - outs[1]).abs().max().item() <= TOL  # NaN (a row not written) fails too
     assert not outs[0][ctx == 0].any()
+
+
+@pytest.mark.parametrize("ctx", [[2577], [2064, 129], [8000, 300, 15]])
+def test_an_infinite_value_stays_infinite(native_lib, device, monkeypatch, ctx):
+    """Parts of an odd number of blocks attend the last one beside a masked copy of itself: an infinity in its values
+    gives an infinite output, as in the stream kernel, not a NaN."""
+    width = max(-(-n // 16) for n in ctx)
+    kp, vp, tables, qkv, _, _, _ = _case(sum(ctx), ctx, max(width, 130), 2)
+    for b, n in enumerate(ctx):
+        vp[tables[b, (n - 1) // 16], (n - 1) % 16, :, ::3] = float("inf")
+        vp[tables[b, 0], 0, :, 1::3] = -float("inf")
+    q = qkv[:, :2048].reshape(len(ctx), 16, 128).contiguous().to(device)
+    outs = []
+    for path in ("stream", "seq"):
+        monkeypatch.setenv("MI_DECODE_PATH", path)
+        outs.append(data_plane.paged_decode_attention(q, kp.to(device), vp.to(device), tables.to(device),
+                                                      torch.tensor(ctx).to(device), SCALE).float())
+    inf = outs[0].isinf()
+    assert inf.float().mean() > 0.6 and torch.equal(outs[0][inf], outs[1][inf])
+    assert (outs[0][~inf] - outs[1][~inf]).abs().max().item() <= TOL
