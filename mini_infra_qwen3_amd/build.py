@@ -1,6 +1,6 @@
 """Builds libmi_paged.so (the HIP kernels + C ABI) in-tree with hipcc for gfx950, and
 libmi_calib.so (HBM streaming-copy calibration kernels that bench.py reads the data-plane rates
-against; not part of the ABI).
+against, and the rounding check of the tests; not part of the ABI).
 
 Usage: ``python -m mini_infra_qwen3_amd.build`` (also called by ``__graft_entry__.build()``).
 Every source is compiled on each call; objects go to ``_build/`` and the libraries next to
