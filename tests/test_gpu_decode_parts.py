@@ -54,7 +54,7 @@ def test_fused_equals_the_two_entry_points(native_lib, device, width, ctx, group
     kp, vp, tables, qkv, (qw, kw), cos, sin = _case(width + group, ctx, width, group)
     heads, kv = group * 8, 8
     slots = torch.tensor([int(tables[b, (n - 1) // 16]) * 16 + (n - 1) % 16 if n else -1 for b, n in enumerate(ctx)])
-    # Three rows put their token elsewhere in their own blocks: the first part, and a middle block.
+    # Up to two rows put their token elsewhere in their own blocks: in the first block, and in a middle one.
     slots[0] = int(tables[0, 0]) * 16 + 3
     if len(ctx) > 2 and ctx[2] > 40:
         slots[2] = int(tables[2, (ctx[2] - 1) // 32]) * 16 + 15

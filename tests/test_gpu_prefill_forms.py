@@ -119,13 +119,14 @@ def test_uncovered_tokens_of_many_rows(native_lib, device):
     for f, n in zip(first.tolist(), lens.tolist()):
         covered[f:f + n] = True
     for exact in (False, True):
-        torch.full((tokens, heads * 128), float("nan"), dtype=torch.bfloat16, device=device)  # likely the next buffer
-        out = data_plane.mixed_paged_attention(
+        out = torch.full((tokens, heads * 128), float("nan"), dtype=torch.bfloat16, device=device)
+        data_plane.mixed_paged_attention(
             q, k, v, pool.clone(), pool.clone(), rows, 6, torch.zeros((rows, 0), dtype=torch.long, device=device),
             torch.zeros(rows, dtype=torch.long, device=device), lens.to(device),
-            torch.zeros((0, 1), dtype=torch.long, device=device), none, none, SCALE, exact=exact,
-            chunk_first=first.to(device), chunk_tokens=tokens).cpu()
-        assert not out[~covered].any()
+            torch.zeros((0, 1), dtype=torch.long, device=device), none, none, SCALE, out=out, exact=exact,
+            chunk_first=first.to(device), chunk_tokens=tokens)
+        out = out.cpu()
+        assert (out[~covered] == 0).all()
         assert (out[covered].float().abs().sum(1) > 0).all() and torch.isfinite(out[covered].float()).all()
 
 

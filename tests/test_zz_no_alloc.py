@@ -1,8 +1,8 @@
 """mi_paged_decode_attention_noalloc (scratch in the library's fixed device array) against
 mi_paged_decode_attention with a caller workspace, called through the C ABI: bit-identical
 outputs on two calls in a row, the second smaller (the array keeps the first call's partials,
-which the second must not read), on launches that take the block-range kernel and cut sequences
-between ranges (so the scratch is used)."""
+which the second must not read), on launches that take the block-range kernel or the parts of the
+per-sequence kernels and cut sequences (so the scratch is used)."""
 
 import ctypes
 
@@ -53,10 +53,15 @@ def _call(lib, noalloc, query, key_pool, value_pool, tables, ctx, max_blocks):
     return out
 
 
-def test_noalloc_matches_the_workspace_entry_point_on_two_calls(native_lib, device):
+@pytest.mark.parametrize("path", ["auto", "stream"])
+def test_noalloc_matches_the_workspace_entry_point_on_two_calls(native_lib, device, monkeypatch, path):
     lib = native_lib
-    # batch 96 x 8 KV heads > 256 CUs: the block-range kernel; contexts up to 2600 tokens cut
-    # sequences between ranges.  Then a smaller launch: fewer sequences, shorter contexts, fewer ranges.
+    # batch 96 x 8 KV heads with contexts up to 2600 tokens: the block-range kernel cuts sequences between
+    # ranges.  Then a smaller launch, fewer sequences and shorter contexts: with fewer ranges of the same
+    # kernel ("stream"), or in parts ("auto").
+    monkeypatch.delenv("MI_DECODE_PATH", raising=False)
+    if path != "auto":
+        monkeypatch.setenv("MI_DECODE_PATH", path)
     for seed, batch, lo, hi in [(0, 96, 300, 2600), (1, 40, 40, 700)]:
         print(f"[no-alloc] seed {seed} batch {batch} contexts U[{lo}, {hi}]", flush=True)
         case = _case(seed, batch, lo, hi, 12000, device)
@@ -70,7 +75,7 @@ def test_noalloc_matches_the_workspace_entry_point_on_two_calls(native_lib, devi
 
 
 def test_noalloc_small_launch_and_repeat(native_lib, device):
-    """A launch the per-sequence kernel serves (no scratch), then the first case again: still exact."""
+    """A small launch (sequences whole, no scratch), then the first case again: still exact."""
     lib = native_lib
     for seed, batch, lo, hi in [(2, 6, 1, 500), (0, 96, 300, 2600)]:
         case = _case(seed, batch, lo, hi, 12000, device)
