@@ -1572,7 +1572,12 @@ extern "C" int32_t mi_mixed_paged_attention_exact(
     // tokens 35 / 45, of 64 with 4 of 20-60 11 / 18, of 300 with 16 of 100-300 34 / 39, of 2048 with 8 to 1150 429 / 447;
     // one of 400-650 with 7 to 1150 86 / 81, of 60-120 with 16 to 1150 101 / 47, of 24 with 1 of 300-400 36 / 24, two of
     // 1024 with 64 to 1000 271 / 265, three of 1024 with 200 to 600 441 / 426.
-    const bool beside = chunks && static_cast<int64_t>(max_blocks - max_history_blocks) * kBlockSize <= prefill_width + 128 &&
+    // A chunk row's keys, from below: a ragged row of a launch wider than the chunk tokens share out (a captured
+    // step, tiled for the longest prompt) has that share, and a history table as wide as any step's says
+    // nothing (steps of 128 chunk tokens with decode rows to 1150 took 6.7 against 6.1 ms by it).
+    const int64_t share = ragged && chunks ? (chunk_tokens + prefill_rows - 1) / prefill_rows : prefill_width;
+    const int64_t keys = share < prefill_width ? share : prefill_width + static_cast<int64_t>(max_history_blocks) * kBlockSize;
+    const bool beside = chunks && static_cast<int64_t>(max_blocks) * kBlockSize <= keys + 128 &&
                         2 * static_cast<int64_t>(decode_rows) * num_kv_heads <= device_cus() &&
                         (a1.cache_tiles > 0 || a0.cache_tiles == 0);  // the cached form is off where either set's is
     if (max_blocks > 0 && !beside) {

@@ -97,6 +97,13 @@ for width, hist, decode_rows, mb in [(96, 19, 1, 13), (96, 19, 1, 33), (96, 19, 
     assert mixed(1 if width else 0, width, hist, decode_rows, mb, exact="_exact") == 0
     result.append((16 * mb <= 16 * hist + width + 128 and decode_rows <= 16 or mb == 0, bool(width),
                    [(l["kernel"], l["args"]) for l in launches()]))
+# Ragged rows: a launch wider than a row's share of the chunk tokens counts the share, without the history.
+for rows, width, tokens, decode_rows, mb in [(1, 1023, 128, 8, 16), (1, 1023, 128, 8, 17), (1, 1023, 1024, 8, 135), (3, 1023, 1024, 8, 29),
+                                             (3, 1023, 1024, 8, 30), (2, 512, 1024, 8, 104), (2, 512, 1023, 8, 104), (2, 513, 1024, 8, 41)]:
+    assert mixed(rows, width, 64, decode_rows, mb, exact="_exact", first=P, tokens=tokens) == 0
+    share = -(-tokens // rows)
+    keys = share if share < width else width + 64 * 16
+    result.append((16 * mb <= keys + 128, True, [(l["kernel"], l["args"]) for l in launches()]))
 # A score cache that the decode rows' tables outgrow: the chunk rows keep theirs.
 for mb in range(1, 400):
     assert mixed(1, 16 * mb, 0, 1, mb + 8, exact="_exact") == 0 and prefill_exact(1, 16 * mb) == 0
