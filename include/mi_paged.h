@@ -219,7 +219,7 @@ int64_t mi_paged_decode_spread_bytes(int32_t batch, int32_t max_blocks, int32_t 
  * tight serving loops, harnesses that forbid hipMalloc).
  *
  * Same arguments, results and errors as mi_paged_decode_attention, bit for bit.  The partials of
- * sequences cut between block ranges go to a fixed device array of the library,
+ * sequences that a launch cuts go to a fixed device array of the library,
  * MI_PAGED_NOALLOC_SCRATCH_BYTES bytes per GPU, held from the first call on a device until the
  * process ends.  A launch that needs more (mi_paged_decode_workspace_bytes above it; 4.3 MB at
  * 16 query / 8 KV heads on 256 CUs) returns MI_ERR_WORKSPACE before any launch, copy or scratch
@@ -336,7 +336,7 @@ int32_t mi_chunked_prefill_attention_exact(void* out, int64_t out_row_stride, in
                                            int32_t head_dim, int32_t block_size, float scale, void* stream);
 
 /*
- * Kernel 4, mixed form -- the attention of a mixed chunk + decode step in one launch: the varlen
+ * Kernel 4, mixed form -- the attention of a mixed chunk + decode step in one call: the varlen
  * attention the reference plans for mixing prefill chunks and decode tokens in one forward
  * (src/mini_infra/core/scheduler.py:310-311, src/mini_infra/core/types.py:108), over the same
  * rows the model's two paths would serve: chunk rows as mi_chunked_prefill_attention and decode
@@ -352,19 +352,20 @@ int32_t mi_chunked_prefill_attention_exact(void* out, int64_t out_row_stride, in
  *     rows, device [P]), C = chunk_tokens and row b's chunk_lens[b] real tokens are tokens
  *     chunk_first[b] .. chunk_first[b] + chunk_lens[b] - 1 (first clamped to [0, C - chunk_lens[b]]):
  *     no padding is stored or read, so C can be the sum of the lengths, and each token of [0, C)
- *     that no row covers (a padded step's tail) gets a zero row (a small launch before the
- *     attention's);
+ *     that no row covers (a padded step's tail) gets a zero row;
  *   tokens [C, T): D decode rows, one token each, context_lens[b] tokens including it: the
  *     first context_lens[b] - 1 are read from the pool through block_tables[b], the last is the
  *     row's own key / value, which the launch also appends to pool slot slot_mapping[b] (a slot
  *     outside the pool is skipped; context 0 marks a padding row: zero output, no append).
- * Chunk rows give the bits of mi_chunked_prefill_attention.  Decode rows are served by the same
- * chunk kernel (a 1-token chunk), within the same tolerance of the reference chain as kernel 3.
- * Either part may be empty (P = 0 or L = 0, D = 0).
+ * Chunk rows give the bits of mi_chunked_prefill_attention.  Decode rows take the decode kernels'
+ * block step in the same launch (without a table, or with more than 511 blocks, one-token chunks),
+ * within the same tolerance of the reference chain as kernel 3; tables of more than 8192 blocks may
+ * take a launch of their own.  Either part may be empty (P = 0 or L = 0, D = 0).
  *
  * mi_mixed_paged_attention_exact -- the same with the reference numerics of
- * mi_chunked_prefill_attention_exact (decode rows as one-token chunks there too, their sums exact);
- * decode rows then give the bits of mi_paged_decode_attention_exact.
+ * mi_chunked_prefill_attention_exact: decode rows as one-token chunks beside the chunk rows where they
+ * are few and short, else through the exact decode kernel in a launch before theirs.  The sums are
+ * exact, so either way decode rows give the bits of mi_paged_decode_attention_exact.
  */
 int32_t mi_mixed_paged_attention(void* out, int64_t out_tok_stride, const void* query, int64_t query_tok_stride,
                                  int64_t query_head_stride, const void* key, int64_t key_tok_stride,

@@ -537,6 +537,8 @@ __global__ __launch_bounds__(64 * kWaves, (kGroupsPerCu * kWaves + 3) / 4) void 
 //    kernel's per-block arithmetic and merged in order.  One workgroup holds all stripes (and writes
 //    the rows), or kStripeWaves each hold some and the merge launch joins them: the bits are the same.
 //  * parts, longer tables or more pairs: contiguous ranges of the table, two blocks a step.
+// Spreading is for launches whose workspace is their own: mi_paged_decode_attention keeps small launches whole
+// (one workgroup per pair), the spread entry points cut them.
 // Measured against the form before (the stripes of a pair always in one workgroup, with a ring that
 // re-read the last block past its end), us per layer with the prologue and the merge, passes in a graph:
 // one sequence of 417 tokens 8.4 -> 6.9 (stripes in one workgroup); 8 of U[32, 1150] 18.4 -> 13.3, 24
@@ -1195,11 +1197,11 @@ __global__ __launch_bounds__(kMergeThreads) void paged_decode_merge_kernel(const
   }
 }
 
-// The stream form's merge where the ranges are no shorter than two sequences apart: one workgroup per sequence, a
-// thread per (query head, 8 dims) of all heads, kMergeUnroll partials a step.  Few sequences are cut then,
-// into two or three, and the launch is its pass over the contexts, which the form above makes once per
-// KV head: this one / that one, us, at 512 sequences with 16 heads 6 / 12, with 64 heads 9 / 37, at 2048
-// with 16 heads 14 / 32 (batch 200 of U[32, 300], attention and merge, 33.7 / 36.4).
+// The stream form's merge where a sequence spans under two ranges on average: one workgroup per sequence, a thread
+// per (query head, 8 dims) of all heads, kMergeUnroll partials a step.  A sequence is cut into two or three
+// then, or not at all, and the launch is its pass over the contexts, which the form above makes once per
+// KV head beside reads for 16 partials: 512 sequences with 16 heads 5-6 us where that form takes 12, with 64
+// heads 9 / 37, 2048 with 16 heads 14 / 32 (200 of U[32, 300], attention and merge, 33.7 / 36.4).
 template <int kHeads>
 constexpr int merge_rows_threads() {
   return kHeads * 16 < 256 ? 256 : kHeads * 16;
@@ -1307,7 +1309,7 @@ int streams_for(int32_t batch, int32_t max_blocks, int32_t num_kv_heads) {
 constexpr int kPartGroupsPerCu = MI_DECODE_PART_GROUPS;
 // Stripes up to this table length and number of (sequence, KV head) pairs: beyond 128 blocks a stripe
 // is a serial chain of more than 16 of them; beyond 256 pairs, parts won (64 sequences of U[32, 1150]
-// 39.5 against 41.7 us, 40 of them 26.0 against 27.1).
+// 39.5 against 41.7 us, 40 of them 26.0 against 27.1, with the prologue in the launch, as it was then).
 constexpr int kStripeMaxBlocks = MI_DECODE_STRIPE_BLOCKS;
 constexpr int kStripeMaxPairs = MI_DECODE_STRIPE_PAIRS;
 
@@ -1692,11 +1694,11 @@ extern "C" int32_t mi_paged_decode_attention_fused_spread(
       workspace, workspace_bytes, mi::Workspace::kOwn, stream);
 }
 
-// ---- The no-allocation variant.  The stream kernel's cut-sequence partials go to `scratch`, a
-// fixed device array of this library (each GPU holds its own copy for the life of the process),
-// instead of a caller workspace.  No part of it needs clearing: a partial slot is written by its
-// range before the merge launch reads it.  Every call on one GPU shares the array, so calls that
-// overlap on one GPU (different streams, or threads) race on it.
+// ---- The no-allocation variant.  The partials of sequences that the stream or the parts kernel cuts go to
+// `scratch`, a fixed device array of this library (each GPU holds its own copy for the life of the
+// process), instead of a caller workspace.  No part of it needs clearing: a partial slot is written
+// before the merge launch uses it.  Every call on one GPU shares the array, so calls that overlap on
+// one GPU (different streams, or threads) race on it.
 namespace mi {
 namespace {
 constexpr int64_t kScratchBytes = MI_PAGED_NOALLOC_SCRATCH_BYTES;  // 4.3 MB used at 16 / 8 heads on 256 CUs

@@ -401,8 +401,9 @@ def paged_decode_attention_fused(
     exact: bool = False,
 ) -> torch.Tensor:
     """``qk_norm_rope`` (decode form: the new K/V rows go to ``slot_mapping``) followed by
-    ``paged_decode_attention``, in one launch where the per-sequence kernel serves the batch
-    (with ``exact``: always one launch of the reference-numerics kernel).
+    ``paged_decode_attention``.  Small batches (one (sequence, KV head) pair per CU at most) do the
+    norm, the rotation and the append in the attention's launch, with a merge after it where sequences
+    are cut; so does the reference-numerics kernel (``exact``) at any batch.
 
     q ``[B, Hq * 128]``, k / v ``[B, Hkv * 128]``: the new tokens' projection rows (row views are
     fine); cos / sin ``[B, 128]``; the rest as in the two functions.  Same results, bit for bit.
@@ -579,8 +580,9 @@ def mixed_paged_attention(
     chunk_first: torch.Tensor | None = None,
     chunk_tokens: int | None = None,
 ) -> torch.Tensor:
-    """The attention of a mixed chunk + decode step in one launch (``mi_mixed_paged_attention``, or
-    ``mi_mixed_paged_attention_exact`` with ``exact``), which also appends the decode tokens' K/V.
+    """The attention of a mixed chunk + decode step (``mi_mixed_paged_attention``, or
+    ``mi_mixed_paged_attention_exact`` with ``exact``, whose decode rows may take a launch of their
+    own), which also appends the decode tokens' K/V.
 
     A flattened batch of T = C + D tokens: query ``[T, H, D]``, key / value ``[T, H_kv, D]``
     (token-major, D contiguous; the rotated q / k of ``qk_norm_rope``).  Tokens ``[0, C)`` are P

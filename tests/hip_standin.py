@@ -110,6 +110,10 @@ result = None
 
 
 def run(body: str):
+    from mini_infra_qwen3_amd import _native, build
+
+    if not _native.LIBRARY_PATH.exists():
+        build.build(verbose=False)
     with tempfile.TemporaryDirectory() as tmp:
         source, standin = Path(tmp, "standin.c"), Path(tmp, "libstandin.so")
         source.write_text(_SOURCE)
