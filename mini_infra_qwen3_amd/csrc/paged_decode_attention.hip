@@ -1463,16 +1463,13 @@ bool is_small(int32_t batch, int32_t num_kv_heads) {
   return static_cast<int64_t>(batch) * num_kv_heads <= device_cus();
 }
 
-// mi_paged_decode_attention.
-int32_t decode_attention(void* out, int64_t out_row_stride, const void* query, int64_t query_row_stride,
-                         int64_t query_head_stride, const void* key_pool, const void* value_pool, int64_t num_blocks,
-                         const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks,
-                         const int64_t* context_lens, int64_t context_lens_stride, int32_t batch, int32_t num_heads,
-                         int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale, void* workspace,
-                         int64_t workspace_bytes, Workspace use, void* stream) {
-  if (batch < 0 || max_blocks < 0 || num_blocks < 0)
-    return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention: negative size");
-  if (batch == 0) return ok();
+// The checks of mi_paged_decode_attention (batch > 0), which launch nothing.
+int32_t check_attention(const void* out, int64_t out_row_stride, const void* query, int64_t query_row_stride,
+                        int64_t query_head_stride, const void* key_pool, const void* value_pool, int64_t num_blocks,
+                        const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks,
+                        const int64_t* context_lens, int64_t context_lens_stride, int32_t batch, int32_t num_heads,
+                        int32_t num_kv_heads, int32_t head_dim, int32_t block_size, const void* workspace,
+                        int64_t workspace_bytes, Workspace use) {
   if (const int32_t rc = reject_empty_pool("mi_paged_decode_attention", num_blocks, max_blocks > 0)) return rc;
   if (!out || !query || !key_pool || !value_pool || !context_lens || (max_blocks > 0 && !block_tables))
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention: null pointer argument");
@@ -1488,13 +1485,31 @@ int32_t decode_attention(void* out, int64_t out_row_stride, const void* query, i
   if (static_cast<int64_t>(kMaxBatchPerLaunch) * max_blocks >= (1ll << 31))
     return fail(MI_ERR_UNSUPPORTED, "mi_paged_decode_attention: max_blocks %d too large", max_blocks);
 
-  const int32_t streams = streams_for(batch, max_blocks, num_kv_heads);
   const int64_t need = mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size);
   if (use != Workspace::kNone && max_blocks > 0 && (!workspace || workspace_bytes < need))
     return fail(MI_ERR_WORKSPACE, "mi_paged_decode_attention: workspace of %lld bytes needed, got %lld",
                 static_cast<long long>(need), static_cast<long long>(workspace_bytes));
   if (use != Workspace::kNone && max_blocks > 0 && !aligned16(workspace))
     return fail(MI_ERR_UNSUPPORTED, "mi_paged_decode_attention: workspace must be 16-byte aligned");
+  return MI_OK;
+}
+
+// mi_paged_decode_attention.
+int32_t decode_attention(void* out, int64_t out_row_stride, const void* query, int64_t query_row_stride,
+                         int64_t query_head_stride, const void* key_pool, const void* value_pool, int64_t num_blocks,
+                         const int64_t* block_tables, int64_t block_table_stride, int32_t max_blocks,
+                         const int64_t* context_lens, int64_t context_lens_stride, int32_t batch, int32_t num_heads,
+                         int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale, void* workspace,
+                         int64_t workspace_bytes, Workspace use, void* stream) {
+  if (batch < 0 || max_blocks < 0 || num_blocks < 0)
+    return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_attention: negative size");
+  if (batch == 0) return ok();
+  if (const int32_t rc = check_attention(out, out_row_stride, query, query_row_stride, query_head_stride, key_pool, value_pool,
+                                         num_blocks, block_tables, block_table_stride, max_blocks, context_lens,
+                                         context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size,
+                                         workspace, workspace_bytes, use))
+    return rc;
+  const int32_t streams = streams_for(batch, max_blocks, num_kv_heads);
   float* ws_acc = static_cast<float*>(workspace);
   float* ws_ml = ws_acc ? ws_acc + static_cast<int64_t>(streams) * 2 * num_heads * kHeadDim : nullptr;
 
@@ -1609,15 +1624,21 @@ int32_t decode_attention_fused(
   const bool room = use == Workspace::kOwn && workspace && workspace_bytes >= need && aligned16(workspace);
   const bool sequences = small && use_seq_path(batch, max_blocks, num_kv_heads);  // the per-sequence kernels serve it
   if (!sequences || !pieces) {
-    // The append and q rotation in a launch of their own (large launches; rows of other alignments).
-    int32_t rc = mi_qk_norm_rope(q_scratch, nullptr, nullptr, q, q_row_stride, k, k_row_stride, v, v_row_stride,
+    // The append and q rotation in a launch of their own (large launches; rows of other alignments), once
+    // nothing can refuse the attention after it.
+    const Workspace given = sequences && !room ? Workspace::kNone : use;
+    const int64_t q_head = head_dim, q_row = num_heads * q_head;
+    int32_t rc = check_attention(out, out_row_stride, q_scratch, q_row, q_head, key_pool, value_pool, num_blocks,
+                                 block_tables, block_table_stride, max_blocks, context_lens, context_lens_stride, batch,
+                                 num_heads, num_kv_heads, head_dim, block_size, workspace, workspace_bytes, given);
+    if (rc != MI_OK) return rc;
+    rc = mi_qk_norm_rope(q_scratch, nullptr, nullptr, q, q_row_stride, k, k_row_stride, v, v_row_stride,
                                  q_weight, k_weight, cos, sin, batch, num_heads, num_kv_heads, head_dim, eps,
                                  slot_mapping, slot_stride, key_pool, value_pool, num_blocks * block_size, stream);
     if (rc != MI_OK) return rc;
-    return decode_attention(out, out_row_stride, q_scratch, static_cast<int64_t>(num_heads) * head_dim, head_dim, key_pool,
-                            value_pool, num_blocks, block_tables, block_table_stride, max_blocks, context_lens,
-                            context_lens_stride, batch, num_heads, num_kv_heads, head_dim, block_size, scale, workspace,
-                            workspace_bytes, sequences && !room ? Workspace::kNone : use, stream);
+    return decode_attention(out, out_row_stride, q_scratch, q_row, q_head, key_pool, value_pool, num_blocks, block_tables,
+                            block_table_stride, max_blocks, context_lens, context_lens_stride, batch, num_heads,
+                            num_kv_heads, head_dim, block_size, scale, workspace, workspace_bytes, given, stream);
   }
   // The per-sequence kernel with the prologue.  Shape checks as in the two entry points.
   if (!out || !key_pool || !value_pool || !context_lens || !block_tables)

@@ -108,3 +108,16 @@ for batch, kv in [(33, 8), (64, 8), (191, 8), (192, 8), (256, 8), (512, 8), (409
     for pairs, mb, kernel in routes:
         per_sequence = pairs < 6 * 256 and pairs * mb <= 98304
         assert (kernel != "paged_decode_kernel") == per_sequence, (pairs, mb, kernel)
+
+
+def test_refused_fused_launches_append_nothing():
+    """A call that the attention's checks refuse launches nothing, the append included."""
+    got = hip_standin.run(CALLS + """
+result = []
+for entry in ("mi_paged_decode_attention_fused", "mi_paged_decode_attention_fused_spread"):
+    for batch, mb, ws, nbytes in [(64, 72, None, 0), (64, 72, P, 1 << 10), (64, 72, P + 8, 1 << 30), (8, 600, None, 0), (64, 1 << 20, P, 1 << 40)]:
+        result.append((fused(entry, batch, mb, ws, nbytes), len(launches())))
+    assert fused(entry, 64, 72) == 0 and len(launches()) == 3
+""")
+    for rc, count in got:
+        assert rc < 0 and count == 0
