@@ -265,21 +265,23 @@ def paged_decode_workspace_bytes(batch: int, max_blocks: int, num_heads: int, he
 
 
 def _decode_workspace(lib, workspace: torch.Tensor | None, batch: int, max_blocks: int, num_heads: int, num_kv_heads: int,
-                      head_dim: int, block_size: int, device: torch.device) -> tuple[bool, torch.Tensor | None]:
-    """(spread, workspace) of a bandwidth decode launch.  A small launch that can cut its sequences gets a
-    buffer of this call's own (``spread``): the caller's may be in use by another small launch on another
-    stream.  Others get ``workspace``, or a new buffer when it is missing or too small; None when the
-    launch needs none.  The caller keeps the buffer until the launch is enqueued."""
+                      head_dim: int, block_size: int, device: torch.device, extra: int = 0
+                      ) -> tuple[int, torch.Tensor | None]:
+    """(spread bytes, workspace) of a bandwidth decode launch.  A small launch that can cut its sequences
+    (spread bytes > 0) gets a buffer of this call's own, with ``extra`` bytes after the workspace's: the
+    caller's may be in use by another small launch on another stream.  Others get ``workspace``, or a
+    new buffer when it is missing or too small; None when the launch needs none.  The caller keeps the
+    buffer until the launch is enqueued."""
     need = lib.mi_paged_decode_spread_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size)
     if need > 0:
-        return True, torch.empty(need, dtype=torch.uint8, device=device)
+        return need, torch.empty(need + extra, dtype=torch.uint8, device=device)
     need = lib.mi_paged_decode_workspace_bytes(batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size)
     if need <= 0:
-        return False, None
+        return 0, None
     if workspace is None or workspace.numel() * workspace.element_size() < need:
-        return False, torch.empty(need, dtype=torch.uint8, device=device)
+        return 0, torch.empty(need, dtype=torch.uint8, device=device)
     _require_gpu("workspace", workspace, device)
-    return False, workspace
+    return 0, workspace
 
 
 def paged_decode_exact_workspace_bytes(batch: int, max_blocks: int, num_heads: int, num_kv_heads: int,
@@ -472,17 +474,23 @@ def paged_decode_attention_fused(
             float(scale), ws_ptr, ws_bytes, _stream(device))
         _native.check(rc, "mi_paged_decode_attention_exact")
         return out
-    q_scratch = torch.empty((batch, num_heads, head_dim), dtype=torch.bfloat16, device=device)
     lib = _native.load()
-    spread, ws = _decode_workspace(lib, workspace, batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size, device)
+    scratch_bytes = 2 * batch * num_heads * head_dim
+    spread, ws = _decode_workspace(lib, workspace, batch, max_blocks, num_heads, num_kv_heads, head_dim, block_size, device,
+                                   extra=scratch_bytes)
     ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel() * ws.element_size())
+    if spread:  # one buffer: the workspace (a multiple of 16 bytes), then the rotated queries' scratch
+        q_scratch, ws_bytes = ws_ptr + spread, spread
+    else:
+        scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=device)
+        q_scratch = scratch.data_ptr()
     rc = (lib.mi_paged_decode_attention_fused_spread if spread else lib.mi_paged_decode_attention_fused)(
         out.data_ptr(), out.stride(0), q2.data_ptr(), q2.stride(0), k2.data_ptr(), k2.stride(0), v2.data_ptr(),
         v2.stride(0), q_weight.data_ptr(), k_weight.data_ptr(), cos2.data_ptr(), sin2.data_ptr(), float(eps),
         slot_mapping.data_ptr(), slot_mapping.stride(0) if batch > 1 else 1, key_pool.data_ptr(), value_pool.data_ptr(),
         num_blocks, block_tables.data_ptr(), block_tables.stride(0) if batch > 1 else max(max_blocks, 1), max_blocks,
         context_lens.data_ptr(), context_lens.stride(0) if batch > 1 else 1, batch, num_heads, num_kv_heads,
-        head_dim, block_size, float(scale), q_scratch.data_ptr(), ws_ptr, ws_bytes, _stream(device))
+        head_dim, block_size, float(scale), q_scratch, ws_ptr, ws_bytes, _stream(device))
     _native.check(rc, "mi_paged_decode_attention_fused")
     return out
 
